@@ -75,13 +75,14 @@ int ramgpu_set_species(ramgpu_ctx *ctx, int s, int charge, int cex_kind, double 
 
 /* ModRamTiming::DTs, ModRamParams::BetaLim, ModRamVariables::FracCFL */
 int ramgpu_set_params(ramgpu_ctx *ctx, double dts, double betalim, double fraccfl);
-/* Launch shape of the energy / pitch-angle plane kernels (no counterpart in
- * the reference; a tuning control): blocks of `threads` (a multiple of 64,
- * at most 1024) in which each thread owns one K of ceil(NPA/floor(threads/NE))
- * rows, at most `maxc` (8 or 16; 16 with at most 512 threads).  0, 0
- * restores the shape the library picks from NE, NPA and the device's LDS.
- * The SUMRC sums add the plane's cells in an order that follows the shape, so
- * ensembles keep each member's shape. */
+/* Launch shape of the plane kernels of the single energy, pitch-angle, loss
+ * and Coulomb operators (no counterpart in the reference; a tuning control):
+ * blocks of `threads` (a multiple of 64, at most 1024) in which each thread
+ * owns one K of ceil(NPA/floor(threads/NE)) rows, at most `maxc` (8 or 16; 16
+ * with at most 512 threads).  0, 0 restores the shape the library picks from
+ * NE, NPA and the device's LDS.  SUMRC adds the plane's cells in an order
+ * that follows the shape.  The fused step of ramgpu_ram_run picks the shape
+ * of its own plane kernel from the problem's sizes. */
 int ramgpu_set_plane_shape(ramgpu_ctx *ctx, int threads, int maxc);
 int ramgpu_get_plane_shape(ramgpu_ctx *ctx, int *threads, int *maxc);
 

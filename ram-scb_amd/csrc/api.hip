@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -378,13 +379,10 @@ void launch_plane_t(int seq, int threads, dim3 grid, size_t lds, hipStream_t st,
     case SEQ_CEX: hipLaunchKernelGGL((k_plane<SEQ_CEX, MAXC>), grid, blk, lds, st, L, rec); break;
     case SEQ_ATM: hipLaunchKernelGGL((k_plane<SEQ_ATM, MAXC>), grid, blk, lds, st, L, rec); break;
     case SEQ_SUM: hipLaunchKernelGGL((k_plane<SEQ_SUM, MAXC>), grid, blk, lds, st, L, rec); break;
-    case SEQ_LOSS: hipLaunchKernelGGL((k_plane<SEQ_LOSS, MAXC>), grid, blk, lds, st, L, rec); break;
-    case SEQ_TAPE: hipLaunchKernelGGL((k_plane<SEQ_TAPE, MAXC>), grid, blk, lds, st, L, rec); break;
     case SEQ_WAVE: hipLaunchKernelGGL((k_plane<SEQ_WAVE, MAXC>), grid, blk, lds, st, L, rec); break;
     case SEQ_COULEN: hipLaunchKernelGGL((k_plane<SEQ_COULEN, MAXC>), grid, blk, lds, st, L, rec); break;
     case SEQ_COULMU: hipLaunchKernelGGL((k_plane<SEQ_COULMU, MAXC>), grid, blk, lds, st, L, rec); break;
-    case SEQ_STEPC: hipLaunchKernelGGL((k_plane<SEQ_STEPC, MAXC>), grid, blk, lds, st, L, rec); break;
-    default: hipLaunchKernelGGL((k_plane<SEQ_STEP, MAXC>), grid, blk, lds, st, L, rec); break;
+    default: hipLaunchKernelGGL((k_plane<SEQ_STEPC, MAXC>), grid, blk, lds, st, L, rec); break;
   }
 }
 
@@ -393,6 +391,54 @@ void launch_plane(int seq, PlaneShape sh, dim3 grid, size_t lds, hipStream_t st,
     launch_plane_t<8>(seq, sh.threads, grid, lds, st, L, rec);
   else
     launch_plane_t<16>(seq, sh.threads, grid, lds, st, L, rec);
+}
+
+// Rows per thread the fused step's plane kernel is built for.
+#define STEP_ROWS(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16)
+
+// Rows per thread of the fused step's plane kernel, a function of NE, NPA and
+// the problem's planes per CU.
+// A plane's cost is the rows that its busiest SIMD sweeps, set-up counting as
+// four: between waves/4 and its ceiling, as blocks overlap.  Fewer resident
+// waves hide less latency (measured, planes of 35x72, 48x90 and 64x90 on
+// MI355X: 9 of 16 waves cost 1.2-1.3 times, 12 of 16 1.1), and up to 9 rows
+// the kernel keeps DRIFTMU's Courant numbers in registers (0.94).  Plane
+// launch of 4 species in us, by rows:
+//   35x72 (20x25): 6: 105, 8: 118, 11: 95, 12: 94, 16: 121
+//   48x90 (40x48): 6: 612, 9: 453, 10: 553, 16: 734
+//   64x90 (20x48): 8: 385, 10: 456, 12: 308, 16: 411
+// One species of 20x25x35x72 has under two planes per CU: 6 rows 37, 12 rows 42.
+// The last chunk needs two rows: R with NPA mod R = 1 is left out.
+StepShape step_shape(int ne, int npa, long planes, int ncu, size_t lds_cu) {
+  StepShape best{0, 0};
+  double bcost = 0;
+  for (int r = 2; r <= kMaxCellsPerThread; ++r) {
+    const int threads = step_threads(ne, npa, r), waves = threads / 64;
+    const size_t lds = step_lds_bytes(ne, npa, r);
+    if (npa % r == 1 || threads > kPlaneMaxThreads || lds > lds_cu) continue;
+    const int res = std::min<long>(step_resident(lds, ne, npa, r), (planes + ncu - 1) / ncu);
+    if (res < 1) continue;
+    const double rows = 0.5 * (waves / 4.0 + (waves + 3) / 4) * (r + 4);
+    const double cost = rows * (r <= 9 ? 0.94 : 1.0) * std::pow(16.0 / (res * waves), 0.4);
+    if (best.threads == 0 || cost < bcost) {
+      best = {threads, r};
+      bcost = cost;
+    }
+  }
+  return best;
+}
+
+void launch_step(int seq, StepShape sh, dim3 grid, size_t lds, hipStream_t st, const Launch &L, int rec) {
+  const dim3 blk(sh.threads);
+  switch (sh.rows) {
+#define ROWS(r)                                                                                              \
+  case r:                                                                                                    \
+    if (seq == SEQ_TAPE) hipLaunchKernelGGL((k_plane_step<SEQ_TAPE, r>), grid, blk, lds, st, L, rec);        \
+    else hipLaunchKernelGGL((k_plane_step<SEQ_STEP, r>), grid, blk, lds, st, L, rec);                        \
+    break;
+    STEP_ROWS(ROWS)
+#undef ROWS
+  }
 }
 
 int run_plane(ramgpu_ctx *c, int seq, int rec, int s0, int nsp, const double *src, double *dst) {
@@ -405,7 +451,10 @@ int run_plane(ramgpu_ctx *c, int seq, int rec, int s0, int nsp, const double *sr
   const size_t lds = seq_coul(seq) ? plane_coul_lds_bytes(c->ne, c->npa, c->plane.threads)
                                     : plane_fwd_lds_bytes(c->ne, c->npa, c->plane.threads);
   tbeg(c, RAMGPU_KERNEL_PLANE);
-  launch_plane(seq, c->plane, dim3(L.nv), lds, c->stream, L, rec);
+  if (seq == SEQ_STEP || seq == SEQ_TAPE)
+    launch_step(seq, c->step, dim3(L.nv), step_lds_bytes(c->ne, c->npa, c->step.rows), c->stream, L, rec);
+  else
+    launch_plane(seq, c->plane, dim3(L.nv), lds, c->stream, L, rec);
   tend(c);
   return launch_check("k_plane");
 }
@@ -466,10 +515,13 @@ int set_plane_lds_limit(size_t limit) {
 #define PLANE_K(S) (const void *)k_plane<S, 8>, (const void *)k_plane<S, 16>
   const void *fns[] = {
       PLANE_K(SEQ_E), PLANE_K(SEQ_MU), PLANE_K(SEQ_CEX), PLANE_K(SEQ_ATM), PLANE_K(SEQ_SUM),
-      PLANE_K(SEQ_STEP), PLANE_K(SEQ_LOSS), PLANE_K(SEQ_TAPE), PLANE_K(SEQ_WAVE),
+      PLANE_K(SEQ_WAVE),
       PLANE_K(SEQ_COULEN), PLANE_K(SEQ_COULMU), PLANE_K(SEQ_STEPC),
       (const void *)k_r<0>, (const void *)k_r<1>, (const void *)k_r<2>,
       (const void *)k_r_bwd<0>, (const void *)k_r_bwd<1>, (const void *)k_p<0>, (const void *)k_p<1>,
+#define STEP_K(r) (const void *)k_plane_step<SEQ_STEP, r>, (const void *)k_plane_step<SEQ_TAPE, r>,
+      STEP_ROWS(STEP_K)
+#undef STEP_K
       (const void *)k_p_bwd, (const void *)k_pitch_diffusion};
 #undef PLANE_K
   for (const void *f : fns) {
@@ -572,7 +624,11 @@ int ramgpu_create(ramgpu_ctx **out, int ns, int nr, int nt, int ne, int npa, int
   c->ne = ne;
   c->npa = npa;
   hipDeviceProp_t prop;
-  if (hipGetDeviceProperties(&prop, device) == hipSuccess) c->lds_limit = prop.sharedMemPerBlock;
+  int ncu = 256;
+  if (hipGetDeviceProperties(&prop, device) == hipSuccess) {
+    c->lds_limit = prop.sharedMemPerBlock;
+    ncu = prop.multiProcessorCount;
+  }
   int rc = RAMGPU_OK;
   auto cleanup = [&](int code) {
     ramgpu_destroy(c);
@@ -600,6 +656,10 @@ int ramgpu_create(ramgpu_ctx **out, int ns, int nr, int nt, int ne, int npa, int
   c->plane = plane_shape(ne, npa, c->lds_limit);
   if (c->plane.threads == 0) return cleanup(fail(RAMGPU_EINVAL, "no plane kernel shape for %dx%d", ne, npa));
   t.plane_chunks = plane_chunks_for(ne, npa, c->plane.threads);
+  c->step = step_shape(ne, npa, (long)ns * (nr - 1) * nt, ncu, c->lds_limit);
+  if (c->step.threads == 0) return cleanup(fail(RAMGPU_EINVAL, "no plane kernel shape for %dx%d", ne, npa));
+  t.step_cells = step_wave_cells(ne);
+  t.step_apart = step_edges_apart(ne, npa, c->step.rows);
   c->d_pdc.assign(ns, nullptr);
   c->d_flc.assign(ns, nullptr);
   c->d_flc_mem.assign(ns, nullptr);
@@ -624,6 +684,7 @@ int ramgpu_create(ramgpu_ctx **out, int ns, int nr, int nt, int ne, int npa, int
   A(t.carry, (size_t)ns * ne * npa);
   A(t.latl, (size_t)ns * nr * ne);
   A(t.ex64, 64);
+  A(t.kt, (size_t)ns * SKT_N * ne); A(t.lt4, (size_t)4 * npa);
   A(c->d_tab, 1);
   A(t.cflmax, (size_t)ns * (2 + ne + npa));
   A(t.dtdrift, (size_t)ns * 4);

@@ -17,6 +17,8 @@
 
 #include <algorithm>
 #include <cstdlib>
+#include <numeric>
+#include <utility>
 #include <vector>
 
 #include "ctx.h"
@@ -36,6 +38,14 @@ struct Plan {
   int *vmap = nullptr;
   int nv = 0;
   int cap = 0;  // 0: one block per virtual block; else the persistent grid size
+  // plane kinds: one launch per shape of the members' fused plane kernels,
+  // over the virtual blocks [v0, v0 + nv) of its members
+  struct Group {
+    StepShape sh;
+    size_t lds;
+    int v0, nv;
+  };
+  std::vector<Group> groups;
 };
 
 }  // namespace
@@ -47,10 +57,9 @@ struct ramgpu_batch {
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   Tab *d_tabs = nullptr;
   Plan plan[BK_N];
-  size_t plane_lds = 0, radial_lds = 0, azim_lds = 0, ghost_lds = 0;
+  size_t radial_lds = 0, azim_lds = 0, ghost_lds = 0;
   int mpts_max = 0;  // most satellite points of a member (ensemble adjoint)
-  // forward plane blocks of every member: the largest block a member
-  // chose and the largest row bound among them
+  // the largest block and row bound of the members' single-operator plane kernels at creation
   PlaneShape plane{64, 8, 0};
   std::vector<char> wave;  // each member's WAVELO at creation (its coefficient units)
   int sum_ns = 0;
@@ -95,12 +104,24 @@ int blocks_of(int kind, const ramgpu_ctx *c) {
 
 bool per_member(int kind) { return kind == BK_SCHED || kind == BK_COEFIJ || kind == BK_MEM || kind == BK_COPY; }
 
-// Job table and block map of one kernel kind, members in order.
+// Job table and block map of one kernel kind, members in order; the plane
+// kinds with the members of one plane-kernel shape together.
 int build_plan(ramgpu_batch *b, int kind) {
   std::vector<Job> jobs;
   std::vector<int> vmap;
-  for (size_t mi = 0; mi < b->m.size(); ++mi) {
+  const bool plane = kind == BK_PLANE || kind == BK_PLOOP;
+  std::vector<size_t> order(b->m.size());
+  std::iota(order.begin(), order.end(), size_t(0));
+  auto shape = [&](size_t mi) { return std::make_pair(b->m[mi]->step.rows, b->m[mi]->step.threads); };
+  if (plane)
+    std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) { return shape(x) < shape(y); });
+  std::vector<Plan::Group> groups;
+  for (size_t o = 0; o < order.size(); ++o) {
+    const size_t mi = order[o];
     const ramgpu_ctx *c = b->m[mi];
+    if (plane && (o == 0 || shape(order[o - 1]) != shape(mi)))
+      groups.push_back(Plan::Group{c->step, 0, (int)vmap.size(), 0});
+    if (plane) groups.back().lds = std::max(groups.back().lds, step_lds_bytes(c->ne, c->npa, c->step.rows));
     const int nsp = per_member(kind) ? 1 : c->ns;
     const int nb = blocks_of(kind, c);
     if (nb >= (1 << kVmapShift) || jobs.size() + nsp >= (1u << (31 - kVmapShift)))
@@ -117,7 +138,9 @@ int build_plan(ramgpu_batch *b, int kind) {
       for (int s = 0; s < nsp; ++s)
         for (int x = 0; x < nb; ++x) vmap.push_back(vmap_entry(j0 + s, x));
     }
+    if (plane) groups.back().nv = (int)vmap.size() - groups.back().v0;
   }
+  b->plan[kind].groups = groups;
   Plan &p = b->plan[kind];
   int rc;
   if ((rc = batch_alloc(b, (void **)&p.jobs, jobs.size() * sizeof(Job))) ||
@@ -142,6 +165,18 @@ Launch launch_for(const ramgpu_batch *b, int kind) {
 unsigned grid_for(const ramgpu_batch *b, int kind) {
   const Plan &p = b->plan[kind];
   return (unsigned)((p.cap > 0 && p.cap < p.nv) ? p.cap : p.nv);
+}
+
+// The fused plane kernel of every member: one launch per shape.
+void enq_planes(ramgpu_batch *b, int kind, int seq, Launch L, int rec) {
+  const Plan &p = b->plan[kind];
+  const int *vmap = L.vmap;
+  for (const Plan::Group &g : p.groups) {
+    L.vmap = vmap + g.v0;
+    L.nv = g.nv;
+    const int grid = (p.cap > 0 && p.cap < g.nv) ? p.cap : g.nv;
+    launch_step(seq, g.sh, dim3((unsigned)grid), g.lds, b->stream, L, rec);
+  }
 }
 
 void destroy_graphs(ramgpu_batch *b) {
@@ -224,7 +259,7 @@ int enqueue_step(ramgpu_batch *b, bool sched) {
   hipLaunchKernelGGL(k_p<1>, dim3(grid_for(b, BK_P)), dim3(kLineThreads), b->azim_lds, st, lp);
   btend(b);
   btbeg(b, RAMGPU_KERNEL_PLANE);
-  launch_plane(SEQ_STEP, b->plane, dim3(grid_for(b, BK_PLANE)), b->plane_lds, st, lk, 1);
+  enq_planes(b, BK_PLANE, SEQ_STEP, lk, 1);
   btend(b);
   btbeg(b, RAMGPU_KERNEL_P);
   hipLaunchKernelGGL(k_p<0>, dim3(grid_for(b, BK_P)), dim3(kLineThreads), b->azim_lds, st, lp);
@@ -296,7 +331,7 @@ void enq_taped_step(ramgpu_batch *b, int g, int dsl_out, bool bookkeeping = true
   else
     hipLaunchKernelGGL(k_p<0>, dim3(L.nv), dim3(kLineThreads), b->azim_lds, st, L);
   L = slot_launch(b, BK_PLOOP, g + T_E1 + 1, g + T_P2 + 1);
-  launch_plane(SEQ_TAPE, b->plane, dim3(L.nv), b->plane_lds, st, L, bookkeeping ? 1 : 0);
+  enq_planes(b, BK_PLOOP, SEQ_TAPE, L, bookkeeping ? 1 : 0);
   L = slot_launch(b, BK_POOP, g + T_P2 + 1, g + T_R2 + 1);
   hipLaunchKernelGGL(k_p<0>, dim3(L.nv), dim3(kLineThreads), b->azim_lds, st, L);
   L = slot_launch(b, BK_R, g + T_R2 + 1, dsl_out);
@@ -450,25 +485,9 @@ int ramgpu_batch_create(ramgpu_batch **out, ramgpu_ctx *const *members, int nmem
     b->azim_lds = std::max(b->azim_lds, azim_lds_bytes(c->nt, c->ne, c->npa));
     b->ghost_lds = std::max(b->ghost_lds, (size_t)4 * c->nt * sizeof(double));
     b->plane.threads = std::max(b->plane.threads, c->plane.threads);
+    b->plane.maxc = std::max(b->plane.maxc, c->plane.maxc);
     b->wave.push_back((char)takes_wave(c));
   }
-  // one block size for all members, the largest any member chose: each
-  // member keeps its own rows per thread (its Tab's plane_chunks), so its
-  // planes are swept exactly as when it runs alone; the threads above its
-  // chunks are idle
-  {
-    size_t lds = 0;
-    int maxc = 8;
-    for (ramgpu_ctx *c : b->m) {
-      maxc = std::max(maxc, c->plane.maxc);
-      lds = std::max(lds, plane_fwd_lds_bytes(c->ne, c->npa, b->plane.threads));
-    }
-    if (lds > b->m[0]->lds_limit) return cleanup(fail(RAMGPU_EINVAL, "the members' planes do not fit one block's LDS"));
-    b->plane = {b->plane.threads, maxc, 0};
-    b->plane_lds = lds;
-  }
-
-
   if ((rc = batch_alloc(b, (void **)&b->d_bsoff, nmembers * sizeof(int))) ||
       (rc = batch_alloc(b, (void **)&b->d_step, sizeof(int))))
     return cleanup(rc);
@@ -824,7 +843,7 @@ int ramgpu_batch_autotune(ramgpu_batch *b, int reps, double *ms_best) {
         else if (kind == BK_P)
           hipLaunchKernelGGL(k_p<0>, dim3(grid_for(b, kind)), dim3(kLineThreads), b->azim_lds, b->stream, L);
         else
-          launch_plane(SEQ_STEP, b->plane, dim3(grid_for(b, kind)), b->plane_lds, b->stream, L, 0);
+          enq_planes(b, kind, SEQ_STEP, L, 0);
         (void)hipEventRecord(e1, b->stream);
         if (hipEventSynchronize(e1) != hipSuccess) {
           rc = fail(RAMGPU_EHIP, "autotune launch failed");

@@ -35,6 +35,7 @@ __global__ void k_ghost(Launch L);
 template <int MODE> __global__ void k_r(Launch L);
 template <int MODE> __global__ void k_p(Launch L);
 template <int SEQ, int MAXC> __global__ void k_plane(Launch L, int rec);
+template <int SEQ, int R> __global__ void k_plane_step(Launch L, int rec);
 __global__ void k_finalize(Launch L, int cflmask, int summode);
 __global__ void k_vs(double *vt, const double *lz, const double *phi, const double *kp_ptr,
                      double kp_val, int nr1, int nt, const double *bs_src, double *bs_dst, int ns);
@@ -51,6 +52,11 @@ struct PlaneShape {
   int threads, maxc, rows;  // block size, row bound (template) and rows per thread of the forward plane kernels
 };
 
+// block size and rows per thread of the fused step's plane kernel (k_plane_step)
+struct StepShape {
+  int threads, rows;
+};
+
 struct ramgpu_ctx {
   int device = 0;
   int ns = 0, nr = 0, nt = 0, ne = 0, npa = 0;
@@ -63,6 +69,7 @@ struct ramgpu_ctx {
   double last_ms = 0.0;
   size_t lds_limit = 65536;
   PlaneShape plane{ramgpu::kPlaneThreads, 16, 0};
+  StepShape step{0, 0};
   Tab t{};            // host image of the problem descriptor
   Tab *d_tab = nullptr;  // its device copy, read by every kernel
   bool tab_dirty = true;
@@ -155,6 +162,9 @@ PlaneShape plane_shape(int ne, int npa, size_t lds_cu);
 int coef_units(const ramgpu_ctx *c, int threads);
 bool takes_wave(const ramgpu_ctx *c);
 PlaneShape plane_shape_for(int ne, int npa, int threads);
+StepShape step_shape(int ne, int npa, long planes, int ncu, size_t lds_cu);
+// launch k_plane_step<seq, rows>
+void launch_step(int seq, StepShape sh, dim3 grid, size_t lds, hipStream_t st, const ramgpu::Launch &L, int rec);
 // launch k_plane<seq, maxc>
 void launch_plane(int seq, PlaneShape sh, dim3 grid, size_t lds, hipStream_t st, const ramgpu::Launch &L, int rec);
 // tape slots: the inputs of the operators of one ram_run step, in order

@@ -85,6 +85,15 @@ __global__ void k_species(Launch L) {
           sv = pow(10.0, y) * t.v[s + t.ns * k];
         }
         t.sigv[s * t.ne + k] = sv;
+        double *kt = t.kt + (size_t)s * SKT_N * t.ne + k;
+        kt[SKT_EKPQ * t.ne] = t.ekp[s * t.ne + k] * qs;
+        kt[SKT_MKPQ * t.ne] = t.mkp[s * t.ne + k] * qs;
+        kt[SKT_SIGV * t.ne] = sv;
+        kt[SKT_DE * t.ne] = t.de[k];
+        kt[SKT_RDE * t.ne] = 1.0 / t.de[k];
+        kt[SKT_WE * t.ne] = t.we[k];
+        kt[SKT_RWE * t.ne] = 1.0 / t.we[k];
+        kt[SKT_EKW * t.ne] = ekev * t.we[k];
       }
     }
     if (threadIdx.x == 0) {
@@ -97,6 +106,8 @@ __global__ void k_species(Launch L) {
       rel[2] = sqrt((g2 * g2 - 1.0) / (g1 * g1 - 1.0));
       rel[3] = grzero;
       rel[4] = sqrt((g1 * g1 - 1.0) / (grzero * grzero - 1.0));
+      rel[5] = 1.0 / g2;
+      rel[6] = 1.0 / g1;
     }
     if (s == 0) {
       for (int k = threadIdx.x; k < t.ne; k += blockDim.x) {
@@ -106,6 +117,10 @@ __global__ void k_species(Launch L) {
       for (int l = threadIdx.x; l < t.npa; l += blockDim.x) {
         t.rdmu[l] = 1.0 / t.dmu[l];
         t.rwmu[l] = 1.0 / t.wmu[l];
+        t.lt4[4 * l] = t.dmu[l];
+        t.lt4[4 * l + 1] = 1.0 / t.dmu[l];
+        t.lt4[4 * l + 2] = t.wmu[l];
+        t.lt4[4 * l + 3] = 1.0 / t.wmu[l];
       }
     }
   }
@@ -793,45 +808,6 @@ struct FwdCtx {
   int cst;
 };
 
-// x, hidden from the optimiser: row indices derived from it are formed
-// afresh in each phase instead of being kept in registers across phases.
-__device__ __forceinline__ int fresh(int x) {
-  asm volatile("" : "+v"(x));
-  return x;
-}
-
-// The value of x in lane `lane` of the wave (a wave-uniform value).
-__device__ __forceinline__ double lane_value(double x, int lane) {
-  const long long b = __double_as_longlong(x);
-  const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffLL), lane);
-  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-
-// A block-uniform x (read from LDS) held in scalar registers.
-__device__ __forceinline__ double uniform(double x) {
-  const long long b = __double_as_longlong(x);
-  const int lo = __builtin_amdgcn_readfirstlane((int)(b & 0xffffffffLL));
-  const int hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-
-// x, formed here: keeps the compiler from sinking the arithmetic that
-// makes a row's result down to the barrier, where it would hold every
-// operand of every row instead of one result per row.
-__device__ __forceinline__ double settle(double x) {
-  asm("" : "+v"(x));
-  return x;
-}
-
-// The value of v in lane-1 (lane 0: -0.0, which adds as an exact zero).
-__device__ __forceinline__ double from_lane_below(double v) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffLL), 0x138 /* wave_shr:1 */, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp((int)0x80000000, (int)(b >> 32), 0x138, 0xf, 0xf, false);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-
 // Block set-up: the context of plane b of species s, this thread's cells
 // (from src, device layout of one species) and the plane's tables.
 template <int MAXC>
@@ -906,11 +882,8 @@ constexpr int kPassRows = 8;
 // upwind sweep with CccolE(K) = (COULE+COULI)(S,K,L)*XNE(L), its own ghost
 // factors (the square roots of the inverse ratios of DRIFTE's) and rows
 // L=2..NPA only.
-//
-// TAPE: also write each updated cell's clamp decision (1: the forward
-// clamped it) to cb (this plane's bytes, [L][K]), for the adjoint.
-template <int MAXC, bool COUL = false, bool TAPE = false>
-__device__ void plane_e(const Tab &t, const FwdCtx &c, const PlaneFwd &d, bool rec, unsigned char *cb = nullptr) {
+template <int MAXC, bool COUL = false>
+__device__ void plane_e(const Tab &t, const FwdCtx &c, const PlaneFwd &d, bool rec) {
   const int NE = c.NE, NPA = c.NPA, S = c.S;
   if (COUL) rec = false;
   {
@@ -975,7 +948,6 @@ __device__ void plane_e(const Tab &t, const FwdCtx &c, const PlaneFwd &d, bool r
         if (j >= c.nr) break;
         double w = v[n];
         if (first) w = w + xw[n - kPassRows];
-        if (TAPE) cb[(l0 + j) * NE + k] = (w < 0) ? 1 : 0;
         if (w < 0) w = 1E-15;
         if (!COUL || l0 + j >= 1) c.col[(l0 + j) * S] = w;
       }
@@ -998,9 +970,8 @@ __device__ void plane_e(const Tab &t, const FwdCtx &c, const PlaneFwd &d, bool r
 // read before any row is rewritten; the chunk's first row takes the term
 // of the chunk below after the last pass, and the top row is set last
 // from the finished row below it (the same thread's, by plane_chunks_for).
-// TAPE: as plane_e's.
-template <int MAXC, bool TAPE = false>
-__device__ void plane_mu(const Tab &t, const FwdCtx &c, const PlaneFwd &d, bool rec, unsigned char *cb = nullptr) {
+template <int MAXC>
+__device__ void plane_mu(const Tab &t, const FwdCtx &c, const PlaneFwd &d, bool rec) {
   const int NE = c.NE, NPA = c.NPA;
   if (rec) {
     for (int l = threadIdx.x; l < kMuSpread * NPA; l += blockDim.x) d.cmx[NE + l] = 0ull;
@@ -1066,7 +1037,6 @@ __device__ void plane_mu(const Tab &t, const FwdCtx &c, const PlaneFwd &d, bool 
       if (j >= nr) break;
       if (j >= 1 && l <= NPA - 2) {
         double w = v[n];
-        if (TAPE) cb[l * NE + k] = (w < 0) ? 1 : 0;
         if (w < 0) w = 1E-15;
         col[l * cst] = w;
       }
@@ -1076,7 +1046,6 @@ __device__ void plane_mu(const Tab &t, const FwdCtx &c, const PlaneFwd &d, bool 
   // plane, the first chunk's, is not updated)
   if (c.nr > 0 && c.q >= 1) {
     double w = v0 + d.X[threadIdx.x - NE];
-    if (TAPE) cb[l0 * NE + k] = (w < 0) ? 1 : 0;
     if (w < 0) w = 1E-15;
     col[l0 * cst] = w;
   }
@@ -1336,10 +1305,8 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, 4) k_plane(Launch L, int rec
       block_copy<8>(dst, src, NE * NPA);
       continue;
     }
-    constexpr bool need_loss = SEQ == SEQ_CEX || SEQ == SEQ_ATM || SEQ == SEQ_STEP || SEQ == SEQ_LOSS ||
-                               SEQ == SEQ_TAPE || SEQ == SEQ_WAVE || SEQ == SEQ_STEPC;
-    constexpr bool need_kl = SEQ == SEQ_E || SEQ == SEQ_MU || SEQ == SEQ_STEP || SEQ == SEQ_TAPE ||
-                             SEQ == SEQ_STEPC;
+    constexpr bool need_loss = SEQ == SEQ_CEX || SEQ == SEQ_ATM || SEQ == SEQ_WAVE || SEQ == SEQ_STEPC;
+    constexpr bool need_kl = SEQ == SEQ_E || SEQ == SEQ_MU || SEQ == SEQ_STEPC;
     FwdCtx c;
     PlaneFwd d;
     fwd_setup<MAXC>(t, u, sm, launch_src(L, t), need_loss, need_kl, c, d);
@@ -1392,36 +1359,6 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, 4) k_plane(Launch L, int rec
       plane_sum_slot<MAXC>(t, c, d, u.b, kSumCoul + 2);
       plane_e<MAXC, true>(t, c, d, false);
       plane_sum_slot<MAXC>(t, c, d, u.b, kSumCoul + 3);
-      plane_mu<MAXC>(t, c, d, false);
-      plane_e<MAXC>(t, c, d, false);
-    } else if constexpr (SEQ == SEQ_LOSS) {
-      plane_loss<MAXC>(t, c, d, u.b);
-    } else if constexpr (SEQ == SEQ_TAPE) {
-      // src is tape slot 0 (this phase's input); phase m's output, the input
-      // of phase m+1, goes to slot m+1, the last to dst.  A thread stores
-      // its own cells, which only it writes.
-      // The clamp decisions of the four drift phases go to the bytes of the
-      // tape slot 7 after slot 0, one byte plane per phase.
-      const size_t ns = f2_elems(t);
-      double *slot = const_cast<double *>(launch_src(L, t)) + po;
-      unsigned char *cb = reinterpret_cast<unsigned char *>(const_cast<double *>(launch_src(L, t)) + 7 * ns) + po;
-      // each phase ends with a barrier, so its output is whole in LDS; the
-      // loss chain rewrites cells at once, so a barrier follows the store
-      // before it (the later phases rewrite cells only after barriers)
-      plane_e<MAXC, false, true>(t, c, d, rec_here, cb);
-      fwd_store(c, d, t.rne, slot + ns);
-      plane_mu<MAXC, true>(t, c, d, rec_here, cb + ns);
-      fwd_store(c, d, t.rne, slot + 2 * ns);
-      __syncthreads();
-      plane_loss<MAXC>(t, c, d, u.b);
-      fwd_store(c, d, t.rne, slot + 3 * ns);
-      plane_mu<MAXC, true>(t, c, d, false, cb + 2 * ns);
-      fwd_store(c, d, t.rne, slot + 4 * ns);
-      plane_e<MAXC, false, true>(t, c, d, false, cb + 3 * ns);
-    } else {  // SEQ_STEP
-      plane_e<MAXC>(t, c, d, rec_here);
-      plane_mu<MAXC>(t, c, d, rec_here);
-      plane_loss<MAXC>(t, c, d, u.b);
       plane_mu<MAXC>(t, c, d, false);
       plane_e<MAXC>(t, c, d, false);
     }
@@ -1863,17 +1800,11 @@ template __global__ void k_plane<SEQ_MU, 8>(Launch, int);
 template __global__ void k_plane<SEQ_CEX, 8>(Launch, int);
 template __global__ void k_plane<SEQ_ATM, 8>(Launch, int);
 template __global__ void k_plane<SEQ_SUM, 8>(Launch, int);
-template __global__ void k_plane<SEQ_STEP, 8>(Launch, int);
-template __global__ void k_plane<SEQ_LOSS, 8>(Launch, int);
-template __global__ void k_plane<SEQ_TAPE, 8>(Launch, int);
 template __global__ void k_plane<SEQ_E, 16>(Launch, int);
 template __global__ void k_plane<SEQ_MU, 16>(Launch, int);
 template __global__ void k_plane<SEQ_CEX, 16>(Launch, int);
 template __global__ void k_plane<SEQ_ATM, 16>(Launch, int);
 template __global__ void k_plane<SEQ_SUM, 16>(Launch, int);
-template __global__ void k_plane<SEQ_STEP, 16>(Launch, int);
-template __global__ void k_plane<SEQ_LOSS, 16>(Launch, int);
-template __global__ void k_plane<SEQ_TAPE, 16>(Launch, int);
 template __global__ void k_plane<SEQ_COULEN, 8>(Launch, int);
 template __global__ void k_plane<SEQ_COULEN, 16>(Launch, int);
 template __global__ void k_plane<SEQ_COULMU, 8>(Launch, int);

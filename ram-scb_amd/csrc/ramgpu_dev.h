@@ -52,6 +52,10 @@ enum KleField { KLE_HS, KLE_RHS, KLE_DRD2, KLE_DPD2, KLE_GR, KLE_GP, KLE_DB1, KL
 // packed per-(I,J,L) DRIFTMU terms, klm[((i*NT+j)*NPA+l)*8 + ..]
 enum KlmField { KLM_BHS, KLM_RBHS, KLM_DRM2, KLM_DPM2, KLM_CMUDOT, KLM_GMR, KLM_GMP, KLM_DI2 };
 
+// per-species per-K terms of the plane step, kt[(s*SKT_N + field)*NE + k]; the
+// charge's sign is folded into EKP and MKP (x/QS == x*QS for QS = +-1)
+enum StepKt { SKT_EKPQ, SKT_MKPQ, SKT_SIGV, SKT_DE, SKT_RDE, SKT_WE, SKT_RWE, SKT_EKW, SKT_N };
+
 // All device pointers and scalars of one problem (one ensemble member).
 // Lives in device memory; kernels read it through a pointer.
 struct Tab {
@@ -92,7 +96,9 @@ struct Tab {
   double *edot;   // [s][i][k]
   double *sigv;   // [s][k] 10**Y*V(S,K) of CEPARA
   double *atlos;  // [s][i][k]
-  double *rel;    // [s][8]: GREL1, GREL2, sq1, GRZERO, sq0
+  double *rel;    // [s][8]: GREL1, GREL2, sq1, GRZERO, sq0, 1/GREL2, 1/GREL1
+  double *kt;     // [s][8][k] the plane step's per-K terms (StepKt)
+  double *lt4;    // [l][4] DMU, 1/DMU, WMU, 1/WMU
   int *carry;     // [s][NE*NPA] DRIFTR ghost carry
   double *latl;   // [s][i][k] log(ATLOS): ATLOS**(1/FNHS) = exp(log(ATLOS)/FNHS)
   // WAVELO (electron lifetimes) of the species with wpi[s] set: WALOS1/2/3
@@ -127,6 +133,7 @@ struct Tab {
   // owns K = n%NE of the rows of chunk n/NE (plane_chunks_for); the
   // threads above, in a block of any size, are idle
   int plane_chunks;
+  int step_cells, step_apart;  // step_wave_cells, step_edges_apart of k_plane_step's shape
   // state
   double *f2;
   double *partials;  // [slot][s][maxblk]
@@ -175,16 +182,19 @@ struct Launch {
   int bstep;  // reverse mode of an ensemble: the step whose FGEOS adjoint (Tab::bbar) DRIFTR's adjoint feeds
 };
 
-inline __host__ __device__ size_t f2_species_stride(const Tab &t) {
+template <class T>
+inline __host__ __device__ size_t f2_species_stride(const T &t) {
   return (size_t)t.nr * t.nt * t.npa * t.ne;
 }
 
 // the input and output F2 of a launch for problem t, and whether they differ
-inline __host__ __device__ const double *launch_src(const Launch &L, const Tab &t) {
+template <class T>
+inline __host__ __device__ const double *launch_src(const Launch &L, const T &t) {
   if (L.ssl > 0) return t.tape + (size_t)(L.ssl - 1) * t.ns * f2_species_stride(t);
   return L.src ? L.src : t.f2;
 }
-inline __host__ __device__ double *launch_dst(const Launch &L, const Tab &t) {
+template <class T>
+inline __host__ __device__ double *launch_dst(const Launch &L, const T &t) {
   if (L.dsl > 0) return t.tape + (size_t)(L.dsl - 1) * t.ns * f2_species_stride(t);
   if (L.dsl < 0) return t.f2;
   return L.dst ? L.dst : t.f2;
@@ -192,13 +202,16 @@ inline __host__ __device__ double *launch_dst(const Launch &L, const Tab &t) {
 inline __host__ __device__ bool out_of_place(const Launch &L) { return L.dsl != 0 || (L.dst && L.dst != L.src); }
 
 // block counts of the kernels, per (problem, species)
-inline __host__ __device__ int blocks_r(const Tab &t) {
+template <class T>
+inline __host__ __device__ int blocks_r(const T &t) {
   return (t.nt * t.ne * t.npa + kLineThreads - 1) / kLineThreads;
 }
-inline __host__ __device__ int blocks_p(const Tab &t) {
+template <class T>
+inline __host__ __device__ int blocks_p(const T &t) {
   return ((t.nr - 1) * t.ne * t.npa + kLineThreads - 1) / kLineThreads;
 }
-inline __host__ __device__ int blocks_kl(const Tab &t) { return (t.nr - 1) * t.nt; }
+template <class T>
+inline __host__ __device__ int blocks_kl(const T &t) { return (t.nr - 1) * t.nt; }
 
 // LDS bytes of the azimuthal sweep: pl of a block's (I,L) pairs and pij of
 // its I values
@@ -242,6 +255,43 @@ inline __host__ __device__ size_t plane_fwd_lds_bytes(int ne, int npa, int threa
   return ((size_t)npa * (ne + 3) + (size_t)npa + (size_t)threads + 16 * (size_t)npa + 2 * (size_t)npa +
           11 * (size_t)ne + 4 * (size_t)npa + 128 + 64 + 24 + (size_t)ne + (size_t)kMuSpread * npa) *
          sizeof(double);
+}
+// Mapping and LDS of the fused step's plane kernel (k_plane_step).  Q =
+// ceil(NPA/R) chunks of R rows of NE threads; a wave takes step_wave_cells
+// of the Q*NE columns: 64 where no chunk straddles two waves, else 63, lane 0
+// repeating the last column of the wave before.
+constexpr size_t kLdsCu = 160 * 1024;  // gfx950
+inline __host__ __device__ int step_chunks(int npa, int rows) { return (npa + rows - 1) / rows; }
+inline __host__ __device__ int step_wave_cells(int ne) { return 64 % ne == 0 ? 64 : 63; }
+inline __host__ __device__ int step_threads(int ne, int npa, int rows) {
+  const int w = step_wave_cells(ne);
+  return (step_chunks(npa, rows) * ne + w - 1) / w * 64;
+}
+constexpr int kStepSpread = 2;  // LDS slots per row of DRIFTMU's CFL maximum (by K mod 2)
+constexpr int kStepSimdWaves = 4;  // waves per SIMD that the kernel's registers leave room for
+// Its LDS in doubles: the plane's rows of NE+3 energy-stencil positions, the
+// per-L terms (21 NPAP + 5), 10 per-K terms, the exponential's table, 112
+// wave sums, the CFL slots; and 4*Q*NE doubles at the chunks' edges, in the
+// rows' place (behind a further barrier) where they would cost a CU a block.
+inline __host__ __device__ size_t step_lds_doubles(int ne, int npa, int rows) {
+  const size_t q = step_chunks(npa, rows), npap = q * rows, plane = npap * (ne + 3), edges = 4 * q * ne;
+  return (plane > edges ? plane : edges) + 1 + 21 * npap + 5 + 10 * (size_t)ne + 64 + 112 + ne +
+         (size_t)kStepSpread * npa;
+}
+// Blocks a CU holds with `lds` bytes each: a block's waves go to the SIMDs in
+// turn from the first, so a SIMD takes ceil(waves/4) of each.
+inline __host__ __device__ int step_resident(size_t lds, int ne, int npa, int rows) {
+  const int simd = (step_threads(ne, npa, rows) / 64 + 3) / 4;
+  const int by_waves = kStepSimdWaves / simd, by_lds = (int)(kLdsCu / lds);
+  return by_waves < by_lds ? by_waves : by_lds;
+}
+inline __host__ __device__ bool step_edges_apart(int ne, int npa, int rows) {
+  const size_t base = step_lds_doubles(ne, npa, rows) * 8, edges = 4 * (size_t)step_chunks(npa, rows) * ne * 8;
+  return step_resident(base + edges, ne, npa, rows) >= step_resident(base, ne, npa, rows);
+}
+inline __host__ __device__ size_t step_lds_bytes(int ne, int npa, int rows) {
+  return step_lds_doubles(ne, npa, rows) * 8 +
+         (step_edges_apart(ne, npa, rows) ? 4 * (size_t)step_chunks(npa, rows) * ne * 8 : 0);
 }
 // The Coulomb operators' LDS after the forward plane kernels': per L the
 // bounce-averaged density XNE, BASCNE, FNHS, BOUNHS, MU, 1/FNHS and 1/MU

@@ -91,6 +91,38 @@ __device__ __forceinline__ double face_value_sel(double f0, double fp1, double f
   return (fabs(x) <= 1.E-27 || r <= 0) ? fup : v;
 }
 
+// a/x, correctly rounded: the reciprocal from the hardware's by one cubic
+// iteration, the quotient by the residual correction of div_rn.  It is the
+// compiler's own division without its scaling of extreme exponents, so the
+// result is a/x for |x| within 2^-900..2^900 and quotients in the normal
+// range (F2 and its differences); infinities, NaN and zeros are set right
+// by the last instruction.  8 instead of 11 VALU instructions.
+__device__ __forceinline__ double div_fast(double a, double x) {
+  double y = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, y, 1.0);
+  y = fma(y, fma(e, e, e), y);
+  double q = a * y;
+  q = fma(fma(-x, q, a), y, q);
+  return __builtin_amdgcn_div_fixup(q, x, a);
+}
+
+// Twice the face value of face_value, for callers that fold the factor 1/2
+// into the next product: f0 = F(I), fp1 = F(I+1), p and a the upwind pair
+// (F(I), F(I-1)) or, for C < 0 (neg), (F(I+1), F(I+2)), so that R =
+// (p-a)/(sgn*X); cn as in face_value.  Every product with sgn or 1/2 is
+// exact, so the roundings are face_value's: 0.5*u2 is its value bit for bit.
+__device__ __forceinline__ double face_value2(double f0, double fp1, double p, double a, bool neg, double cn,
+                                              double beta) {
+  const double sg = neg ? -1.0 : 1.0;
+  const double x = fp1 - f0;
+  const double sx = sg * x;
+  const double t = (f0 + fp1) - sx;  // 2 FUP
+  const double r = div_fast(p - a, sx);
+  const double lim = fmax(fmin(beta * r, 1.0), fmin(r, beta));
+  const double y = lim * ((cn - sg) * x);  // -2 LIM*CORR
+  return t - ((fabs(x) <= 1.E-27 || r <= 0) ? 0.0 : y);
+}
+
 // The same face value with its partial derivatives with respect to the four
 // stencil values (reverse mode).  fb = FUP + lim(R)*CORR is piecewise linear:
 // on each piece lim = a + b*R, so with kap = -0.5*(cn-sg), X = fp1-f0,
@@ -140,6 +172,18 @@ template <class T>
 __device__ __forceinline__ gptr<T> as_global(T *p) {
   return (gptr<T>)p;
 }
+// Constant-memory views: uniform loads through them are scalar loads at any
+// point of a kernel (memory no kernel writes while it reads it: the problem
+// descriptor, the tables earlier launches formed).  Through a generic pointer
+// the compiler must assume that the kernel's own stores change them, and
+// reads every descriptor field by a vector load before the load it points to.
+template <class T>
+using cptr = const __attribute__((address_space(4))) T *;
+template <class T>
+__device__ __forceinline__ cptr<T> as_const(const T *p) {
+  return (cptr<T>)(unsigned long long)p;
+}
+typedef const __attribute__((address_space(4))) Tab CTab;
 // element n of a double4 / double2 table read through a global view
 __device__ __forceinline__ double4 ld_d4(gptr<const double> p, size_t n) {
   const gptr<const double> q = p + 4 * n;
@@ -148,6 +192,71 @@ __device__ __forceinline__ double4 ld_d4(gptr<const double> p, size_t n) {
 __device__ __forceinline__ double2 ld_d2(gptr<const double> p, size_t n) {
   const gptr<const double> q = p + 2 * n;
   return make_double2(q[0], q[1]);
+}
+
+// x, hidden from the optimiser: row indices derived from it are formed
+// afresh in each phase instead of being kept in registers across phases.
+__device__ __forceinline__ int fresh(int x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
+// The value of x in lane `lane` of the wave (a wave-uniform value).
+__device__ __forceinline__ double lane_value(double x, int lane) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffLL), lane);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// A block-uniform x (read from LDS) held in scalar registers.
+__device__ __forceinline__ double uniform(double x) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_readfirstlane((int)(b & 0xffffffffLL));
+  const int hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// x, formed here: keeps the compiler from sinking the arithmetic that
+// makes a row's result down to the barrier, where it would hold every
+// operand of every row instead of one result per row.
+__device__ __forceinline__ double settle(double x) {
+  asm("" : "+v"(x));
+  return x;
+}
+
+// The value of v in lane-1 (lane 0: -0.0, which adds as an exact zero).
+__device__ __forceinline__ double from_lane_below(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffLL), 0x138 /* wave_shr:1 */, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp((int)0x80000000, (int)(b >> 32), 0x138, 0xf, 0xf, false);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// The value of v in lane-1 (lane 0: 0).
+__device__ __forceinline__ double from_lane_below0(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffLL), 0x138 /* wave_shr:1 */, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x138, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// v plus the v of the lanes that one DPP control moves in (0 elsewhere).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffLL), CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);
+  return v + __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+// The wave's sum of v, in lane 63 (rows of 16 by shifts, then across rows).
+__device__ __forceinline__ double wave_sum(double v) {
+  v = dpp_add<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);  // row_bcast:15
+  return dpp_add<0x143, 0xc>(v);  // row_bcast:31
 }
 
 // ---------------------------------------------------------------------------
@@ -172,6 +281,21 @@ __device__ __forceinline__ Unit unit_of(const Launch &L, int vb) {
   const int e = L.vmap[vb];
   const Job jb = L.jobs[e >> kVmapShift];
   return {L.tabs + jb.tab, jb.s, e & ((1 << kVmapShift) - 1)};
+}
+
+// The unit of virtual block vb with the descriptor in constant memory.
+struct CUnit {
+  CTab *t;
+  int s, b;
+};
+__device__ __forceinline__ CUnit const_unit(const Launch &L, int vb) {
+  if (!L.vmap) {
+    const Unit u = unit_of(L, vb);
+    return {as_const(L.tabs), u.s, u.b};
+  }
+  const int e = as_const(L.vmap)[vb];
+  const cptr<Job> jb = as_const(L.jobs) + (e >> kVmapShift);
+  return {as_const(L.tabs) + jb->tab, jb->s, e & ((1 << kVmapShift) - 1)};
 }
 
 // ---------------------------------------------------------------------------
@@ -417,9 +541,9 @@ enum PlaneSeq : int {
   SEQ_CEX = 2,   // CHAREXCHANGE
   SEQ_ATM = 3,   // ATMOL
   SEQ_SUM = 4,   // SUMRC partial sum, slot 0
-  SEQ_STEP = 5,  // the middle of ram_run: DRIFTE, DRIFTMU, loss chain, DRIFTMU, DRIFTE
-  SEQ_LOSS = 6,  // the loss chain alone (WAVELO, CEX, ATMOL, ATMOL, CEX, WAVELO with seven SUMRC partials)
-  SEQ_TAPE = 7,  // SEQ_STEP out of place, also writing the input of each later phase to a tape
+  SEQ_STEP = 5,  // the middle of ram_run: DRIFTE, DRIFTMU, loss chain, DRIFTMU, DRIFTE (k_plane_step)
+  SEQ_LOSS = 6,  // the loss chain alone (plane adjoints)
+  SEQ_TAPE = 7,  // SEQ_STEP out of place, also writing the input of each later phase to a tape (k_plane_step)
   SEQ_WAVE = 8,  // WAVELO
   SEQ_COULEN = 9,   // COULEN
   SEQ_COULMU = 10,  // COULMU

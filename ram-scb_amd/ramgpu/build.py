@@ -7,6 +7,8 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -18,9 +20,11 @@ LIB = PKG / "libramgpu.so"
 
 HIP_SOURCES = ["kernels.hip", "api.hip", "batch.hip", "adjoint.hip", "adjoint_api.hip", "moments.hip",
                "coulomb.hip", "pitch.hip", "bounce.hip"]
+# sources compiled once per part: (source, macro, parts)
+HIP_PARTS = [("plane_step.hip", "STEP_PART", 5)]
 
 HIPCC_FLAGS = [
-    "--offload-arch=gfx950", "-O3", "-fPIC", "-shared", "-std=c++17",
+    "--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17",
     # no packed FP32 instructions anywhere in the device code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-ffp-contract=off", "-Wall",
@@ -34,20 +38,34 @@ def hipcc() -> str:
     raise FileNotFoundError("hipcc not found")
 
 
-def build_library(verbose: bool = False) -> Path:
-    srcs = [str(CSRC / s) for s in HIP_SOURCES]
-    tmp = LIB.with_suffix(".so.tmp")
-    cmd = [hipcc(), *HIPCC_FLAGS, f"-I{INCLUDE}", f"-I{CSRC}", *srcs, "-o", str(tmp)]
+def _run(cmd, verbose: bool = False):
     if verbose:
         print(" ".join(cmd), flush=True)
     r = subprocess.run(cmd, capture_output=True, text=True)
-    noise = "is not a recognized feature for this target"
-    err = "\n".join(l for l in r.stderr.splitlines() if noise not in l)
+    noise = ("is not a recognized feature for this target", "argument unused during compilation")
+    err = "\n".join(l for l in r.stderr.splitlines() if not any(n in l for n in noise))
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed ({r.returncode}):\n{err}")
     if verbose and err.strip():
         print(err)
-    os.replace(tmp, LIB)
+
+
+def build_library(verbose: bool = False) -> Path:
+    """Compiles every source (and every part of the split ones) side by side,
+    then links the library."""
+    cc = [hipcc(), *HIPCC_FLAGS, f"-I{INCLUDE}", f"-I{CSRC}"]
+    units = [(s, Path(s).stem, []) for s in HIP_SOURCES]
+    units += [(s, f"{Path(s).stem}_{n}", [f"-D{macro}={n}"]) for s, macro, parts in HIP_PARTS for n in range(parts)]
+    with tempfile.TemporaryDirectory(prefix="ramgpu_build_") as tmp:
+        objs = [str(Path(tmp) / f"{name}.o") for _, name, _ in units]
+        jobs = [[*cc, *defs, "-c", str(CSRC / src), "-o", obj] for (src, _, defs), obj in zip(units, objs)]
+        workers = max(1, min(8, os.cpu_count() or 1, int(os.environ.get("MAX_JOBS") or 8)))
+        with ThreadPoolExecutor(workers) as pool:
+            for f in [pool.submit(_run, j, verbose) for j in jobs]:
+                f.result()
+        out = LIB.with_suffix(".so.tmp")
+        _run([hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", str(out)], verbose)
+    os.replace(out, LIB)
     return LIB
 
 
