@@ -406,6 +406,7 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step
     if (TAPE) store(slot + 3 * tn);
     drift_mu(false, TAPE ? cb + 2 * tn : nullptr);
     if (TAPE) store(slot + 4 * tn);
+    if (!apart) __syncthreads();  // the chunks' edge terms are read
     rows_out();
     drift_e(false, TAPE ? cb + 3 * tn : nullptr);
     store(dst + po);
