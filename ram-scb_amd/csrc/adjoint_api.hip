@@ -63,7 +63,8 @@ void launch_plane_bwd(int seq, int threads, dim3 grid, size_t lds, hipStream_t s
 // host Fortran-layout F2 <-> device-layout buffer (through the context's stage)
 int upload_f2(ramgpu_ctx *c, double *dst, const double *host) {
   const size_t n = (size_t)c->ns * c->nr * c->nt * c->ne * c->npa;
-  HIP_TRY(hipMemcpyAsync(c->d_stage, host, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+  const int rc = copy_to_device(c->device, c->stream, c->d_stage, host, n * sizeof(double));
+  if (rc) return rc;
   hipLaunchKernelGGL(k_f2_in, dim3(1024), dim3(256), 0, c->stream, dst, (const double *)c->d_stage, c->ns, c->nr,
                      c->nt, c->ne, c->npa);
   return launch_check("k_f2_in");
@@ -75,9 +76,7 @@ int download_f2(ramgpu_ctx *c, double *host, const double *src) {
                      c->npa);
   int rc = launch_check("k_f2_out");
   if (rc) return rc;
-  HIP_TRY(hipMemcpyAsync(host, c->d_stage, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  return RAMGPU_OK;
+  return copy_to_host(c->device, c->stream, host, c->d_stage, n * sizeof(double));
 }
 
 }  // namespace ramgpu_host
@@ -87,33 +86,39 @@ namespace {
 size_t nf2(const ramgpu_ctx *c) { return (size_t)c->ns * c->nr * c->nt * c->ne * c->npa; }
 size_t nfg(const ramgpu_ctx *c) { return (size_t)c->ns * c->nt * c->ne * c->npa; }
 
+// Device blocks of one call (dev_take), given back when it returns and the
+// context's stream is idle.
 struct DevBuf {
-  std::vector<void *> p;
+  struct Item {
+    void *p;
+    size_t bytes;
+  };
+  ramgpu_ctx *c;
+  std::vector<Item> items;
+  explicit DevBuf(ramgpu_ctx *cc) : c(cc) {}
   ~DevBuf() {
-    for (void *q : p) (void)hipFree(q);
+    (void)hipStreamSynchronize(c->stream);
+    for (const Item &q : items) dev_give(c->device, q.p, q.bytes);
+  }
+  template <class T>
+  bool take(T **out, size_t n) {
+    void *q = nullptr;
+    const size_t bytes = std::max<size_t>(n, 1) * sizeof(T);
+    if (!dev_take(c->device, &q, bytes)) return false;
+    items.push_back({q, bytes});
+    *out = (T *)q;
+    return true;
   }
   template <class T>
   int alloc(T **out, size_t n) {
-    void *q = nullptr;
-    if (hipMalloc(&q, std::max<size_t>(n, 1) * sizeof(T)) != hipSuccess)
-      return fail(RAMGPU_ENOMEM, "hipMalloc of %zu bytes failed", n * sizeof(T));
-    p.push_back(q);
-    *out = (T *)q;
-    return RAMGPU_OK;
+    return take(out, n) ? RAMGPU_OK : fail(RAMGPU_ENOMEM, "hipMalloc of %zu bytes failed", n * sizeof(T));
   }
 };
 
 // an allocation the caller can do without (no error is recorded when it fails)
 template <class T>
 bool try_alloc(DevBuf &b, T **out, size_t n) {
-  void *q = nullptr;
-  if (hipMalloc(&q, std::max<size_t>(n, 1) * sizeof(T)) != hipSuccess) {
-    (void)hipGetLastError();
-    return false;
-  }
-  b.p.push_back(q);
-  *out = (T *)q;
-  return true;
+  return b.take(out, n);
 }
 
 // The second stream of ramgpu_adjoint_run and the events that order the two
@@ -240,7 +245,7 @@ int op_bwd(ramgpu_ctx *c, int s, int which, double *adj, double *fgeos_adj) {
   int rc = check_ctx(c);
   if (rc || (rc = check_species(c, s)) || (rc = prepare(c))) return rc;
   if (!adj) return fail(RAMGPU_EINVAL, "adj is null");
-  DevBuf b;
+  DevBuf b(c);
   double *da = nullptr, *db = nullptr;
   if ((rc = b.alloc(&da, nf2(c)))) return rc;
   if ((rc = upload_f2(c, da, adj))) return rc;
@@ -293,7 +298,7 @@ int ramgpu_ram_run_bwd(ramgpu_ctx *c, double *adj, double *fgeos_adj) {
   if (rc || (rc = ready(c)) || (rc = forward_only(c)) || (rc = prepare(c))) return rc;
   if (!adj) return fail(RAMGPU_EINVAL, "adj is null");
   const size_t n = nf2(c);
-  DevBuf b;
+  DevBuf b(c);
   double *tape = nullptr, *da = nullptr, *db = nullptr, *save_f2 = nullptr, *save_e = nullptr;
   if ((rc = b.alloc(&tape, T_N * n)) || (rc = b.alloc(&da, n)) || (rc = b.alloc(&save_f2, n)) ||
       (rc = b.alloc(&save_e, (size_t)c->ns * 7)))
@@ -334,7 +339,7 @@ int ramgpu_adjoint_run(ramgpu_ctx *c, int nsteps, int ckpt_every, const double *
   const int nseg = (nsteps + ckpt_every - 1) / ckpt_every;
   const int seglen = std::min(ckpt_every, nsteps);
   const size_t tape_n = (size_t)seglen * T_N * n;
-  DevBuf b;
+  DevBuf b(c);
   double *ckpt, *tape, *lam, *bbar = nullptr, *dw, *dtarget, *lossv, *scratch_loss, *final_f2, *final_e;
   double *d_kp = nullptr, *d_bs = nullptr;
   int *dpts;
@@ -479,8 +484,7 @@ int ramgpu_adjoint_run(ramgpu_ctx *c, int nsteps, int ckpt_every, const double *
   }
   if (grad_f2 && (rc = download_f2(c, grad_f2, lam))) return rc;
   if (grad_fgeos) {
-    HIP_TRY(hipMemcpyAsync(grad_fgeos, bbar, (size_t)nsteps * ng * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    if ((rc = copy_to_host(c->device, c->stream, grad_fgeos, bbar, (size_t)nsteps * ng * sizeof(double)))) return rc;
   }
   return RAMGPU_OK;
 }

@@ -95,7 +95,7 @@ namespace ramgpu_host {
 template <class T>
 int dev_alloc(ramgpu_ctx *c, T **p, size_t n) {
   void *q = nullptr;
-  if (hipMalloc(&q, std::max<size_t>(n, 1) * sizeof(T)) != hipSuccess)
+  if (!dev_malloc(c->device, &q, std::max<size_t>(n, 1) * sizeof(T)))
     return fail(RAMGPU_ENOMEM, "hipMalloc of %zu bytes failed", n * sizeof(T));
   (void)hipMemset(q, 0, std::max<size_t>(n, 1) * sizeof(T));
   c->allocs.push_back(q);
@@ -618,6 +618,8 @@ int ramgpu_create(ramgpu_ctx **out, int ns, int nr, int nt, int ne, int npa, int
   HIP_TRY(hipSetDevice(device));
   ramgpu_ctx *c = new ramgpu_ctx();
   c->device = device;
+  context_opened();
+  c->counted = true;
   c->ns = ns;
   c->nr = nr;
   c->nt = nt;
@@ -737,6 +739,7 @@ int ramgpu_destroy(ramgpu_ctx *c) {
   if (c->ev1) (void)hipEventDestroy(c->ev1);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   if (c->stream2) (void)hipStreamDestroy(c->stream2);
+  if (c->counted) context_closed();
   delete c;
   return RAMGPU_OK;
 }
@@ -919,11 +922,8 @@ int ramgpu_set_boundary_scale(ramgpu_ctx *c, const double *scale) {
 int ramgpu_put_f2(ramgpu_ctx *c, const double *f2) {
   int rc = check_ctx(c);
   if (rc) return rc;
-  const size_t n = (size_t)c->ns * c->nr * c->nt * c->ne * c->npa;
-  if ((rc = set_f64(c, c->d_stage, f2, n, "f2"))) return rc;
-  hipLaunchKernelGGL(k_f2_in, dim3(1024), dim3(256), 0, c->stream, c->t.f2, (const double *)c->d_stage,
-                     c->ns, c->nr, c->nt, c->ne, c->npa);
-  if ((rc = launch_check("k_f2_in"))) return rc;
+  if (!f2) return fail(RAMGPU_EINVAL, "f2 is null");
+  if ((rc = upload_f2(c, c->t.f2, f2))) return rc;
   HIP_TRY(hipStreamSynchronize(c->stream));
   c->have_f2 = true;
   return RAMGPU_OK;
@@ -933,13 +933,7 @@ int ramgpu_get_f2(ramgpu_ctx *c, double *f2) {
   int rc = check_ctx(c);
   if (rc) return rc;
   if (!f2) return fail(RAMGPU_EINVAL, "f2 is null");
-  const size_t n = (size_t)c->ns * c->nr * c->nt * c->ne * c->npa;
-  hipLaunchKernelGGL(k_f2_out, dim3(1024), dim3(256), 0, c->stream, c->d_stage, (const double *)c->t.f2,
-                     c->ns, c->nr, c->nt, c->ne, c->npa);
-  if ((rc = launch_check("k_f2_out"))) return rc;
-  HIP_TRY(hipMemcpyAsync(f2, c->d_stage, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  return RAMGPU_OK;
+  return download_f2(c, f2, c->t.f2);
 }
 
 int ramgpu_set_energy_state(ramgpu_ctx *c, const double *setrc, const double *lsdr,
@@ -1169,9 +1163,10 @@ int ramgpu_ram_run_schedule(ramgpu_ctx *c, int nsteps, const double *kp, const d
   if (rc) return rc;
   // the whole schedule is staged on the device before the timed steps
   double *d_kp = nullptr, *d_bs = nullptr;
-  HIP_TRY(hipMalloc(&d_kp, std::max(nsteps, 1) * sizeof(double)));
-  if (bscale && hipMalloc(&d_bs, std::max(nsteps, 1) * c->ns * sizeof(double)) != hipSuccess) {
-    (void)hipFree(d_kp);
+  const size_t nkp = std::max(nsteps, 1) * sizeof(double), nbs = nkp * c->ns;
+  if (!dev_take(c->device, (void **)&d_kp, nkp)) return fail(RAMGPU_ENOMEM, "hipMalloc of the Kp schedule failed");
+  if (bscale && !dev_take(c->device, (void **)&d_bs, nbs)) {
+    dev_give(c->device, d_kp, nkp);
     return fail(RAMGPU_ENOMEM, "hipMalloc of the boundary-scale schedule failed");
   }
   if (hipMemcpyAsync(d_kp, kp, nsteps * sizeof(double), hipMemcpyHostToDevice, c->stream) != hipSuccess ||
@@ -1180,8 +1175,9 @@ int ramgpu_ram_run_schedule(ramgpu_ctx *c, int nsteps, const double *kp, const d
       hipStreamSynchronize(c->stream) != hipSuccess)
     rc = fail(RAMGPU_EHIP, "staging the Kp schedule failed");
   if (rc == RAMGPU_OK) rc = run_schedule_staged(c, nsteps, d_kp, d_bs);
-  (void)hipFree(d_kp);
-  if (d_bs) (void)hipFree(d_bs);
+  (void)hipStreamSynchronize(c->stream);
+  dev_give(c->device, d_kp, nkp);
+  if (d_bs) dev_give(c->device, d_bs, nbs);
   if (rc) return rc;
   return fill_out(c, out);
 }

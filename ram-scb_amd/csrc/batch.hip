@@ -82,7 +82,7 @@ struct ramgpu_batch {
 namespace {
 
 int batch_alloc(ramgpu_batch *b, void **p, size_t bytes) {
-  if (hipMalloc(p, std::max<size_t>(bytes, 16)) != hipSuccess)
+  if (!dev_malloc(b->device, p, std::max<size_t>(bytes, 16)))
     return fail(RAMGPU_ENOMEM, "hipMalloc of %zu bytes failed", bytes);
   b->allocs.push_back(*p);
   return RAMGPU_OK;
@@ -634,6 +634,7 @@ int ramgpu_batch_adjoint_run(ramgpu_batch *b, int nsteps, int ckpt_every, const 
   }
   size_t freeb = 0, totb = 0;
   HIP_TRY(hipMemGetInfo(&freeb, &totb));
+  freeb += dev_cached(b->device);  // blocks kept from earlier calls serve this one or are given back
   const size_t fixed = 8 * (2 * nall + (grad_fgeos ? (size_t)nsteps * ngall : 0)) + ((size_t)64 << 20);
   const size_t one = (size_t)(nseg + seglen * T_N) * nall * 8, two = (size_t)(nseg + seglen + T_N) * nall * 8;
   // two-level: states, then one re-taped step at a time (forced with
@@ -648,14 +649,16 @@ int ramgpu_batch_adjoint_run(ramgpu_batch *b, int nsteps, int ckpt_every, const 
   const int CK = 0, ST = nseg, TG = split ? nseg + seglen : nseg;
   auto group = [&](int s, int n0) { return split ? TG : TG + (s - n0) * T_N; };
   // buffers
-  std::vector<void *> bufs;
+  std::vector<std::pair<void *, size_t>> bufs;
   auto release = [&]() {
     (void)hipStreamSynchronize(b->stream);
-    for (void *q : bufs) (void)hipFree(q);
+    for (const auto &q : bufs) dev_give(b->device, q.first, q.second);
+    bufs.clear();
   };
   auto alloc = [&](void **q, size_t bytes) {
-    if (hipMalloc(q, std::max<size_t>(bytes, 16)) != hipSuccess) return false;
-    bufs.push_back(*q);
+    bytes = std::max<size_t>(bytes, 16);
+    if (!dev_take(b->device, q, bytes)) return false;
+    bufs.emplace_back(*q, bytes);
     return true;
   };
   std::vector<double *> fin(M), fin_e(M);
@@ -789,7 +792,10 @@ int ramgpu_batch_adjoint_run(ramgpu_batch *b, int nsteps, int ckpt_every, const 
       }
     }
     if (c->t.bbar) {
-      HIP_TRY(hipMemcpy(grad_fgeos[mi], c->t.bbar, (size_t)nsteps * ng * 8, hipMemcpyDeviceToHost));
+      if ((rc = copy_to_host(b->device, st, grad_fgeos[mi], c->t.bbar, (size_t)nsteps * ng * 8))) {
+        detach();
+        return rc;
+      }
     }
   }
   return detach();
@@ -814,7 +820,7 @@ int ramgpu_batch_autotune(ramgpu_batch *b, int reps, double *ms_best) {
   for (ramgpu_ctx *c : b->m) {
     const size_t nf = f2_species_stride(c->t) * c->ns * sizeof(double), ne = (size_t)c->ns * 4 * sizeof(double);
     void *p = nullptr, *q = nullptr;
-    if (hipMalloc(&p, nf) != hipSuccess || hipMalloc(&q, ne) != hipSuccess) {
+    if (!dev_malloc(b->device, &p, nf) || !dev_malloc(b->device, &q, ne)) {
       if (p) (void)hipFree(p);
       release();
       return fail(RAMGPU_ENOMEM, "autotune: no room to save the state");

@@ -489,17 +489,19 @@ int ramgpu_computehI(ramgpu_ctx *c, int nthe, int ieq, const double *x, const do
   const size_t nl = (size_t)nthe * nr * nt, n3 = (size_t)nr * nt * npa, n2 = (size_t)nr * nt;
   const size_t nd = 4 * nl + nthe + 2 * (size_t)npa + (nr + 1) + kSmoothW * kSmoothW + 10 * n3 + n2;
   const size_t ni = n2 + nt;
+  const size_t wsb = nd * sizeof(double) + ni * sizeof(int);
   char *ws = nullptr;
-  if (hipMalloc(&ws, nd * sizeof(double) + ni * sizeof(int)) != hipSuccess)
+  if (!ramgpu_host::dev_take(c->device, (void **)&ws, wsb))
     return fail(RAMGPU_ENOMEM, "computehI: workspace allocation failed");
   struct Free {
     char *p;
+    size_t bytes;
     ramgpu_ctx *c;
     ~Free() {
       (void)hipStreamSynchronize(c->stream);
-      (void)hipFree(p);
+      ramgpu_host::dev_give(c->device, p, bytes);
     }
-  } guard{ws, c};
+  } guard{ws, wsb, c};
   double *d = (double *)ws;
   HiArgs a{};
   a.nthe = nthe; a.nr = nr; a.nt = nt; a.npa = npa; a.ieq = ieq - 1;

@@ -132,7 +132,7 @@ int coul_alloc(ramgpu_ctx *c) {
   const size_t bytes[4] = {n * sizeof(double), n * sizeof(double2), (size_t)c->ns * 5 * sizeof(double),
                            (size_t)c->nr * c->nt * sizeof(double)};
   for (int q = 0; q < 4; ++q) {
-    if (hipMalloc(&p[q], bytes[q]) != hipSuccess || hipMemset(p[q], 0, bytes[q]) != hipSuccess) {
+    if (!ramgpu_host::dev_malloc(c->device, &p[q], bytes[q]) || hipMemset(p[q], 0, bytes[q]) != hipSuccess) {
       for (int r = 0; r <= q; ++r)
         if (p[r]) (void)hipFree(p[r]);
       return ramgpu_host::fail(RAMGPU_ENOMEM, "allocation of the Coulomb tables failed");

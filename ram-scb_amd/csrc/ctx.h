@@ -59,6 +59,7 @@ struct StepShape {
 
 struct ramgpu_ctx {
   int device = 0;
+  bool counted = false;  // context_opened called
   int ns = 0, nr = 0, nt = 0, ne = 0, npa = 0;
   hipStream_t stream = nullptr;
   // a second stream (default priority) on which ramgpu_adjoint_run
@@ -188,6 +189,22 @@ int forward_only(const ramgpu_ctx *c);
 // then runs: one launch per operator for all species, finalized at its end
 int takes_pitch(const ramgpu_ctx *c);
 int step_composed(ramgpu_ctx *c, int rec);
+// Bulk copies between pageable host memory and the device, in stream order,
+// complete on return (hostio.hip); threads share one bounded ring of pinned
+// memory per process
+int copy_to_host(int device, hipStream_t stream, void *host, const void *dev, size_t bytes);
+int copy_to_device(int device, hipStream_t stream, void *dev, const void *host, size_t bytes);
+// hipMalloc, giving the kept blocks back first when it fails
+bool dev_malloc(int device, void **p, size_t bytes);
+// A device block of exactly `bytes` for the length of a call: one kept from an
+// earlier call or a new one; given back (its device work done) it is kept for
+// a later call, 4 GiB per process at most, until the last context goes or an
+// allocation needs the room
+bool dev_take(int device, void **p, size_t bytes);
+void dev_give(int device, void *p, size_t bytes);
+size_t dev_cached(int device);
+void context_opened();
+void context_closed();
 // host Fortran-layout F2 <-> device-layout buffer, through the context's stage
 int upload_f2(ramgpu_ctx *c, double *dst, const double *host);
 int download_f2(ramgpu_ctx *c, double *host, const double *src);

@@ -203,7 +203,7 @@ namespace {
 
 int alloc_zero(ramgpu_ctx *c, double **p, size_t n) {
   void *q = nullptr;
-  if (hipMalloc(&q, std::max<size_t>(n, 1) * sizeof(double)) != hipSuccess)
+  if (!dev_malloc(c->device, &q, std::max<size_t>(n, 1) * sizeof(double)))
     return fail(RAMGPU_ENOMEM, "hipMalloc of %zu bytes failed", n * sizeof(double));
   c->allocs.push_back(q);
   *p = (double *)q;

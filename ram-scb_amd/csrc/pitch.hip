@@ -23,7 +23,7 @@ int upload_coef(ramgpu_ctx *c, double **slot, const double *d1, const double *d2
     return fail(RAMGPU_EINVAL, "NPA=%d: the pitch-angle line solve's LDS exceeds the device's", c->npa);
   if (!*slot) {
     void *p = nullptr;
-    if (hipMalloc(&p, n * sizeof(double)) != hipSuccess)
+    if (!dev_malloc(c->device, &p, n * sizeof(double)))
       return fail(RAMGPU_ENOMEM, "allocation of a pitch-angle diffusion table failed");
     c->allocs.push_back(p);
     *slot = (double *)p;

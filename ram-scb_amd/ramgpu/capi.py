@@ -177,6 +177,11 @@ def copy_probe(nbytes: int = 1 << 30, reps: int = 20, device: int = 0) -> float:
     return out.value
 
 
+def _per_step(flat, nsteps, m):
+    """(nsteps, NS, NT, NE, NPA) view of nsteps Fortran-ordered (NS,NT,NE,NPA) arrays."""
+    return flat.reshape((nsteps, m.npa, m.ne, m.nt, m.ns)).transpose(0, 4, 3, 2, 1)
+
+
 class RamGpu:
     """One device-resident RAM problem (a ``ramgpu_ctx``)."""
 
@@ -543,15 +548,11 @@ class RamGpu:
             raise ValueError("bscale must have nsteps*NS entries")
         loss = C.c_double(0.0)
         gf = np.zeros(self.dims, order="F")
-        gb = np.zeros((nsteps, self.ns, self.nt, self.ne, self.npa))
         gbf = np.zeros(nsteps * self.ns * self.nt * self.ne * self.npa)
         self._check(self.lib.ramgpu_adjoint_run(
             self.h, nsteps, ckpt_every, None if kpa is None else _p(kpa), None if bsa is None else _p(bsa),
             npts, pts.ctypes.data_as(_ip), _p(w), _p(target), C.byref(loss), _p(gf), _p(gbf)))
-        per = self.ns * self.nt * self.ne * self.npa
-        for n in range(nsteps):
-            gb[n] = gbf[n * per:(n + 1) * per].reshape((self.ns, self.nt, self.ne, self.npa), order="F")
-        return loss.value, gf, gb
+        return loss.value, gf, _per_step(gbf, nsteps, self)
 
     def set_plane_shape(self, threads=0, maxc=0):
         """Block size and row bound of the plane kernels (0, 0: the library's choice)."""
@@ -705,12 +706,5 @@ class RamBatch:
         self._check(self.lib.ramgpu_batch_adjoint_run(
             self.h, nsteps, ckpt_every, _p(kp), None if bs is None else _p(bs), npts, pp, wp, tp, _p(loss),
             gfp, gbp if grad_fgeos else None))
-        out_gb = []
-        for m, gb in zip(self.members, gbs):
-            if gb is None:
-                out_gb.append(None)
-                continue
-            per = m.ns * m.nt * m.ne * m.npa
-            out_gb.append(np.stack([gb[n * per:(n + 1) * per].reshape((m.ns, m.nt, m.ne, m.npa), order="F")
-                                    for n in range(nsteps)]))
+        out_gb = [None if gb is None else _per_step(gb, nsteps, m) for m, gb in zip(self.members, gbs)]
         return loss, gfs, out_gb
