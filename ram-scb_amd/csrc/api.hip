@@ -164,8 +164,12 @@ void tend(ramgpu_ctx *c) {
 // launch that reads it.
 int sync_tab(ramgpu_ctx *c) {
   if (!c->tab_dirty) return RAMGPU_OK;
+  Tab &t = c->t;
+  t.sum_any = 0;
+  for (int s = 0; s < c->ns; ++s)
+    t.sum_any |= ((t.pd_wpi[s] || t.wpi[s]) ? ANY_WPI : 0) | (t.pd_emic[s] ? ANY_EMIC : 0) | (t.cex[s] ? ANY_CEX : 0);
   HIP_TRY(hipStreamSynchronize(c->stream));
-  HIP_TRY(hipMemcpy(c->d_tab, &c->t, sizeof(Tab), hipMemcpyHostToDevice));
+  HIP_TRY(hipMemcpy(c->d_tab, &t, sizeof(Tab), hipMemcpyHostToDevice));
   c->tab_dirty = false;
   return RAMGPU_OK;
 }
@@ -381,8 +385,7 @@ void launch_plane_t(int seq, int threads, dim3 grid, size_t lds, hipStream_t st,
     case SEQ_SUM: hipLaunchKernelGGL((k_plane<SEQ_SUM, MAXC>), grid, blk, lds, st, L, rec); break;
     case SEQ_WAVE: hipLaunchKernelGGL((k_plane<SEQ_WAVE, MAXC>), grid, blk, lds, st, L, rec); break;
     case SEQ_COULEN: hipLaunchKernelGGL((k_plane<SEQ_COULEN, MAXC>), grid, blk, lds, st, L, rec); break;
-    case SEQ_COULMU: hipLaunchKernelGGL((k_plane<SEQ_COULMU, MAXC>), grid, blk, lds, st, L, rec); break;
-    default: hipLaunchKernelGGL((k_plane<SEQ_STEPC, MAXC>), grid, blk, lds, st, L, rec); break;
+    default: hipLaunchKernelGGL((k_plane<SEQ_COULMU, MAXC>), grid, blk, lds, st, L, rec); break;
   }
 }
 
@@ -408,13 +411,17 @@ void launch_plane(int seq, PlaneShape sh, dim3 grid, size_t lds, hipStream_t st,
 //   48x90 (40x48): 6: 612, 9: 453, 10: 553, 16: 734
 //   64x90 (20x48): 8: 385, 10: 456, 12: 308, 16: 411
 // One species of 20x25x35x72 has under two planes per CU: 6 rows 37, 12 rows 42.
+// x: SEQ_STEPX, whose line solves and tables take more LDS; the same rule is
+// right for it (plane launch with Coulomb collisions in us, by rows; 35x72, 4
+// species: 6: 252, 8: 269, 11: 213, 12: 230, 15: 288; 48x90, 2 species of
+// 20x24: 6: 231, 8: 257, 9: 163, 10: 177).
 // The last chunk needs two rows: R with NPA mod R = 1 is left out.
-StepShape step_shape(int ne, int npa, long planes, int ncu, size_t lds_cu) {
+StepShape step_shape(int ne, int npa, long planes, int ncu, size_t lds_cu, bool x) {
   StepShape best{0, 0};
   double bcost = 0;
   for (int r = 2; r <= kMaxCellsPerThread; ++r) {
     const int threads = step_threads(ne, npa, r), waves = threads / 64;
-    const size_t lds = step_lds_bytes(ne, npa, r);
+    const size_t lds = step_lds_bytes(ne, npa, r, x);
     if (npa % r == 1 || threads > kPlaneMaxThreads || lds > lds_cu) continue;
     const int res = std::min<long>(step_resident(lds, ne, npa, r), (planes + ncu - 1) / ncu);
     if (res < 1) continue;
@@ -434,6 +441,7 @@ void launch_step(int seq, StepShape sh, dim3 grid, size_t lds, hipStream_t st, c
 #define ROWS(r)                                                                                              \
   case r:                                                                                                    \
     if (seq == SEQ_TAPE) hipLaunchKernelGGL((k_plane_step<SEQ_TAPE, r>), grid, blk, lds, st, L, rec);        \
+    else if (seq == SEQ_STEPX) hipLaunchKernelGGL((k_plane_step<SEQ_STEPX, r>), grid, blk, lds, st, L, rec); \
     else hipLaunchKernelGGL((k_plane_step<SEQ_STEP, r>), grid, blk, lds, st, L, rec);                        \
     break;
     STEP_ROWS(ROWS)
@@ -451,7 +459,9 @@ int run_plane(ramgpu_ctx *c, int seq, int rec, int s0, int nsp, const double *sr
   const size_t lds = seq_coul(seq) ? plane_coul_lds_bytes(c->ne, c->npa, c->plane.threads)
                                     : plane_fwd_lds_bytes(c->ne, c->npa, c->plane.threads);
   tbeg(c, RAMGPU_KERNEL_PLANE);
-  if (seq == SEQ_STEP || seq == SEQ_TAPE)
+  if (seq == SEQ_STEPX)
+    launch_step(seq, c->stepx, dim3(L.nv), step_lds_bytes(c->ne, c->npa, c->stepx.rows, true), c->stream, L, rec);
+  else if (seq == SEQ_STEP || seq == SEQ_TAPE)
     launch_step(seq, c->step, dim3(L.nv), step_lds_bytes(c->ne, c->npa, c->step.rows), c->stream, L, rec);
   else
     launch_plane(seq, c->plane, dim3(L.nv), lds, c->stream, L, rec);
@@ -516,10 +526,12 @@ int set_plane_lds_limit(size_t limit) {
   const void *fns[] = {
       PLANE_K(SEQ_E), PLANE_K(SEQ_MU), PLANE_K(SEQ_CEX), PLANE_K(SEQ_ATM), PLANE_K(SEQ_SUM),
       PLANE_K(SEQ_WAVE),
-      PLANE_K(SEQ_COULEN), PLANE_K(SEQ_COULMU), PLANE_K(SEQ_STEPC),
+      PLANE_K(SEQ_COULEN), PLANE_K(SEQ_COULMU),
       (const void *)k_r<0>, (const void *)k_r<1>, (const void *)k_r<2>,
       (const void *)k_r_bwd<0>, (const void *)k_r_bwd<1>, (const void *)k_p<0>, (const void *)k_p<1>,
-#define STEP_K(r) (const void *)k_plane_step<SEQ_STEP, r>, (const void *)k_plane_step<SEQ_TAPE, r>,
+#define STEP_K(r)                                                                           \
+  (const void *)k_plane_step<SEQ_STEP, r>, (const void *)k_plane_step<SEQ_TAPE, r>, \
+      (const void *)k_plane_step<SEQ_STEPX, r>,
       STEP_ROWS(STEP_K)
 #undef STEP_K
       (const void *)k_p_bwd, (const void *)k_pitch_diffusion};
@@ -568,28 +580,21 @@ int ramgpu_host::fill_out(ramgpu_ctx *c, ramgpu_species_out *out) {
 int ramgpu_host::step_once(ramgpu_ctx *c) {
   int cflmask, rc;
   if ((rc = step_body(c, &cflmask))) return rc;
-  if (cflmask >= 0 && (rc = run_finalize(c, cflmask, 2, 0, c->ns))) return rc;
-  return RAMGPU_OK;
+  return run_finalize(c, cflmask, 2, 0, c->ns);
 }
 
 // The sweeps of one step; its finalize (cflmask, SUMRC mode 2) is the
-// caller's, except for the composed step (WPADIF or FLC on), which
-// finalizes species by species and returns cflmask -1.
+// caller's.
 int ramgpu_host::step_body(ramgpu_ctx *c, int *cflmask) {
   int rc;
   if ((rc = prepare(c))) return rc;
   const int rec = c->cfl_valid ? 0 : 1;
   const int ns = c->ns;
-  if (takes_pitch(c)) {
-    if ((rc = step_composed(c, rec))) return rc;
-    *cflmask = -1;
-    c->cfl_valid = true;
-    return RAMGPU_OK;
-  }
-  // with Coulomb collisions the plane kernel also runs COULEN and COULMU,
-  // flag bit 1 being COULMU's clamp (TimeRamElapsed > 0)
-  const int seq = c->t.coul ? SEQ_STEPC : SEQ_STEP;
-  const int flags = rec | ((c->t.coul && c->time_elapsed > 0.) ? 2 : 0);
+  // with Coulomb collisions, WPADIF or FLCscatter the plane kernel runs them
+  // too; flag bit 1 is COULMU's clamp (TimeRamElapsed > 0), bit 2
+  // FLCscatter's start (TimeRamElapsed >= Dt_bc, src/ModRamLoss.f90:526)
+  const int seq = (c->t.coul || takes_pitch(c)) ? SEQ_STEPX : SEQ_STEP;
+  const int flags = rec | (c->time_elapsed > 0. ? 2 : 0) | (c->time_elapsed >= c->dt_bc ? 4 : 0);
   if ((rc = run_r(c, rec, 0, ns)) || (rc = run_p(c, rec, 0, ns)) ||
       (rc = run_plane(c, seq, flags, 0, ns)) || (rc = run_p(c, 0, 0, ns)) || (rc = run_r(c, 2, 0, ns)))
     return rc;
@@ -658,15 +663,14 @@ int ramgpu_create(ramgpu_ctx **out, int ns, int nr, int nt, int ne, int npa, int
   c->plane = plane_shape(ne, npa, c->lds_limit);
   if (c->plane.threads == 0) return cleanup(fail(RAMGPU_EINVAL, "no plane kernel shape for %dx%d", ne, npa));
   t.plane_chunks = plane_chunks_for(ne, npa, c->plane.threads);
-  c->step = step_shape(ne, npa, (long)ns * (nr - 1) * nt, ncu, c->lds_limit);
-  if (c->step.threads == 0) return cleanup(fail(RAMGPU_EINVAL, "no plane kernel shape for %dx%d", ne, npa));
+  c->step = step_shape(ne, npa, (long)ns * (nr - 1) * nt, ncu, c->lds_limit, false);
+  c->stepx = step_shape(ne, npa, (long)ns * (nr - 1) * nt, ncu, c->lds_limit, true);
+  if (c->step.threads == 0 || c->stepx.threads == 0) return cleanup(fail(RAMGPU_EINVAL, "no plane kernel shape for %dx%d", ne, npa));
   t.step_cells = step_wave_cells(ne);
   t.step_apart = step_edges_apart(ne, npa, c->step.rows);
+  t.stepx_apart = step_edges_apart(ne, npa, c->stepx.rows, true);
   c->d_pdc.assign(ns, nullptr);
-  c->d_flc.assign(ns, nullptr);
   c->d_flc_mem.assign(ns, nullptr);
-  c->pd_wpi.assign(ns, 0);
-  c->pd_emic.assign(ns, 0);
 #define A(p, n) \
   if ((rc = dev_alloc(c, &p, n))) return cleanup(rc)
   A(c->d_rlz, nr1); A(c->d_ekev, ne); A(c->d_ebnd, ne); A(c->d_we, ne); A(c->d_de, ne);
@@ -1140,10 +1144,8 @@ int run_schedule_staged(ramgpu_ctx *c, int nsteps, const double *d_kp, const dou
     if ((rc = apply_step_inputs(c, d_kp + n, d_bs ? d_bs + (size_t)n * c->ns : nullptr))) break;
     int cflmask = 0;
     if ((rc = step_body(c, &cflmask))) break;
-    if (cflmask >= 0) {
-      c->fin_mask = cflmask;
-      c->fin_mode = 2;
-    }
+    c->fin_mask = cflmask;
+    c->fin_mode = 2;
     c->time_elapsed += 2.0 * c->t.dts;  // src/ModRamScbRun.f90:88, after each ram_run
   }
   const int rf = flush_finalize(c);

@@ -6,7 +6,7 @@
 // reference recomputes them every step, src/ModRamRun.f90:69) with the C
 // library's erf, exp, log, pow and sqrt, in the reference's expression
 // order, and uploaded: COULEN and COULMU then run on the device in the plane
-// kernels (k_plane<SEQ_COULEN|SEQ_COULMU|SEQ_STEPC>).
+// kernels (k_plane<SEQ_COULEN|SEQ_COULMU>, k_plane_step<SEQ_STEPX>).
 #include <hip/hip_runtime.h>
 
 #include <cmath>

@@ -70,7 +70,7 @@ struct ramgpu_ctx {
   double last_ms = 0.0;
   size_t lds_limit = 65536;
   PlaneShape plane{ramgpu::kPlaneThreads, 16, 0};
-  StepShape step{0, 0};
+  StepShape step{0, 0}, stepx{0, 0};  // of SEQ_STEP and SEQ_TAPE; of SEQ_STEPX
   Tab t{};            // host image of the problem descriptor
   Tab *d_tab = nullptr;  // its device copy, read by every kernel
   bool tab_dirty = true;
@@ -119,11 +119,8 @@ struct ramgpu_ctx {
   double *d_necr = nullptr;
   double time_elapsed = 0.0;
   double told = 0.0;  // TimeRamElapsed at the last ramgpu_computehI (TOld)
-  // WPADIF and FLCscatter: per species the WPADIF table (device layout) and
-  // whether ram_run takes it at the WPI positions (in place of WAVELO) and at
-  // the EMIC positions; the FLC table (null: no FLC) and its allocation; Dt_bc
-  std::vector<double *> d_pdc, d_flc, d_flc_mem;
-  std::vector<char> pd_wpi, pd_emic;
+  // allocations of the WPADIF and FLC tables (Tab::pdc, Tab::flc); Dt_bc
+  std::vector<double *> d_pdc, d_flc_mem;
   double dt_bc = 0.0;
 };
 
@@ -163,7 +160,7 @@ PlaneShape plane_shape(int ne, int npa, size_t lds_cu);
 int coef_units(const ramgpu_ctx *c, int threads);
 bool takes_wave(const ramgpu_ctx *c);
 PlaneShape plane_shape_for(int ne, int npa, int threads);
-StepShape step_shape(int ne, int npa, long planes, int ncu, size_t lds_cu);
+StepShape step_shape(int ne, int npa, long planes, int ncu, size_t lds_cu, bool x);
 // launch k_plane_step<seq, rows>
 void launch_step(int seq, StepShape sh, dim3 grid, size_t lds, hipStream_t st, const ramgpu::Launch &L, int rec);
 // launch k_plane<seq, maxc>
@@ -185,10 +182,8 @@ int coul_check_lds(const ramgpu_ctx *c, int threads);
 // RAMGPU_ESTATE for a context with Coulomb collisions, WPADIF or FLC
 // scattering on: the reverse mode and ensembles step without them
 int forward_only(const ramgpu_ctx *c);
-// whether a species takes WPADIF or FLCscatter in ram_run, and the step that
-// then runs: one launch per operator for all species, finalized at its end
+// whether a species takes WPADIF or FLCscatter in ram_run
 int takes_pitch(const ramgpu_ctx *c);
-int step_composed(ramgpu_ctx *c, int rec);
 // Bulk copies between pageable host memory and the device, in stream order,
 // complete on return (hostio.hip); threads share one bounded ring of pinned
 // memory per process

@@ -1066,70 +1066,6 @@ __device__ void plane_mu(const Tab &t, const FwdCtx &c, const PlaneFwd &d, bool 
   __syncthreads();
 }
 
-// The loss chain of ram_run between the two drift halves (src/ModRamRun.f90:
-// 77-159): SUMRC, [WAVELO, SUMRC], [CEX, SUMRC], ATMOL, SUMRC, ATMOL, SUMRC,
-// [CEX, SUMRC], [WAVELO, SUMRC], with the SUMRC partials of this plane block b
-// in slots 0..6.  An operator a species does not take multiplies by 1, which
-// leaves its cells and so its slot's sum bit for bit those of the slot before.
-// WAVELO's factor is one per thread (it depends on I, J, K only), so a
-// thread's partial sums after it are its sums before it times the factor
-// (to rounding: exactly when the factor is 1).  Each thread rewrites only
-// its own cells.
-template <int MAXC>
-__device__ void plane_loss(const Tab &t, const FwdCtx &c, const PlaneFwd &d, int b) {
-  const int NE = c.NE, NPA = c.NPA, NT = c.NT;
-  const bool cex = c.cex != 0;
-  const int upa = c.upa;
-  const bool sum_row = c.j <= NT - 2;
-  const int k = c.ke;
-  const double sigv = d.kt[KT_SIGV * NE + k], latl = d.kt[KT_LATL * NE + k];
-  const double wk = d.kt[KT_WE * NE + k], ek = d.kt[KT_EKEV * NE + k];
-  const double wave = d.kt[KT_WAVE * NE + k];  // 1 for K=1 and without WAVELO
-  const double dts = d.pc[PC_DTS];
-  const double ekw = ek * wk;
-  double a[5] = {0, 0, 0, 0, 0}, tot[7];
-  const int l0 = fresh(c.l0);
-#pragma unroll
-  for (int n = 0; n < MAXC; ++n) {
-    if (n >= c.nr) break;
-    const int l = l0 + n;
-    const bool w_on = sum_row && k >= 1 && l >= 1;
-    const bool cx = cex && k >= 1 && l >= 1;
-    const bool atm = k >= 1 && l + 1 >= upa;
-    double *pf = &c.col[l * c.cst];
-    double f = *pf;
-    // CHARGE=EXP(-ALPHA), ALPHA=10**Y*V*HDNS*DTs (src/ModRamLoss.f90:47-49);
-    // ATLOS**(1/FNHS) (:501) as exp(log(ATLOS)*(1/FNHS)); WAVELO's
-    // exp(-DTs/TAU) on L>=2 (src/ModRamWPI.f90:630); a factor of 1 leaves a
-    // cell outside the operator's range unchanged, and a weight of 0 leaves
-    // it out of the sums
-    const double cxf = cx ? exp_tab(-(sigv * d.cl[2 * l] * dts), d.ex) : 1.0;
-    const double af = atm ? exp_tab(latl * d.cl[2 * l + 1], d.ex) : 1.0;
-    const double wf = (l == 0) ? 1.0 : wave;
-    const double q = w_on ? ekw * d.lt[LT_WMU * NPA + l] : 0.0;  // EKEV*WE*WMU
-    a[0] = fma(f, q, a[0]);
-    f = f * wf;
-    f = f * cxf;
-    a[1] = fma(f, q, a[1]);
-    f = f * af;
-    a[2] = fma(f, q, a[2]);
-    f = f * af;
-    a[3] = fma(f, q, a[3]);
-    f = f * cxf;
-    a[4] = fma(f, q, a[4]);
-    *pf = f * wf;
-  }
-  // slots: before WAVELO, after it, after CEX, ATMOL, ATMOL, CEX, after WAVELO
-  double s7[7] = {a[0], a[0] * wave, a[1], a[2], a[3], a[4], a[4] * wave};
-  block_sum_n<7>(s7, d.red, tot);
-  if (threadIdx.x < 7) {
-    double v = tot[0];
-    for (int m = 1; m < 7; ++m)
-      if (threadIdx.x == m) v = tot[m];
-    t.partials[((size_t)threadIdx.x * t.ns + c.s) * t.maxblk + b] = v;
-  }
-}
-
 // One of the loss operators alone on this thread's cells: CHAREXCHANGE
 // (src/ModRamLoss.f90:467-475: K>=2, L>=2), ATMOL (:495-503: K>=2,
 // L>=int(UPA(I))) or WAVELO (src/ModRamWPI.f90:612-633: K>=2, L>=2; the
@@ -1268,26 +1204,6 @@ __device__ void plane_coulmu(const Tab &t, const FwdCtx &c, const PlaneFwd &d, b
   __syncthreads();
 }
 
-// This block's SUMRC partial of the plane (I>=2, K>=2, L>=2, J<=NT-1,
-// src/ModRamRun.f90:246-255) into slot `slot`, with the weights of the loss
-// chain's sums.
-template <int MAXC>
-__device__ void plane_sum_slot(const Tab &t, const FwdCtx &c, const PlaneFwd &d, int b, int slot) {
-  const int NE = c.NE, NPA = c.NPA, k = c.ke;
-  double a[1] = {0.0}, tot[1];
-  if (c.j <= c.NT - 2 && k >= 1) {
-    const double ekw = d.kt[KT_EKEV * NE + k] * d.kt[KT_WE * NE + k];
-#pragma unroll
-    for (int n = 0; n < MAXC; ++n) {
-      if (n >= c.nr) break;
-      const int l = c.l0 + n;
-      if (l >= 1) a[0] = fma(c.col[l * c.cst], ekw * d.lt[LT_WMU * NPA + l], a[0]);
-    }
-  }
-  block_sum_n<1>(a, d.red, tot);
-  if (threadIdx.x == 0) t.partials[((size_t)slot * t.ns + c.s) * t.maxblk + b] = tot[0];
-}
-
 // MAXC (8 or 16) bounds the rows a thread owns; the sweeps take them in
 // passes of kPassRows, so both bounds fit the register budget of 4 waves
 // per SIMD with blocks of up to 1024 threads.
@@ -1305,8 +1221,8 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, 4) k_plane(Launch L, int rec
       block_copy<8>(dst, src, NE * NPA);
       continue;
     }
-    constexpr bool need_loss = SEQ == SEQ_CEX || SEQ == SEQ_ATM || SEQ == SEQ_WAVE || SEQ == SEQ_STEPC;
-    constexpr bool need_kl = SEQ == SEQ_E || SEQ == SEQ_MU || SEQ == SEQ_STEPC;
+    constexpr bool need_loss = SEQ == SEQ_CEX || SEQ == SEQ_ATM || SEQ == SEQ_WAVE;
+    constexpr bool need_kl = SEQ == SEQ_E || SEQ == SEQ_MU;
     FwdCtx c;
     PlaneFwd d;
     fwd_setup<MAXC>(t, u, sm, launch_src(L, t), need_loss, need_kl, c, d);
@@ -1345,22 +1261,6 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, 4) k_plane(Launch L, int rec
       plane_e<MAXC, true>(t, c, d, false);
     } else if constexpr (SEQ == SEQ_COULMU) {
       plane_coulmu(t, c, d, clamp);
-    } else if constexpr (SEQ == SEQ_STEPC) {
-      // src/ModRamRun.f90:72-89 and 160-172: the Coulomb operators sit
-      // between the drift halves and the loss chain, with a SUMRC after each
-      plane_e<MAXC>(t, c, d, rec_here);
-      plane_mu<MAXC>(t, c, d, rec_here);
-      plane_sum_slot<MAXC>(t, c, d, u.b, kSumCoul);
-      plane_e<MAXC, true>(t, c, d, false);
-      plane_sum_slot<MAXC>(t, c, d, u.b, kSumCoul + 1);
-      plane_coulmu(t, c, d, clamp);
-      plane_loss<MAXC>(t, c, d, u.b);
-      plane_coulmu(t, c, d, clamp);
-      plane_sum_slot<MAXC>(t, c, d, u.b, kSumCoul + 2);
-      plane_e<MAXC, true>(t, c, d, false);
-      plane_sum_slot<MAXC>(t, c, d, u.b, kSumCoul + 3);
-      plane_mu<MAXC>(t, c, d, false);
-      plane_e<MAXC>(t, c, d, false);
     }
 
     if constexpr (SEQ != SEQ_SUM) {
@@ -1378,11 +1278,12 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, 4) k_plane(Launch L, int rec
 // (E,Mu) as the reference's (:115,223,308,404).  The maxima are cleared after
 // use for the next recording.
 // SUMRC bookkeeping (src/ModRamRun.f90:77-175,239-257), summode 1: one SUMRC
-// from slot 0, or with kSumFromRadial from the radial slot (SETRC:=S,
-// ELORC=old-S, and with an accumulator in the bits at kSumAccShift that
-// LS* += ELORC); summode 2: the full ram_run chain from
+// from slot 0 (SETRC:=S, ELORC=old-S); summode 2: the full ram_run chain from
 // the loss chain's slots 0..6 and the radial slot 7, with Coulomb collisions
-// also the slots 8..11 of their operators.  One block per (problem, species).
+// also the slots 8..11 of their operators, with EMIC WPADIF 12 and 13.  A
+// species that takes a line solve books every SUMRC that some species has:
+// FLCscatter has none of its own, so its loss goes to the next one.  One
+// block per (problem, species).
 constexpr int kFinNV = 2 + kSumSlots;  // the DtDriftE and DtDriftMu minima, then the SUMRC slot sums
 __device__ inline void finalize_unit(const Launch &L, int vb, int cflmask, int summode, double *red) {
   constexpr int NV = kFinNV;
@@ -1399,6 +1300,8 @@ __device__ inline void finalize_unit(const Launch &L, int vb, int cflmask, int s
     unsigned long long m01[2] = {0ull, 0ull};
     int cex = 0, wpi = 0;
     const bool coul = t.coul != 0;
+    const bool lines = t.pd_wpi[s] || t.pd_emic[s] || t.flc[s];
+    const bool emic = lines && (t.sum_any & ANY_EMIC);
     if (tid == 0) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) e0[q] = t.energy[s * 4 + q];
@@ -1407,8 +1310,8 @@ __device__ inline void finalize_unit(const Launch &L, int vb, int cflmask, int s
       lscsc = t.lsx[s * 3 + 2];
       m01[0] = m[0];
       m01[1] = m[1];
-      cex = t.cex[s];
-      wpi = t.wpi[s];
+      cex = lines ? t.sum_any & ANY_CEX : t.cex[s];
+      wpi = lines ? t.sum_any & ANY_WPI : t.wpi[s];
     }
     double v[NV];
     v[0] = 10000.0;
@@ -1425,27 +1328,27 @@ __device__ inline void finalize_unit(const Launch &L, int vb, int cflmask, int s
         const double c = __longlong_as_double((long long)m[2 + NE + l]);
         if (c > 0) v[1] = fmin(v[1], a * t.dmu[l] / c);
       }
-    const int mode = summode & kSumModeMask;
+    const int mode = summode;
     if (mode != 0) {
-      // slots 0..6 (and with Coulomb collisions 8..11) from the plane
-      // blocks, slot 7 from the R blocks; a single SUMRC reads slot 0, or
-      // the radial slot
+      // slots 0..6 (and with the optional processes 8..13) from the plane
+      // blocks, slot 7 from the R blocks; a single SUMRC reads slot 0
       const int nbk = blocks_kl(t), nbr = blocks_r(t);
       const double *pp = t.partials + (size_t)s * t.maxblk;
       const size_t slot = (size_t)t.ns * t.maxblk;
-      if (mode == 1 && (summode & kSumFromRadial)) {
-        for (int b = tid; b < nbr; b += T) v[2] += pp[kSumRadial * slot + b];
-      } else {
-        const int nslot = (mode == 1) ? 1 : kSumRadial;
-        for (int b = tid; b < nbk; b += T)
-          for (int sl = 0; sl < nslot; ++sl) v[2 + sl] += pp[sl * slot + b];
-      }
+      const int nslot = (mode == 1) ? 1 : kSumRadial;
+      for (int b = tid; b < nbk; b += T)
+        for (int sl = 0; sl < nslot; ++sl) v[2 + sl] += pp[sl * slot + b];
       if (mode == 2) {
         for (int b = tid; b < nbr; b += T) v[2 + kSumRadial] += pp[kSumRadial * slot + b];
         if (coul)
           for (int b = tid; b < nbk; b += T)
 #pragma unroll
             for (int sl = kSumCoul; sl < kSumCoul + 4; ++sl) v[2 + sl] += pp[sl * slot + b];
+        if (emic)
+          for (int b = tid; b < nbk; b += T) {
+            v[2 + kSumEmic] += pp[kSumEmic * slot + b];
+            v[3 + kSumEmic] += pp[(kSumEmic + 1) * slot + b];
+          }
       }
     }
     // one block reduction (fixed order): minima of v[0..1], sums of the rest
@@ -1488,12 +1391,6 @@ __device__ inline void finalize_unit(const Launch &L, int vb, int cflmask, int s
           const double elorc = old - S[0];
           e[0] = S[0];
           t.partials[((size_t)kSumSlots * t.ns + s) * t.maxblk] = elorc;  // ELORC
-          // LS* += ELORC as ram_run books it after the operator
-          const int acc = (summode >> kSumAccShift) & 15;
-          if (acc >= SUM_LSDR && acc <= SUM_LSATM) e[acc] = e0[acc] + elorc;
-          else if (acc == SUM_LSWAE) t.lsx[s * 3] = lswae + elorc;
-          else if (acc == SUM_LSCOE) t.lsx[s * 3 + 1] = lscoe + elorc;
-          else if (acc == SUM_LSCSC) t.lsx[s * 3 + 2] = lscsc + elorc;
         } else {
           // the accumulators of src/ModRamRun.f90:77-175 from consecutive
           // slot sums, each operator's only where the reference runs it
@@ -1513,6 +1410,10 @@ __device__ inline void finalize_unit(const Launch &L, int vb, int cflmask, int s
             lswae += prev - S[1];
             prev = S[1];
           }
+          if (emic) {
+            lswae += prev - S[kSumEmic];
+            prev = S[kSumEmic];
+          }
           if (cex) {
             lscha += prev - S[2];
             prev = S[2];
@@ -1524,6 +1425,10 @@ __device__ inline void finalize_unit(const Launch &L, int vb, int cflmask, int s
           if (cex) {
             lscha += prev - S[5];
             prev = S[5];
+          }
+          if (emic) {
+            lswae += prev - S[kSumEmic + 1];
+            prev = S[kSumEmic + 1];
           }
           if (wpi) {
             lswae += prev - S[6];
@@ -1809,7 +1714,5 @@ template __global__ void k_plane<SEQ_COULEN, 8>(Launch, int);
 template __global__ void k_plane<SEQ_COULEN, 16>(Launch, int);
 template __global__ void k_plane<SEQ_COULMU, 8>(Launch, int);
 template __global__ void k_plane<SEQ_COULMU, 16>(Launch, int);
-template __global__ void k_plane<SEQ_STEPC, 8>(Launch, int);
-template __global__ void k_plane<SEQ_STEPC, 16>(Launch, int);
 
 }  // namespace ramgpu

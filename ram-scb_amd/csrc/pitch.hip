@@ -1,8 +1,7 @@
-// pitch.hip -- the implicit pitch-angle diffusions of the split step, WPADIF
-// (src/ModRamWPI.f90:643-714) and FLCscatter (src/ModRamLoss.f90:513-575),
-// and the step that takes them: ram_run's species loop as one launch per
-// operator (src/ModRamRun.f90:66-183), for the operators the fused plane
-// kernel does not hold.
+// pitch.hip -- the implicit pitch-angle diffusions, WPADIF
+// (src/ModRamWPI.f90:643-714) and FLCscatter (src/ModRamLoss.f90:513-575):
+// their coefficient tables, and the operators on their own.  In ram_run they
+// run inside the plane kernel (k_plane_step<SEQ_STEPX>).
 #include <hip/hip_runtime.h>
 
 #include <vector>
@@ -59,21 +58,13 @@ int run_pitch(ramgpu_ctx *c, int s, const double *coef) {
   return run_pitch(c, job);
 }
 
-// SUMRC of every species, each ELORC booked to accumulator acc (a species
-// whose F2 the operator before left alone books exactly 0, its sum being
-// the same as at its previous SUMRC)
-int sumrc_into(ramgpu_ctx *c, int acc) {
-  int rc = run_plane(c, SEQ_SUM, 0, 0, c->ns);
-  return rc ? rc : run_finalize(c, 0, 1 | (acc << kSumAccShift), 0, c->ns);
-}
-
 }  // namespace
 
 namespace ramgpu_host {
 
 int takes_pitch(const ramgpu_ctx *c) {
   for (int s = 0; s < c->ns; ++s)
-    if (c->pd_wpi[s] || c->pd_emic[s] || c->d_flc[s]) return 1;
+    if (c->t.pd_wpi[s] || c->t.pd_emic[s] || c->t.flc[s]) return 1;
   return 0;
 }
 
@@ -85,93 +76,6 @@ int forward_only(const ramgpu_ctx *c) {
   return RAMGPU_OK;
 }
 
-// One ram_run step with one launch per operator (src/ModRamRun.f90:66-183):
-// the species' chains are independent, so each operator runs for every
-// species that takes it at once, in the reference's order, and each SUMRC
-// for every species (booking 0 where the operator did not run).  The chain
-// ends with DRIFTR's SUMRC, the seam copy, the magnetopause mask and
-// DtDrift* (the CFL maxima recorded by the first sweeps when rec).
-int step_composed(ramgpu_ctx *c, int rec) {
-  int rc = RAMGPU_OK;
-  const int ns = c->ns;
-  const bool coul = c->t.coul != 0;
-  const int clamp = (coul && c->time_elapsed > 0.) ? 2 : 0;
-  PitchJob wpd{}, emic{}, flc{};
-  bool wave[kMaxSpecies] = {}, any_wave = false, any_cex = false;
-  for (int s = 0; s < ns; ++s) {
-    if (c->pd_wpi[s]) {
-      wpd.s[wpd.n] = s;
-      wpd.coef[wpd.n++] = c->d_pdc[s];
-    } else if (c->t.wpi[s]) {
-      wave[s] = any_wave = true;
-    }
-    if (c->pd_emic[s]) {
-      emic.s[emic.n] = s;
-      emic.coef[emic.n++] = c->d_pdc[s];
-    }
-    if (c->d_flc[s] && c->time_elapsed >= c->dt_bc) {
-      flc.s[flc.n] = s;
-      flc.coef[flc.n++] = c->d_flc[s];
-    }
-    any_cex = any_cex || c->t.cex[s] != 0;
-  }
-#define TRY(x) \
-  if ((rc = (x))) return rc
-  // [WAVELO or WPADIF], [EMIC], [CEX], [FLC]: the loss half, forward and
-  // then reversed around the two ATMOLs; CHAREXCHANGE leaves species
-  // without CEX alone, so it runs for all
-  auto half = [&](bool forward) -> int {
-    for (int q = 0; q < 4; ++q) {
-      const int op = forward ? q : 3 - q;
-      if (op == 0 && (any_wave || wpd.n)) {
-        for (int s = 0; s < ns; ++s)
-          if (wave[s]) TRY(run_plane(c, SEQ_WAVE, 0, s, 1));
-        TRY(run_pitch(c, wpd));
-        TRY(sumrc_into(c, SUM_LSWAE));
-      } else if (op == 1 && emic.n) {
-        TRY(run_pitch(c, emic));
-        TRY(sumrc_into(c, SUM_LSWAE));
-      } else if (op == 2 && any_cex) {
-        TRY(run_plane(c, SEQ_CEX, 0, 0, ns));
-        TRY(sumrc_into(c, SUM_LSCHA));
-      } else if (op == 3 && flc.n) {
-        TRY(run_pitch(c, flc));  // no SUMRC after FLCscatter
-      }
-    }
-    return RAMGPU_OK;
-  };
-  TRY(run_r(c, rec, 0, ns));
-  TRY(run_p(c, rec, 0, ns));
-  TRY(run_plane(c, SEQ_E, rec, 0, ns));
-  TRY(run_plane(c, SEQ_MU, rec, 0, ns));
-  TRY(sumrc_into(c, SUM_LSDR));
-  if (coul) {
-    TRY(run_plane(c, SEQ_COULEN, 0, 0, ns));
-    TRY(sumrc_into(c, SUM_LSCOE));
-    TRY(run_plane(c, SEQ_COULMU, clamp, 0, ns));
-    TRY(sumrc_into(c, SUM_LSCSC));
-  }
-  TRY(half(true));
-  for (int a = 0; a < 2; ++a) {
-    TRY(run_plane(c, SEQ_ATM, 0, 0, ns));
-    TRY(sumrc_into(c, SUM_LSATM));
-  }
-  TRY(half(false));
-  if (coul) {
-    TRY(run_plane(c, SEQ_COULMU, clamp, 0, ns));
-    TRY(sumrc_into(c, SUM_LSCSC));
-    TRY(run_plane(c, SEQ_COULEN, 0, 0, ns));
-    TRY(sumrc_into(c, SUM_LSCOE));
-  }
-  TRY(run_plane(c, SEQ_MU, 0, 0, ns));
-  TRY(run_plane(c, SEQ_E, 0, 0, ns));
-  TRY(run_p(c, 0, 0, ns));
-  TRY(run_r(c, 2, 0, ns));
-  TRY(run_finalize(c, rec ? 15 : 0, 1 | kSumFromRadial | (SUM_LSDR << kSumAccShift), 0, ns));
-#undef TRY
-  return RAMGPU_OK;
-}
-
 }  // namespace ramgpu_host
 
 extern "C" {
@@ -179,13 +83,11 @@ extern "C" {
 int ramgpu_set_wpadif(ramgpu_ctx *c, int s, const double *d1, const double *d2, int at_wpi, int at_emic) {
   int rc = check_ctx(c);
   if (rc || (rc = check_species(c, s))) return rc;
-  if (!d1) {
-    c->pd_wpi[s - 1] = c->pd_emic[s - 1] = 0;
-    return RAMGPU_OK;
-  }
-  if ((rc = upload_coef(c, &c->d_pdc[s - 1], d1, d2))) return rc;
-  c->pd_wpi[s - 1] = at_wpi ? 1 : 0;
-  c->pd_emic[s - 1] = at_emic ? 1 : 0;
+  if (d1 && (rc = upload_coef(c, &c->d_pdc[s - 1], d1, d2))) return rc;
+  c->t.pdc[s - 1] = c->d_pdc[s - 1];
+  c->t.pd_wpi[s - 1] = (d1 && at_wpi) ? 1 : 0;
+  c->t.pd_emic[s - 1] = (d1 && at_emic) ? 1 : 0;
+  c->tab_dirty = true;
   return RAMGPU_OK;
 }
 
@@ -202,23 +104,25 @@ int ramgpu_set_flc(ramgpu_ctx *c, int s, const double *coef, double dt_bc) {
   if (rc || (rc = check_species(c, s))) return rc;
   c->dt_bc = dt_bc;
   if (!coef) {
-    c->d_flc[s - 1] = nullptr;  // the table stays allocated for a later call
+    c->t.flc[s - 1] = nullptr;  // the table stays allocated for a later call
+    c->tab_dirty = true;
     return RAMGPU_OK;
   }
   double *slot = c->d_flc_mem[s - 1];
   if ((rc = upload_coef(c, &slot, coef, nullptr))) return rc;
   c->d_flc_mem[s - 1] = slot;
-  c->d_flc[s - 1] = slot;
+  c->t.flc[s - 1] = slot;
+  c->tab_dirty = true;
   return RAMGPU_OK;
 }
 
 int ramgpu_flcscatter(ramgpu_ctx *c, int s) {
   int rc = check_ctx(c);
   if (rc || (rc = check_species(c, s))) return rc;
-  if (!c->d_flc[s - 1]) return fail(RAMGPU_ESTATE, "species %d has no FLC coefficients (ramgpu_set_flc)", s);
+  if (!c->t.flc[s - 1]) return fail(RAMGPU_ESTATE, "species %d has no FLC coefficients (ramgpu_set_flc)", s);
   if (c->time_elapsed < c->dt_bc) return RAMGPU_OK;  // src/ModRamLoss.f90:526
   if ((rc = prepare(c))) return rc;
-  return run_pitch(c, s - 1, c->d_flc[s - 1]);
+  return run_pitch(c, s - 1, c->t.flc[s - 1]);
 }
 
 }  // extern "C"

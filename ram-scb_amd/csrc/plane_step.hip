@@ -52,7 +52,46 @@ struct StepLds {
   double *kt;  // SKT_N*NE, then EDOT, log(ATLOS) and WAVELO's factor of the plane (NE each)
   double *ex, *red;
   unsigned long long *cmx;
+  // SEQ_STEPX: per row {XNE, BASCNE, MU, 1/MU, FNHS*MU, its reciprocal}; 3*NE handed between chunks by the line solves
+  double *ct, *cy;
 };
+// slots of red per wave
+constexpr int kStepSums = 7, kStepXSums = kSumSlots;
+struct Yes {
+  static constexpr bool value = true;
+};
+struct No {
+  static constexpr bool value = false;
+};
+
+// Per-row terms of the Coulomb operators and the line solves: XNE(L) =
+// NECR(I,J)*BANE(L) with the bounce factor BANE(L) = (1-FNIS/2/FNHS)/(1-MU^2)
+// (src/ModRamCoul.f90:167-172; rows L >= NPA-10 take BANE(NPA-11)),
+// BASCNE(L) = NECR*BOUNIS/2/BOUNHS (:263), MU, FACMU = FNHS*MU and the
+// reciprocals of the last two (those of row 1, MU = 0, are not used).
+__device__ inline void step_line_tables(CTab &t, const StepLds &d, int i, int j, int npap) {
+  const int NPA = t.npa, I = i + 1, J = j + 1;
+  const bool coul = t.coul != 0;
+  const double necr = coul ? t.necr[i + (size_t)t.nr * j] : 0.0;
+  for (int x = threadIdx.x; x < npap; x += blockDim.x) {
+    const int l = min(x, NPA - 1), L = l + 1;
+    double *r = d.ct + 6 * x;
+    double xne = 0.0, xb = 0.0;
+    if (coul) {
+      const int lb = min(L, NPA - 11);
+      const double mub = t.mu[lb - 1];
+      xne = necr * ((1. - GEO3(t.fnis, I, J, lb) / 2. / GEO3(t.fnhs, I, J, lb)) / (1. - mub * mub));
+      xb = necr * GEO3(t.bounis, I, J, L) / 2. / GEO3(t.bounhs, I, J, L);
+    }
+    const double mu = t.mu[l], fac = GEO3(t.fnhs, I, J, L) * mu;
+    r[0] = xne;
+    r[1] = xb;
+    r[2] = mu;
+    r[3] = 1.0 / mu;
+    r[4] = fac;
+    r[5] = 1.0 / fac;
+  }
+}
 
 // Loads of the descriptor and of a plane's scalars go through the constant
 // address space: as plain loads they were vector loads in a chain of two or
@@ -60,11 +99,16 @@ struct StepLds {
 //
 // SEQ_STEP in place (or from src to dst); SEQ_TAPE out of place: also the
 // output of every phase but the last to the tape slots after src, and the
-// clamp decisions of the drift phases.
+// clamp decisions of the drift phases.  SEQ_STEPX in place with the optional
+// processes the problem has on: COULEN and COULMU, WPADIF at the WPI and EMIC
+// positions, FLCscatter (src/ModRamRun.f90:81-172).  rec: bit 0 record the
+// CFL maxima, bit 1 COULMU's clamp (TimeRamElapsed > 0), bit 2 FLCscatter
+// acts (TimeRamElapsed >= Dt_bc).
 template <int SEQ, int R>
 __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step(Launch L, int rec) {
-  constexpr bool TAPE = SEQ == SEQ_TAPE;
-  constexpr bool kKeepE = R <= 4, kKeepMu = R <= 9;
+  constexpr bool TAPE = SEQ == SEQ_TAPE, X = SEQ == SEQ_STEPX;
+  constexpr bool kKeepE = R <= 4 && !X, kKeepMu = R <= (TAPE ? 8 : 9) && !X;
+  constexpr int kSums = X ? kStepXSums : kStepSums;
   extern __shared__ __align__(16) double sm[];
   for (int vb = blockIdx.x; vb < L.nv; vb += gridDim.x) {
     const CUnit u = const_unit(L, vb);
@@ -93,9 +137,14 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step
     d.kt = d.lt + 4 * (NPAP + 1);
     d.ex = d.kt + (SKT_N + 2) * NE;
     d.red = d.ex + 64;
-    d.cmx = (unsigned long long *)(d.red + 112);
-    const bool apart = t.step_apart != 0;
+    d.cmx = (unsigned long long *)(d.red + 16 * kSums);
+    const bool apart = (X ? t.stepx_apart : t.step_apart) != 0;
     d.H = apart ? (double *)(d.cmx + NE + kStepSpread * NPA) : d.F;
+    if constexpr (X) {
+      const int o = (int)((double *)(d.cmx + NE + kStepSpread * NPA) - sm) + (apart ? 4 * ncol : 0);
+      d.ct = sm + (o + 1) / 2 * 2;
+      d.cy = d.ct + 6 * NPAP;
+    }
 
     // this thread's column; a wave's lane 0 repeats the last column of the
     // wave before (step_wave_cells), so that every energy face's upper
@@ -171,6 +220,7 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step
       for (int e = n1 + tid; e < 4 * NPAP; e += T) l0_[e] = l1_[e] = d2{0.0, 0.0};
       for (int e = n2 + tid; e < NPAP; e += T) d.cl[e] = 0.0;
       for (int e = n3 + tid; e < 2 * (NPAP + 1); e += T) l3_[e] = d2{0.0, 0.0};
+      if constexpr (X) step_line_tables(t, d, i, j, NPAP);
       if (rec & 1)
         for (int e = tid; e < NE + kStepSpread * NPA; e += T) d.cmx[e] = 0ull;
     }
@@ -183,8 +233,9 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step
   const double bij = kij[KIJ_BIJ], rbij = kij[KIJ_RBIJ]
 
     // rows into LDS; the thread that holds F(2) forms DRIFTE's relativistic
-    // ghosts F(1), F(0) from it (src/ModRamDrift.f90:333-335)
-    auto rows_out = [&]() __attribute__((always_inline)) {
+    // ghosts F(1), F(0) from it (src/ModRamDrift.f90:333-335), or COULEN's,
+    // with the square roots of the inverse ratios (src/ModRamCoul.f90:180-181)
+    auto rows_out = [&](auto coul) __attribute__((always_inline)) {
       if (own) {
         THREAD_CELLS;
         double *const Frow = d.F + l0 * S + k;
@@ -194,7 +245,13 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step
         }
         if (k == 1) {
           const cptr<double> rel = as_const((const double *)fresh_uniform(tp)->rel) + s * 8;
-          const double r0 = rel[0], r1 = rel[1], r2 = rel[2], r3 = rel[3], r4 = rel[4], rr1 = rel[5], rr0 = rel[6];
+          double r2 = rel[2], r4 = rel[4];
+          if constexpr (decltype(coul)::value) {
+            const cptr<double> crel = as_const((const double *)fresh_uniform(tp)->crel) + s * 5;
+            r2 = crel[2];
+            r4 = crel[4];
+          }
+          const double r0 = rel[0], r1 = rel[1], r3 = rel[3], rr1 = rel[5], rr0 = rel[6];
 #pragma unroll
           for (int n = 0; n < R; ++n) {
             const double g1 = div_rn(f[n] * r0, r1, rr1) * r2;
@@ -218,8 +275,11 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step
 
     // DRIFTE (src/ModRamDrift.f90:333-369); K=1 is not updated.  The owner of
     // face K forms F(K) - C(K)/WE(K)*FBND(K) and the term C(K)/WE(K+1)*FBND(K)
-    // that the next lane adds.
-    auto drift_e = [&](bool first, unsigned char *cb) __attribute__((always_inline)) {
+    // that the next lane adds.  coul: COULEN instead (src/ModRamCoul.f90:
+    // 154-217), the same sweep with CccolE(K) = (COULE+COULI)(S,K,L)*XNE(L) on
+    // rows L=2..NPA, no CFL record.
+    auto drift_e = [&](auto coul, bool first, unsigned char *cb) __attribute__((always_inline)) {
+      constexpr bool COUL = decltype(coul)::value;
       THREAD_CELLS;
       PLANE_SCALARS;
       const double *const Frow = d.F + l0 * S + k;  // row n: Frow[n*S + 0..3] = F(K-1)..F(K+2)
@@ -231,14 +291,21 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step
       const bool top = k + 1 >= NE;  // its upper term goes to a lane that does not use it
       const double we1 = top ? 1.0 : kt[SKT_WE * NE + 1], rwe1 = top ? 1.0 : kt[SKT_RWE * NE + 1];
       const double *const cf = d.cf + 8 * l0;
-      double cmax = 0.0;
+      double cmax = 0.0, cc[COUL ? R : 1];
+      if constexpr (COUL) {
+        const gptr<const double> gc = as_global(tt.cc + (size_t)s * NPA * NE);
+#pragma unroll
+        for (int n = 0; n < R; ++n) cc[n] = gc[(unsigned)(min(l0 + n, NPA - 1) * NE + k)] * d.ct[6 * (l0 + n)];
+      }
 #pragma unroll
       for (int n = 0; n < R; ++n) {
         const double *p = Frow + n * S;
-        const double ce = (kKeepE && !first) ? kce[kKeepE ? n : 0]
-                                             : c_energy(cf + 8 * n, ekp, edot, drd1, dpd1, bij, rbij, rlz, rrlz);
+        double ce;
+        if constexpr (COUL) ce = cc[n];
+        else ce = (kKeepE && !first) ? kce[kKeepE ? n : 0]
+                                     : c_energy(cf + 8 * n, ekp, edot, drd1, dpd1, bij, rbij, rlz, rrlz);
         if (kKeepE && first) kce[n] = ce;
-        cmax = fmax(cmax, fabs(ce));
+        if (!COUL) cmax = fmax(cmax, fabs(ce));
         const bool neg = ce < 0;
         const double f0 = p[1], fp1 = p[2], a = p[neg ? 3 : 0];
         const double u2 = face_value2(f0, fp1, neg ? fp1 : f0, a, neg, div_rn(ce, de, rde), beta);
@@ -247,11 +314,11 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step
         double v = fma(0.5, from_lane_below0(h), w);
         if (k >= 1) {
           if (TAPE && n < nr) clamp_byte(cb, l0 + n, k, v);
-          f[n] = v < 0 ? 1E-15 : v;
+          if (!(COUL && n == 0 && l0 == 0)) f[n] = v < 0 ? 1E-15 : v;
         }
         f[n] = row_done(f[n]);
       }
-      if (first && record && own) atomic_max_pos(&d.cmx[k], fmax(cmax, 1E-10));
+      if (!COUL && first && record && own) atomic_max_pos(&d.cmx[k], fmax(cmax, 1E-10));
     };
 
     // DRIFTMU (src/ModRamDrift.f90:413-466).  F(1)=F(2) for the stencil;
@@ -314,8 +381,13 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step
         const cptr<double> fh = as_const(tt.fnhs) + i + (size_t)(NR + 1) * (j + (size_t)NT * (NPA - 2));
         const cptr<double> mu = as_const(tt.mu) + NPA - 2;
         double b = f[0];
+        // row_done: as a plain choice among f[n] the compiler may make it one
+        // load at a variable index, which puts the rows into scratch memory
 #pragma unroll
-        for (int n = 1; n < R - 1; ++n) b = (l0 + n == NPA - 2) ? f[n] : b;
+        for (int n = 1; n < R - 1; ++n) {
+          const double fn = row_done(f[n]);
+          b = (l0 + n == NPA - 2) ? fn : b;
+        }
         const double topv = b * fh[(size_t)(NR + 1) * NT] * mu[1] / fh[0] / mu[0];
 #pragma unroll
         for (int n = 1; n < R; ++n) f[n] = (l0 + n >= NPA - 1) ? topv : f[n];
@@ -335,12 +407,10 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step
     double *const slot = TAPE ? const_cast<double *>(src) + po : nullptr;
     unsigned char *const cb = TAPE ? reinterpret_cast<unsigned char *>(const_cast<double *>(src) + 7 * tn) + po : nullptr;
 
-    rows_out();
-    drift_e(true, cb);
-    if (TAPE) store(slot + tn);
-    if (!apart) __syncthreads();  // the energy stencil is read
-    drift_mu(true, TAPE ? cb + tn : nullptr);
-    if (TAPE) store(slot + 2 * tn);
+    // EKEV*WE of this thread's cells in SUMRC (I,K,L>=2, J<=NT-1), else 0
+    auto sum_factor = [&](int k) __attribute__((always_inline)) {
+      return (own && j <= NT - 2 && k >= 1) ? d.kt[SKT_EKW * NE + k] : 0.0;
+    };
 
     // The loss chain (src/ModRamRun.f90:77-159): SUMRC, [WAVELO, SUMRC],
     // [CEX, SUMRC], ATMOL, SUMRC, ATMOL, SUMRC, [CEX, SUMRC], [WAVELO,
@@ -348,13 +418,13 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step
     // without it: a factor of exactly 1), ATMOL on K>=2, L>=UPA(I) (its
     // log(ATLOS) is 0 for K=1), WAVELO on K,L>=2; a weight of 0 leaves a cell
     // out of the sums.
-    {
+    auto losses = [&]() __attribute__((always_inline)) {
       THREAD_CELLS;
       CTab &tt = *fresh_uniform(tp);
       const bool cex = tt.cex[s] != 0, wpi = tt.wpi[s] != 0;
       const int upa = as_const(tt.upa)[i];
       const double sigv = d.kt[SKT_SIGV * NE + k], latl = d.kt[(SKT_N + 1) * NE + k];
-      const double ekw = (own && j <= NT - 2 && k >= 1) ? d.kt[SKT_EKW * NE + k] : 0.0;
+      const double ekw = sum_factor(k);
       double wave = 1.0;
       if (wpi && k >= 1) wave = as_global(tt.wavef + (((size_t)s * NR + i) * NT + j) * NE)[(unsigned)k];
       const double dts = tt.dts;
@@ -401,20 +471,258 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step
       for (int m = 0; m < 7; ++m) s7[m] = wave_sum(s7[m]);
       if (lane == 63)
 #pragma unroll
-        for (int m = 0; m < 7; ++m) d.red[wv * 7 + m] = s7[m];
+        for (int m = 0; m < 7; ++m) d.red[wv * kSums + m] = s7[m];
+    };
+
+    // ---- SEQ_STEPX: the optional processes ---------------------------------
+    // SUMRC's partial of the plane as it stands, slot m
+    auto sum_slot = [&](int m) __attribute__((always_inline)) {
+      THREAD_CELLS;
+      const double ekw = sum_factor(k);
+      const double *const lt = d.lt + 4 * l0;
+      double a = 0.0;
+#pragma unroll
+      for (int n = 0; n < R; ++n)
+        a = fma(f[n], ((n == 0 && l0 == 0) || l0 + n >= NPA) ? 0.0 : ekw * lt[4 * n + 2], a);
+      a = wave_sum(a);
+      if (lane == 63) d.red[wv * kSums + m] = a;
+    };
+    // The implicit pitch-angle step of every line (I,J,K>=2): the reference's
+    // recurrences in its order, RK(1)=0, RL(1)=-1, RK and RL forward over
+    // L=2..NPA-1, back substitution, F2(NPA)=F2(NPA-1).  f holds RP and
+    // leaves as the solution; an, gn the couplings.  A line runs through its
+    // chunks one after the other, a chunk's rows in one thread's registers:
+    // a row costs the latency of the recurrence alone (DENOM, its reciprocal,
+    // two quotients), since everything else was formed by all threads.  The
+    // other blocks of the CU fill the idle lanes' issue slots.  Plane launch of
+    // 4 species, 35x72 (20x25 grid), by events: with Coulomb collisions 422 us
+    // (the lines in the plane in LDS, one thread each) -> 213; with WPADIF and
+    // FLCscatter too 1430 us a step as one launch per operator -> 416.
+    auto solve = [&](double (&an)[R], double (&gn)[R]) __attribute__((always_inline)) {
+      THREAD_CELLS;
+      const int last = NPA - 2;  // row of L = NPA-1
+      const bool line = own && k >= 1;
+      double rk = 0.0, rl = -1.0, x = 0.0;
+#pragma unroll 1
+      for (int qq = 0; qq < Q; ++qq) {
+        if (line && q == qq) {
+          if (qq > 0) {
+            rk = d.cy[k];
+            rl = d.cy[NE + k];
+          }
+#pragma unroll
+          for (int n = 0; n < R; ++n) {
+            if (n == 0 && qq == 0) {
+              f[0] = 0.0;
+              an[0] = -1.0;
+            } else if (l0 + n <= last) {
+              const double den = an[n] + gn[n] + gn[n] * rl + 1;
+              double y = __builtin_amdgcn_rcp(den);
+              const double e = fma(-den, y, 1.0);
+              y = fma(y, fma(e, e, e), y);  // 1/DENOM within an ulp, as div_fast's
+              rk = div_rn(f[n] + gn[n] * rk, den, y);
+              rl = div_rn(-an[n], den, y);
+              f[n] = rk;
+              an[n] = rl;
+            }
+          }
+          d.cy[k] = rk;
+          d.cy[NE + k] = rl;
+        }
+        __syncthreads();
+      }
+      if (q == Q - 1) x = rk / (1 + rl);
+#pragma unroll 1
+      for (int qq = Q - 1; qq >= 0; --qq) {
+        if (line && q == qq) {
+          if (qq < Q - 1) x = d.cy[2 * NE + k];
+#pragma unroll
+          for (int n = R - 1; n >= 0; --n) {
+            if (l0 + n < last) x = f[n] - an[n] * x;
+            f[n] = x;
+          }
+          d.cy[2 * NE + k] = x;
+        }
+        __syncthreads();
+      }
+    };
+    // COULMU (src/ModRamCoul.f90:255-292)
+    auto coulmu = [&]() __attribute__((always_inline)) {
+      double an[R], gn[R];
+      {
+        THREAD_CELLS;
+        const gptr<const double> cg = as_global((const double *)(fresh_uniform(tp)->cag + (size_t)s * NPA * NE));
+#pragma unroll
+        for (int n = 0; n < R; ++n) {
+          const double2 v = ld_d2(cg, (unsigned)(min(l0 + n, NPA - 1) * NE + k));
+          an[n] = v.x;
+          gn[n] = v.y;
+        }
+        const int lm = max(l0 - 1, 0);
+        double xbm = d.ct[6 * lm + 1], bhm = d.cm[8 * lm + KLM_BHS];
+#pragma unroll
+        for (int n = 0; n < R; ++n) {
+          const int l = l0 + n;
+          const double *r = d.ct + 6 * l;
+          const double fh = d.cf[8 * l + KLE_HS], rfh = d.cf[8 * l + KLE_RHS], bh = d.cm[8 * l + KLM_BHS], xb = r[1];
+          an[n] = row_done(div_rn(an[n] * xb, fh, rfh) * bh);
+          gn[n] = row_done(div_rn(gn[n] * xbm, fh, rfh) * bhm);
+          const double rp = div_rn(div_rn(f[n], fh, rfh), r[2], r[3]);
+          f[n] = row_done(own && k >= 1 ? rp : f[n]);  // the cell K=1 is not updated
+          xbm = xb;
+          bhm = bh;
+        }
+      }
+      solve(an, gn);
+      {
+        THREAD_CELLS;
+        const bool clamp = (rec & 2) != 0;
+#pragma unroll
+        for (int n = 0; n < R; ++n) {
+          const int l = l0 + n;
+          double v = f[n] * d.cf[8 * l + KLE_HS] * d.ct[6 * l + 2];
+          if (clamp && v < 0.) v = 1E-15;
+          f[n] = row_done(own && k >= 1 ? v : f[n]);
+        }
+      }
+    };
+    // WPADIF (src/ModRamWPI.f90:643-714) and FLCscatter (src/ModRamLoss.f90:
+    // 513-575) with the coefficients D of one species (device layout)
+    auto diffuse = [&](const double *coef) __attribute__((always_inline)) {
+      double an[R], gn[R];
+      {
+        THREAD_CELLS;
+        const gptr<const double> D = as_global(coef + ij * ((size_t)NE * NPA));
+#pragma unroll
+        for (int n = 0; n < R; ++n) an[n] = D[(unsigned)(min(l0 + n, NPA - 1) * NE + k)];
+        const int lm = max(l0 - 1, 0);
+        double pm = div_rn(D[(unsigned)(lm * NE + k)], d.lt[4 * lm], d.lt[4 * lm + 1]);
+        const double dts = fresh_uniform(tp)->dts;
+#pragma unroll
+        for (int n = 0; n < R; ++n) {
+          const int l = l0 + n;
+          const double *r = d.ct + 6 * l, *lt = d.lt + 4 * l;
+          const double fac = r[4], rfac = r[5], p = div_rn(an[n], lt[0], lt[1]);
+          an[n] = row_done(div_rn(div_rn(p * dts, fac, rfac), lt[2], lt[3]));
+          gn[n] = row_done(div_rn(div_rn(pm * dts, fac, rfac), lt[2], lt[3]));
+          f[n] = row_done(own && k >= 1 ? div_rn(f[n], fac, rfac) : f[n]);
+          pm = p;
+        }
+      }
+      solve(an, gn);
+      {
+        THREAD_CELLS;
+#pragma unroll
+        for (int n = 0; n < R; ++n) f[n] = row_done(own && k >= 1 ? f[n] * d.ct[6 * (l0 + n) + 4] : f[n]);
+      }
+    };
+    // CHAREXCHANGE, ATMOL twice (slots 3, 4) and WAVELO on their own
+    auto one_loss = [&](int op) __attribute__((always_inline)) {
+      THREAD_CELLS;
+      CTab &tt = *fresh_uniform(tp);
+      const int upa = as_const(tt.upa)[i];
+      const double dts = tt.dts, ekw = sum_factor(k);
+      const double sigv = d.kt[SKT_SIGV * NE + k], latl = d.kt[(SKT_N + 1) * NE + k];
+      double wave = 1.0, a3 = 0.0, a4 = 0.0;
+      if (op == 2 && tt.wpi[s] != 0 && k >= 1)
+        wave = as_global(tt.wavef + (((size_t)s * NR + i) * NT + j) * NE)[(unsigned)k];
+#pragma unroll
+      for (int n = 0; n < R; ++n) {
+        const int l = l0 + n;
+        const bool row1 = n == 0 && l0 == 0;
+        if (op == 0) {
+          f[n] = row_done(f[n] * exp_tab(row1 ? 0.0 : -(row_done(sigv) * d.cl[l] * dts), d.ex));
+        } else if (op == 1) {
+          const double af = (l + 1 >= upa) ? exp_tab(row_done(latl) * d.cf[8 * l + KLE_RHS], d.ex) : 1.0;
+          const double qw = (row1 || l >= NPA) ? 0.0 : ekw * d.lt[4 * l + 2];
+          double x = f[n] * af;
+          a3 = fma(x, qw, a3);
+          x = x * af;
+          a4 = row_done(fma(x, qw, a4));
+          f[n] = row_done(x);
+        } else {
+          f[n] = row_done(row1 ? f[n] : f[n] * wave);
+        }
+      }
+      if (op == 1) {
+        a3 = wave_sum(a3);
+        a4 = wave_sum(a4);
+        if (lane == 63) {
+          d.red[wv * kSums + 3] = a3;
+          d.red[wv * kSums + 4] = a4;
+        }
+      }
+    };
+    // [WAVELO or WPADIF], [EMIC WPADIF], [CEX], [FLC], ATMOL, ATMOL and back
+    // (src/ModRamRun.f90:91-159), with a SUMRC slot after every operator but
+    // FLCscatter, of a species with a line solve in the chain
+    auto losses_solves = [&]() {
+#pragma unroll 1
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll 1
+        for (int o = 0; o < 4; ++o) {
+          const int op = h == 0 ? o : 3 - o;
+          CTab &tt = *fresh_uniform(tp);
+          if (op == 0) {
+            if (h == 0) sum_slot(0);
+            if (tt.pd_wpi[s]) diffuse(tt.pdc[s]);
+            else if (tt.wpi[s]) one_loss(2);
+            sum_slot(h == 0 ? 1 : 6);
+          } else if (op == 1) {
+            if (tt.pd_emic[s]) diffuse(tt.pdc[s]);
+            sum_slot(h == 0 ? kSumEmic : kSumEmic + 1);
+          } else if (op == 2) {
+            if (tt.cex[s]) one_loss(0);
+            sum_slot(h == 0 ? 2 : 5);
+          } else if ((rec & 4) && tt.flc[s]) {
+            diffuse(tt.flc[s]);
+          }
+        }
+        if (h == 0) one_loss(1);
+      }
+    };
+
+    rows_out(No());
+    drift_e(No(), true, cb);
+    if (TAPE) store(slot + tn);
+    if (!apart) __syncthreads();  // the energy stencil is read
+    drift_mu(true, TAPE ? cb + tn : nullptr);
+    if (TAPE) store(slot + 2 * tn);
+    if constexpr (X) {
+      const bool coul = tp->coul != 0;
+      if (coul) {
+        sum_slot(kSumCoul);
+        if (!apart) __syncthreads();  // the chunks' edge terms are read
+        rows_out(Yes());
+        drift_e(Yes(), false, nullptr);
+        sum_slot(kSumCoul + 1);
+        coulmu();
+      }
+      if (tp->pd_wpi[s] || tp->pd_emic[s] || tp->flc[s]) losses_solves();
+      else losses();
+      if (coul) {
+        coulmu();
+        sum_slot(kSumCoul + 2);
+        rows_out(Yes());
+        drift_e(Yes(), false, nullptr);
+        sum_slot(kSumCoul + 3);
+        if (!apart) __syncthreads();  // the energy stencil is read
+      }
+    } else {
+      losses();
     }
     if (TAPE) store(slot + 3 * tn);
     drift_mu(false, TAPE ? cb + 2 * tn : nullptr);
     if (TAPE) store(slot + 4 * tn);
     if (!apart) __syncthreads();  // the chunks' edge terms are read
-    rows_out();
-    drift_e(false, TAPE ? cb + 3 * tn : nullptr);
+    rows_out(No());
+    drift_e(No(), false, TAPE ? cb + 3 * tn : nullptr);
     store(dst + po);
     // SUMRC partials and the CFL maxima, complete since the first DRIFTMU's
     // and the loss chain's next barriers
-    if (tid < 7) {
+    if (tid < kSums) {
       double v = 0.0;
-      for (int w = 0; w < (int)(blockDim.x >> 6); ++w) v += d.red[w * 7 + tid];
+      for (int w = 0; w < (int)(blockDim.x >> 6); ++w) v += d.red[w * kSums + tid];
       CTab &tt = *fresh_uniform(tp);
       tt.partials[((size_t)tid * tt.ns + s) * tt.maxblk + u.b] = v;
     }
@@ -445,7 +753,8 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step
 // translation unit of its own.
 #define STEP_INST(r)                                               \
   template __global__ void k_plane_step<SEQ_STEP, r>(Launch, int); \
-  template __global__ void k_plane_step<SEQ_TAPE, r>(Launch, int);
+  template __global__ void k_plane_step<SEQ_TAPE, r>(Launch, int); \
+  template __global__ void k_plane_step<SEQ_STEPX, r>(Launch, int);
 #if defined(STEP_ONE)
 STEP_INST(STEP_ONE)
 #elif STEP_PART == 0

@@ -30,18 +30,13 @@ constexpr int kMaxPlaneCells = kPlaneThreads * kMaxCellsPerThread;  // NE*NPA bo
 // SUMRC partial-sum slots of one ram_run: 0..6 the loss chain's (plane
 // blocks), 7 the last SUMRC (radial blocks), 8..11 the Coulomb operators'
 // (plane blocks: after the first drift half, after COULEN; after the second
-// COULMU, after the second COULEN)
-constexpr int kSumSlots = 12;
+// COULMU, after the second COULEN), 12, 13 after the EMIC WPADIFs
+constexpr int kSumSlots = 14;
 constexpr int kSumRadial = 7;
 constexpr int kSumCoul = 8;
-// k_finalize's summode: bits 0-1 the mode (0 none, 1 one SUMRC, 2 the
-// fused step's chain); with mode 1, kSumFromRadial reads the radial slot
-// and bits kSumAccShift.. name the accumulator the ELORC goes to
-constexpr int kSumModeMask = 3;
-constexpr int kSumFromRadial = 1 << 2;
-constexpr int kSumAccShift = 4;
-enum SumAcc { SUM_NONE = 0, SUM_LSDR = 1, SUM_LSCHA = 2, SUM_LSATM = 3, SUM_LSWAE = 4, SUM_LSCOE = 5,
-              SUM_LSCSC = 6 };
+constexpr int kSumEmic = 12;
+enum SumAny { ANY_WPI = 1, ANY_EMIC = 2, ANY_CEX = 4 };
+// k_finalize's summode: 0 none, 1 one SUMRC (slot 0), 2 the fused step's chain
 constexpr int kMuSpread = 4;           // LDS slots per pitch-angle row of DRIFTMU's CFL maximum (by K mod 4)
 constexpr int kFinalizeThreads = 1024;  // one block per (problem, species) of k_finalize (and of k_ghost)
 
@@ -117,6 +112,12 @@ struct Tab {
   // ..] = GREL(S,1), GREL(S,2), SQRT((GREL1^2-1)/(GREL2^2-1)), GRZERO(S),
   // SQRT((GRZERO^2-1)/(GREL1^2-1)); NECR (NR,NT) in the reference's layout
   int coul;
+  // WPADIF and FLCscatter: per species whether ram_run takes WPADIF at the
+  // WPI positions (in place of WAVELO) and at the EMIC positions, and the
+  // coefficient tables (F2's device layout; flc null: no FLCscatter)
+  int pd_wpi[kMaxSpecies], pd_emic[kMaxSpecies];
+  int sum_any;  // SumAny bits: the operators that some species takes
+  const double *pdc[kMaxSpecies], *flc[kMaxSpecies];
   double *cc;
   double2 *cag;
   double *crel;
@@ -134,6 +135,7 @@ struct Tab {
   // threads above, in a block of any size, are idle
   int plane_chunks;
   int step_cells, step_apart;  // step_wave_cells, step_edges_apart of k_plane_step's shape
+  int stepx_apart;             // step_edges_apart of SEQ_STEPX's
   // state
   double *f2;
   double *partials;  // [slot][s][maxblk]
@@ -285,13 +287,21 @@ inline __host__ __device__ int step_resident(size_t lds, int ne, int npa, int ro
   const int by_waves = kStepSimdWaves / simd, by_lds = (int)(kLdsCu / lds);
   return by_waves < by_lds ? by_waves : by_lds;
 }
-inline __host__ __device__ bool step_edges_apart(int ne, int npa, int rows) {
-  const size_t base = step_lds_doubles(ne, npa, rows) * 8, edges = 4 * (size_t)step_chunks(npa, rows) * ne * 8;
+// SEQ_STEPX's further LDS: wider sums, the per-row terms of the line solves
+// and what they hand between chunks
+inline __host__ __device__ size_t step_extra_bytes(int ne, int npa, int rows) {
+  return (16 * (size_t)(kSumSlots - 7) + 1 + 6 * (size_t)step_chunks(npa, rows) * rows + 3 * (size_t)ne) *
+         sizeof(double);
+}
+// x: SEQ_STEPX
+inline __host__ __device__ bool step_edges_apart(int ne, int npa, int rows, bool x = false) {
+  const size_t base = step_lds_doubles(ne, npa, rows) * 8 + (x ? step_extra_bytes(ne, npa, rows) : 0);
+  const size_t edges = 4 * (size_t)step_chunks(npa, rows) * ne * 8;
   return step_resident(base + edges, ne, npa, rows) >= step_resident(base, ne, npa, rows);
 }
-inline __host__ __device__ size_t step_lds_bytes(int ne, int npa, int rows) {
-  return step_lds_doubles(ne, npa, rows) * 8 +
-         (step_edges_apart(ne, npa, rows) ? 4 * (size_t)step_chunks(npa, rows) * ne * 8 : 0);
+inline __host__ __device__ size_t step_lds_bytes(int ne, int npa, int rows, bool x = false) {
+  return step_lds_doubles(ne, npa, rows) * 8 + (x ? step_extra_bytes(ne, npa, rows) : 0) +
+         (step_edges_apart(ne, npa, rows, x) ? 4 * (size_t)step_chunks(npa, rows) * ne * 8 : 0);
 }
 // The Coulomb operators' LDS after the forward plane kernels': per L the
 // bounce-averaged density XNE, BASCNE, FNHS, BOUNHS, MU, 1/FNHS and 1/MU

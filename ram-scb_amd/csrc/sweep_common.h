@@ -547,12 +547,12 @@ enum PlaneSeq : int {
   SEQ_WAVE = 8,  // WAVELO
   SEQ_COULEN = 9,   // COULEN
   SEQ_COULMU = 10,  // COULMU
-  SEQ_STEPC = 11,   // SEQ_STEP with Coulomb collisions: DRIFTE, DRIFTMU, COULEN, COULMU, loss chain,
-                    // COULMU, COULEN, DRIFTMU, DRIFTE with their SUMRC partials
+  SEQ_STEPX = 11,   // SEQ_STEP with the optional processes the problem has on: COULEN, COULMU, WPADIF, FLCscatter
+                    // at their places with their SUMRC partials (k_plane_step)
 };
 // plane kernels whose LDS holds the Coulomb operators' tables
 __host__ __device__ constexpr bool seq_coul(int seq) {
-  return seq == SEQ_COULEN || seq == SEQ_COULMU || seq == SEQ_STEPC;
+  return seq == SEQ_COULEN || seq == SEQ_COULMU;
 }
 
 // Elements of one F2-sized buffer (all species) of the problem t.
