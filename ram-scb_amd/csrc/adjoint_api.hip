@@ -166,7 +166,7 @@ size_t bwd_lds(const ramgpu_ctx *c) {
 
 // backward kernels over species s0..s0+nsp-1
 int bwd_r(ramgpu_ctx *c, int final_sweep, const double *x, double *adj, double *bbar, int s0, int nsp) {
-  const Launch L = launch_of(c, s0, nsp, blocks_r(c->t));
+  const Launch L = launch_of(c, s0, nsp, blocks_line_r(c->t));
   tbeg(c, RAMGPU_KERNEL_R_BWD);
   if (final_sweep)
     hipLaunchKernelGGL(k_r_bwd<1>, dim3(L.nv), dim3(kLineThreads), radial_lds_bytes(c->nr, c->ne, c->npa), c->stream,
@@ -179,7 +179,7 @@ int bwd_r(ramgpu_ctx *c, int final_sweep, const double *x, double *adj, double *
 }
 
 int bwd_p(ramgpu_ctx *c, const double *x, double *adj, int s0, int nsp) {
-  const Launch L = launch_of(c, s0, nsp, blocks_p(c->t));
+  const Launch L = launch_of(c, s0, nsp, blocks_line_p(c->t));
   tbeg(c, RAMGPU_KERNEL_P_BWD);
   hipLaunchKernelGGL(k_p_bwd, dim3(L.nv), dim3(kLineThreads), azim_lds_bytes(c->nt, c->ne, c->npa), c->stream, L, x,
                      adj);

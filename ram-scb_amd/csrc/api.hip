@@ -295,14 +295,8 @@ int run_r(ramgpu_ctx *c, int mode, int s0, int nsp, const double *src, double *d
   Launch L = launch_of(c, s0, nsp, blocks_r(c->t));
   L.src = src;
   L.dst = dst;
-  const size_t lds = radial_lds_bytes(c->nr, c->ne, c->npa);
   tbeg(c, RAMGPU_KERNEL_R);
-  if (mode == 0)
-    hipLaunchKernelGGL(k_r<0>, dim3(L.nv), dim3(kLineThreads), lds, c->stream, L);
-  else if (mode == 1)
-    hipLaunchKernelGGL(k_r<1>, dim3(L.nv), dim3(kLineThreads), lds, c->stream, L);
-  else
-    hipLaunchKernelGGL(k_r<2>, dim3(L.nv), dim3(kLineThreads), lds, c->stream, L);
+  launch_r(mode, r_shape(c), dim3(L.nv), c->stream, L);
   tend(c);
   return launch_check("k_r");
 }
@@ -310,16 +304,11 @@ int run_r(ramgpu_ctx *c, int mode, int s0, int nsp, const double *src, double *d
 int run_p(ramgpu_ctx *c, int rec, int s0, int nsp, const double *src, double *dst) {
   // out of place, extra lines copy the unswept I=1 rows
   const bool copy = dst && dst != src;
-  const int P = c->ne * c->npa;
-  const int nb = copy ? ((c->nr - 1) * P + c->nt * P + kLineThreads - 1) / kLineThreads : blocks_p(c->t);
-  Launch L = launch_of(c, s0, nsp, nb);
+  Launch L = launch_of(c, s0, nsp, copy ? blocks_p_copy(c->t) : blocks_p(c->t));
   L.src = src;
   L.dst = dst;
   tbeg(c, RAMGPU_KERNEL_P);
-  if (rec)
-    hipLaunchKernelGGL(k_p<1>, dim3(L.nv), dim3(kLineThreads), azim_lds_bytes(c->nt, c->ne, c->npa), c->stream, L);
-  else
-    hipLaunchKernelGGL(k_p<0>, dim3(L.nv), dim3(kLineThreads), azim_lds_bytes(c->nt, c->ne, c->npa), c->stream, L);
+  launch_p(rec ? 1 : 0, p_shape(c), dim3(L.nv), c->stream, L);
   tend(c);
   return launch_check("k_p");
 }
@@ -527,8 +516,8 @@ int set_plane_lds_limit(size_t limit) {
       PLANE_K(SEQ_E), PLANE_K(SEQ_MU), PLANE_K(SEQ_CEX), PLANE_K(SEQ_ATM), PLANE_K(SEQ_SUM),
       PLANE_K(SEQ_WAVE),
       PLANE_K(SEQ_COULEN), PLANE_K(SEQ_COULMU),
-      (const void *)k_r<0>, (const void *)k_r<1>, (const void *)k_r<2>,
-      (const void *)k_r_bwd<0>, (const void *)k_r_bwd<1>, (const void *)k_p<0>, (const void *)k_p<1>,
+      (const void *)k_r<0>, (const void *)k_r<1>, (const void *)k_r<2>, (const void *)k_p<0>, (const void *)k_p<1>,
+      (const void *)k_r_bwd<0>, (const void *)k_r_bwd<1>,
 #define STEP_K(r)                                                                           \
   (const void *)k_plane_step<SEQ_STEP, r>, (const void *)k_plane_step<SEQ_TAPE, r>, \
       (const void *)k_plane_step<SEQ_STEPX, r>,
@@ -651,6 +640,8 @@ int ramgpu_create(ramgpu_ctx **out, int ns, int nr, int nt, int ne, int npa, int
   const size_t nf2 = (size_t)ns * nr * nt * ne * npa;
   Tab &t = c->t;
   t.ns = ns; t.nr = nr; t.nt = nt; t.ne = ne; t.npa = npa;
+  t.r_rows = line_rows(nr, (long)ns * nt * ne * npa, ncu);
+  t.p_rows = line_rows(nt, (long)ns * (nr - 1) * ne * npa, ncu);
   t.maxblk = std::max(blocks_kl(t), blocks_r(t));  // partial sums per (slot, species)
   if (plane_bwd_lds_bytes(ne, npa) > c->lds_limit)
     return cleanup(fail(RAMGPU_EINVAL, "NE*NPA=%d plane does not fit the device LDS (%zu bytes)", ne * npa,
@@ -665,7 +656,8 @@ int ramgpu_create(ramgpu_ctx **out, int ns, int nr, int nt, int ne, int npa, int
   t.plane_chunks = plane_chunks_for(ne, npa, c->plane.threads);
   c->step = step_shape(ne, npa, (long)ns * (nr - 1) * nt, ncu, c->lds_limit, false);
   c->stepx = step_shape(ne, npa, (long)ns * (nr - 1) * nt, ncu, c->lds_limit, true);
-  if (c->step.threads == 0 || c->stepx.threads == 0) return cleanup(fail(RAMGPU_EINVAL, "no plane kernel shape for %dx%d", ne, npa));
+  if (c->step.threads == 0 || c->stepx.threads == 0)
+    return cleanup(fail(RAMGPU_EINVAL, "no plane kernel shape for %dx%d", ne, npa));
   t.step_cells = step_wave_cells(ne);
   t.step_apart = step_edges_apart(ne, npa, c->step.rows);
   t.stepx_apart = step_edges_apart(ne, npa, c->stepx.rows, true);

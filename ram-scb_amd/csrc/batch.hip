@@ -31,15 +31,18 @@ namespace {
 // kernel kinds of an ensemble launch; the last four serve reverse mode: P and
 // plane out of place (with the copy lines / planes of the unswept I=1 rows),
 // one unit per member (misfit) and a whole-F2 copy per member
-enum BatchKind { BK_SCHED, BK_COEFIJ, BK_GHOST, BK_R, BK_P, BK_PLANE, BK_FIN, BK_POOP, BK_PLOOP, BK_MEM, BK_COPY, BK_N };
+enum BatchKind {
+  BK_SCHED, BK_COEFIJ, BK_GHOST, BK_R, BK_P, BK_PLANE, BK_FIN, BK_POOP, BK_PLOOP, BK_RB, BK_PB, BK_MEM, BK_COPY, BK_N
+};
 
 struct Plan {
   Job *jobs = nullptr;
   int *vmap = nullptr;
   int nv = 0;
   int cap = 0;  // 0: one block per virtual block; else the persistent grid size
-  // plane kinds: one launch per shape of the members' fused plane kernels,
-  // over the virtual blocks [v0, v0 + nv) of its members
+  // sweep and plane kinds: one launch per shape of the members' kernels,
+  // over the virtual blocks [v0, v0 + nv) of its members; a sweep's shape is
+  // its rows (0: one thread per line) and the line's cells' chunks
   struct Group {
     StepShape sh;
     size_t lds;
@@ -63,6 +66,10 @@ struct ramgpu_batch {
   PlaneShape plane{64, 8, 0};
   std::vector<char> wave;  // each member's WAVELO at creation (its coefficient units)
   int sum_ns = 0;
+  // DRIFTP and DRIFTR with lines in chunks (line_rows): only if the members'
+  // lines together are as few.  DRIFTR's last sweep keeps a member's own
+  // choice, which its SUMRC's order of summation goes with.
+  bool chunks = false;
   std::vector<int> bs_off;  // first species of member m in a schedule row
   int *d_bsoff = nullptr;
   int *d_step = nullptr;
@@ -88,14 +95,15 @@ int batch_alloc(ramgpu_batch *b, void **p, size_t bytes) {
   return RAMGPU_OK;
 }
 
-int blocks_of(int kind, const ramgpu_ctx *c) {
-  const int P = c->ne * c->npa;
+int blocks_of(const ramgpu_batch *b, int kind, const ramgpu_ctx *c) {
   switch (kind) {
     case BK_COEFIJ: return coef_units(c, 256);
     case BK_R: return blocks_r(c->t);
-    case BK_P: return blocks_p(c->t);
+    case BK_P: return b->chunks ? blocks_p(c->t) : blocks_line_p(c->t);
     case BK_PLANE: return blocks_kl(c->t);
-    case BK_POOP: return ((c->nr - 1) * P + c->nt * P + kLineThreads - 1) / kLineThreads;
+    case BK_POOP: return blocks_p_copy(c->t, b->chunks);
+    case BK_RB: return blocks_line_r(c->t);
+    case BK_PB: return blocks_line_p(c->t);
     case BK_PLOOP: return blocks_kl(c->t) + c->nt;
     case BK_COPY: return 256;
     default: return 1;
@@ -104,26 +112,43 @@ int blocks_of(int kind, const ramgpu_ctx *c) {
 
 bool per_member(int kind) { return kind == BK_SCHED || kind == BK_COEFIJ || kind == BK_MEM || kind == BK_COPY; }
 
-// Job table and block map of one kernel kind, members in order; the plane
-// kinds with the members of one plane-kernel shape together.
+// Job table and block map of one kernel kind, members in order; the sweep
+// and plane kinds with the members of one kernel shape together.
 int build_plan(ramgpu_batch *b, int kind) {
   std::vector<Job> jobs;
   std::vector<int> vmap;
   const bool plane = kind == BK_PLANE || kind == BK_PLOOP;
+  const bool grouped = plane || kind == BK_R || kind == BK_P || kind == BK_POOP;
   std::vector<size_t> order(b->m.size());
   std::iota(order.begin(), order.end(), size_t(0));
-  auto shape = [&](size_t mi) { return std::make_pair(b->m[mi]->step.rows, b->m[mi]->step.threads); };
-  if (plane)
+  auto shape_of = [&](const ramgpu_ctx *c, size_t *lds) {
+    if (plane) {
+      *lds = step_lds_bytes(c->ne, c->npa, c->step.rows);
+      return c->step;
+    }
+    const LineShape h = kind == BK_R ? r_shape(c) : p_shape(c, b->chunks);
+    *lds = h.lds;
+    return StepShape{h.threads, h.rows};
+  };
+  auto shape = [&](size_t mi) {
+    size_t lds;
+    const StepShape h = shape_of(b->m[mi], &lds);
+    return std::make_pair(h.rows, h.threads);
+  };
+  if (grouped)
     std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) { return shape(x) < shape(y); });
   std::vector<Plan::Group> groups;
   for (size_t o = 0; o < order.size(); ++o) {
     const size_t mi = order[o];
     const ramgpu_ctx *c = b->m[mi];
-    if (plane && (o == 0 || shape(order[o - 1]) != shape(mi)))
-      groups.push_back(Plan::Group{c->step, 0, (int)vmap.size(), 0});
-    if (plane) groups.back().lds = std::max(groups.back().lds, step_lds_bytes(c->ne, c->npa, c->step.rows));
+    if (grouped) {
+      size_t lds = 0;
+      const StepShape sh = shape_of(c, &lds);
+      if (o == 0 || shape(order[o - 1]) != shape(mi)) groups.push_back(Plan::Group{sh, 0, (int)vmap.size(), 0});
+      groups.back().lds = std::max(groups.back().lds, lds);
+    }
     const int nsp = per_member(kind) ? 1 : c->ns;
-    const int nb = blocks_of(kind, c);
+    const int nb = blocks_of(b, kind, c);
     if (nb >= (1 << kVmapShift) || jobs.size() + nsp >= (1u << (31 - kVmapShift)))
       return fail(RAMGPU_EINVAL, "ensemble too large for the launch tables");
     const int j0 = (int)jobs.size();
@@ -138,7 +163,7 @@ int build_plan(ramgpu_batch *b, int kind) {
       for (int s = 0; s < nsp; ++s)
         for (int x = 0; x < nb; ++x) vmap.push_back(vmap_entry(j0 + s, x));
     }
-    if (plane) groups.back().nv = (int)vmap.size() - groups.back().v0;
+    if (grouped) groups.back().nv = (int)vmap.size() - groups.back().v0;
   }
   b->plan[kind].groups = groups;
   Plan &p = b->plan[kind];
@@ -177,6 +202,29 @@ void enq_planes(ramgpu_batch *b, int kind, int seq, Launch L, int rec) {
     const int grid = (p.cap > 0 && p.cap < g.nv) ? p.cap : g.nv;
     launch_step(seq, g.sh, dim3((unsigned)grid), g.lds, b->stream, L, rec);
   }
+}
+
+// DRIFTR or DRIFTP (kind BK_P or BK_POOP) of every member: one launch per
+// shape.  L: the launch's slots.
+void enq_lines(ramgpu_batch *b, int kind, Launch L, int mode) {
+  const Plan &p = b->plan[kind];
+  L.jobs = p.jobs;
+  for (const Plan::Group &g : p.groups) {
+    L.vmap = p.vmap + g.v0;
+    L.nv = g.nv;
+    const int grid = (p.cap > 0 && p.cap < g.nv) ? p.cap : g.nv;
+    const LineShape sh{g.sh.rows, g.sh.threads, g.lds};
+    if (kind == BK_R) launch_r(mode, sh, dim3((unsigned)grid), b->stream, L);
+    else launch_p(mode, sh, dim3((unsigned)grid), b->stream, L);
+  }
+}
+void enq_r(ramgpu_batch *b, Launch L, int mode) {
+  if (mode == 2 || b->chunks) return enq_lines(b, BK_R, L, mode);
+  const Plan &p = b->plan[BK_RB];
+  L.jobs = p.jobs;
+  L.vmap = p.vmap;
+  L.nv = p.nv;
+  launch_r(mode, {0, kLineThreads, b->radial_lds}, dim3(grid_for(b, BK_RB)), b->stream, L);
 }
 
 void destroy_graphs(ramgpu_batch *b) {
@@ -253,19 +301,19 @@ int enqueue_step(ramgpu_batch *b, bool sched) {
   const Launch lr = launch_for(b, BK_R), lp = launch_for(b, BK_P), lk = launch_for(b, BK_PLANE),
                lf = launch_for(b, BK_FIN);
   btbeg(b, RAMGPU_KERNEL_R);
-  hipLaunchKernelGGL(k_r<1>, dim3(grid_for(b, BK_R)), dim3(kLineThreads), b->radial_lds, st, lr);
+  enq_r(b, lr, 1);
   btend(b);
   btbeg(b, RAMGPU_KERNEL_P);
-  hipLaunchKernelGGL(k_p<1>, dim3(grid_for(b, BK_P)), dim3(kLineThreads), b->azim_lds, st, lp);
+  enq_lines(b, BK_P, lp, 1);
   btend(b);
   btbeg(b, RAMGPU_KERNEL_PLANE);
   enq_planes(b, BK_PLANE, SEQ_STEP, lk, 1);
   btend(b);
   btbeg(b, RAMGPU_KERNEL_P);
-  hipLaunchKernelGGL(k_p<0>, dim3(grid_for(b, BK_P)), dim3(kLineThreads), b->azim_lds, st, lp);
+  enq_lines(b, BK_P, lp, 0);
   btend(b);
   btbeg(b, RAMGPU_KERNEL_R);
-  hipLaunchKernelGGL(k_r<2>, dim3(grid_for(b, BK_R)), dim3(kLineThreads), b->radial_lds, st, lr);
+  enq_r(b, lr, 2);
   btend(b);
   btbeg(b, RAMGPU_KERNEL_FINALIZE);
   hipLaunchKernelGGL(k_finalize, dim3(grid_for(b, BK_FIN)), dim3(kFinalizeThreads), 0, st, lf, 15, 2);
@@ -321,21 +369,15 @@ void enq_misfit(ramgpu_batch *b, int ssl, int step, int adjoint) {
 void enq_taped_step(ramgpu_batch *b, int g, int dsl_out, bool bookkeeping = true) {
   hipStream_t st = b->stream;
   Launch L = slot_launch(b, BK_R, g + T_R1 + 1, g + T_P1 + 1);
-  if (bookkeeping)
-    hipLaunchKernelGGL(k_r<1>, dim3(grid_for(b, BK_R)), dim3(kLineThreads), b->radial_lds, st, L);
-  else
-    hipLaunchKernelGGL(k_r<0>, dim3(grid_for(b, BK_R)), dim3(kLineThreads), b->radial_lds, st, L);
+  enq_r(b, L, bookkeeping ? 1 : 0);
   L = slot_launch(b, BK_POOP, g + T_P1 + 1, g + T_E1 + 1);
-  if (bookkeeping)
-    hipLaunchKernelGGL(k_p<1>, dim3(L.nv), dim3(kLineThreads), b->azim_lds, st, L);
-  else
-    hipLaunchKernelGGL(k_p<0>, dim3(L.nv), dim3(kLineThreads), b->azim_lds, st, L);
+  enq_lines(b, BK_POOP, L, bookkeeping ? 1 : 0);
   L = slot_launch(b, BK_PLOOP, g + T_E1 + 1, g + T_P2 + 1);
   enq_planes(b, BK_PLOOP, SEQ_TAPE, L, bookkeeping ? 1 : 0);
   L = slot_launch(b, BK_POOP, g + T_P2 + 1, g + T_R2 + 1);
-  hipLaunchKernelGGL(k_p<0>, dim3(L.nv), dim3(kLineThreads), b->azim_lds, st, L);
+  enq_lines(b, BK_POOP, L, 0);
   L = slot_launch(b, BK_R, g + T_R2 + 1, dsl_out);
-  hipLaunchKernelGGL(k_r<2>, dim3(grid_for(b, BK_R)), dim3(kLineThreads), b->radial_lds, st, L);
+  enq_r(b, L, 2);
   if (bookkeeping) {
     const Launch lf = launch_for(b, BK_FIN);
     hipLaunchKernelGGL(k_finalize, dim3(grid_for(b, BK_FIN)), dim3(kFinalizeThreads), 0, st, lf, 15, 2);
@@ -345,17 +387,17 @@ void enq_taped_step(ramgpu_batch *b, int g, int dsl_out, bool bookkeeping = true
 // adjoint of the step taped at group g: Tab::lam in place, Tab::bbar[step]
 void enq_step_bwd(ramgpu_batch *b, int g, int step, size_t bwd_lds, int bwd_threads) {
   hipStream_t st = b->stream;
-  Launch L = slot_launch(b, BK_R, g + T_R2 + 1, 0, step);
-  hipLaunchKernelGGL(k_r_bwd<1>, dim3(grid_for(b, BK_R)), dim3(kLineThreads), b->radial_lds, st, L, nullptr, nullptr,
+  Launch L = slot_launch(b, BK_RB, g + T_R2 + 1, 0, step);
+  hipLaunchKernelGGL(k_r_bwd<1>, dim3(grid_for(b, BK_RB)), dim3(kLineThreads), b->radial_lds, st, L, nullptr, nullptr,
                      nullptr);
-  L = slot_launch(b, BK_P, g + T_P2 + 1, 0);
-  hipLaunchKernelGGL(k_p_bwd, dim3(grid_for(b, BK_P)), dim3(kLineThreads), b->azim_lds, st, L, nullptr, nullptr);
+  L = slot_launch(b, BK_PB, g + T_P2 + 1, 0);
+  hipLaunchKernelGGL(k_p_bwd, dim3(grid_for(b, BK_PB)), dim3(kLineThreads), b->azim_lds, st, L, nullptr, nullptr);
   L = slot_launch(b, BK_PLANE, g + T_E1 + 1, 0);
   launch_plane_bwd(SEQ_STEP, bwd_threads, dim3(grid_for(b, BK_PLANE)), bwd_lds, st, L, nullptr, nullptr);
-  L = slot_launch(b, BK_P, g + T_P1 + 1, 0);
-  hipLaunchKernelGGL(k_p_bwd, dim3(grid_for(b, BK_P)), dim3(kLineThreads), b->azim_lds, st, L, nullptr, nullptr);
-  L = slot_launch(b, BK_R, g + T_R1 + 1, 0, step);
-  hipLaunchKernelGGL(k_r_bwd<0>, dim3(grid_for(b, BK_R)), dim3(kLineThreads), b->radial_lds, st, L, nullptr, nullptr,
+  L = slot_launch(b, BK_PB, g + T_P1 + 1, 0);
+  hipLaunchKernelGGL(k_p_bwd, dim3(grid_for(b, BK_PB)), dim3(kLineThreads), b->azim_lds, st, L, nullptr, nullptr);
+  L = slot_launch(b, BK_RB, g + T_R1 + 1, 0, step);
+  hipLaunchKernelGGL(k_r_bwd<0>, dim3(grid_for(b, BK_RB)), dim3(kLineThreads), b->radial_lds, st, L, nullptr, nullptr,
                      nullptr);
 }
 
@@ -478,6 +520,7 @@ int ramgpu_batch_create(ramgpu_batch **out, ramgpu_ctx *const *members, int nmem
     return cleanup(fail(RAMGPU_EHIP, "stream/event creation failed"));
   int rc;
   if ((rc = batch_alloc(b, (void **)&b->d_tabs, nmembers * sizeof(Tab)))) return cleanup(rc);
+  long lines = 0;
   for (ramgpu_ctx *c : b->m) {
     b->bs_off.push_back(b->sum_ns);
     b->sum_ns += c->ns;
@@ -487,7 +530,9 @@ int ramgpu_batch_create(ramgpu_batch **out, ramgpu_ctx *const *members, int nmem
     b->plane.threads = std::max(b->plane.threads, c->plane.threads);
     b->plane.maxc = std::max(b->plane.maxc, c->plane.maxc);
     b->wave.push_back((char)takes_wave(c));
+    lines += (long)c->ns * std::max(c->nt, c->nr - 1) * c->ne * c->npa;
   }
+  b->chunks = lines <= line_rows_max(b->ncu);
   if ((rc = batch_alloc(b, (void **)&b->d_bsoff, nmembers * sizeof(int))) ||
       (rc = batch_alloc(b, (void **)&b->d_step, sizeof(int))))
     return cleanup(rc);
@@ -845,9 +890,9 @@ int ramgpu_batch_autotune(ramgpu_batch *b, int reps, double *ms_best) {
       for (int r = 0; r <= reps; ++r) {  // first launch warms up
         (void)hipEventRecord(e0, b->stream);
         if (kind == BK_R)
-          hipLaunchKernelGGL(k_r<0>, dim3(grid_for(b, kind)), dim3(kLineThreads), b->radial_lds, b->stream, L);
+          enq_lines(b, BK_R, L, 0);
         else if (kind == BK_P)
-          hipLaunchKernelGGL(k_p<0>, dim3(grid_for(b, kind)), dim3(kLineThreads), b->azim_lds, b->stream, L);
+          enq_lines(b, BK_P, L, 0);
         else
           enq_planes(b, kind, SEQ_STEP, L, 0);
         (void)hipEventRecord(e1, b->stream);

@@ -34,6 +34,8 @@ __global__ void k_coef(Launch L);
 __global__ void k_ghost(Launch L);
 template <int MODE> __global__ void k_r(Launch L);
 template <int MODE> __global__ void k_p(Launch L);
+template <int MODE, int R> __global__ void k_r_rows(Launch L);
+template <int MODE, int R> __global__ void k_p_rows(Launch L);
 template <int SEQ, int MAXC> __global__ void k_plane(Launch L, int rec);
 template <int SEQ, int R> __global__ void k_plane_step(Launch L, int rec);
 __global__ void k_finalize(Launch L, int cflmask, int summode);
@@ -55,6 +57,12 @@ struct PlaneShape {
 // block size and rows per thread of the fused step's plane kernel (k_plane_step)
 struct StepShape {
   int threads, rows;
+};
+
+// block size, rows per thread and LDS of the line sweeps
+struct LineShape {
+  int rows, threads;
+  size_t lds;
 };
 
 struct ramgpu_ctx {
@@ -161,6 +169,14 @@ int coef_units(const ramgpu_ctx *c, int threads);
 bool takes_wave(const ramgpu_ctx *c);
 PlaneShape plane_shape_for(int ne, int npa, int threads);
 StepShape step_shape(int ne, int npa, long planes, int ncu, size_t lds_cu, bool x);
+// rows per thread of k_r_rows or k_p_rows for `lines` lines of n cells (0:
+// k_r, k_p), a context's blocks and LDS, and the launches
+inline long line_rows_max(int ncu) { return 256L * ncu; }  // a wave of lines per SIMD
+int line_rows(int n, long lines, int ncu);
+LineShape r_shape(const ramgpu_ctx *c);
+LineShape p_shape(const ramgpu_ctx *c, bool chunks = true);
+void launch_r(int mode, LineShape sh, dim3 grid, hipStream_t st, const ramgpu::Launch &L);
+void launch_p(int mode, LineShape sh, dim3 grid, hipStream_t st, const ramgpu::Launch &L);
 // launch k_plane_step<seq, rows>
 void launch_step(int seq, StepShape sh, dim3 grid, size_t lds, hipStream_t st, const ramgpu::Launch &L, int rec);
 // launch k_plane<seq, maxc>

@@ -547,20 +547,15 @@ __global__ void __launch_bounds__(kLineThreads, 4) k_r(Launch L) {
         gh1 = ghost_value(t, s, j, k, l, t.conf1);
         gh2 = ghost_value(t, s, j, k, l, t.conf2);
       }
-      double wek = 0, wml = 0, ekk = 0;
-      if (MODE == 2) {
-        wek = t.we[k];
-        wml = t.wmu[l];
-        ekk = t.ekev[k];
-      }
-      const bool sum_line = MODE == 2 && k >= 1 && l >= 1 && j <= NT - 2;
+      double wsum = 0.0;  // EKEV*WE*WMU of the line in SUMRC
+      if (MODE == 2 && k >= 1 && l >= 1 && j <= NT - 2) wsum = t.ekev[k] * t.we[k] * t.wmu[l];
       // face 1: FBND(1) = F(2) on inflow lines, 0 otherwise (:156,164)
       const double f1 = fw[0], f2v = fw[1], f3 = fw[2];
       double fnext = fw[3];  // F(4)
       const double4 r1 = RTERM(0);
       const double c1 = c_radial_of(r1, RSTERM(0), qrow[0], p4k);
       if (MODE == 1 && r1.w == 0.0) cmax = fmax(cmax, fmax(fabs(c1), 1E-10));
-      double gprev = c1 * (in ? f2v : 0.0);
+      double hprev = c1 * (in ? 2.0 * f2v : 0.0);  // twice the flux: the factor 1/2 (exact) is in the update
       if (MODE == 2) {
         const double mg1 = r1.w, mgs = mgt[0];
         if (mg1 == 1.0) fo[0] = 1e-31;
@@ -589,14 +584,14 @@ __global__ void __launch_bounds__(kLineThreads, 4) k_r(Launch L) {
     const double fp1 = last ? gh1 : w1;                                            \
     /* upwind side for C<0: ghost F(NR+2) at face NR, F(NR+1) at face NR-1 */      \
     const double fneg = last ? gh2 : ((I + 2 <= NR) ? w2 : fgh);                   \
-    const double fv = face_value_sel(w0, fp1, neg ? fneg : w0, neg ? fp1 : wm1, ci, ci, beta); \
-    const double fb = (last && !in) ? w0 : fv; /* FBND(NR) = F(NR) on outflow lines */ \
-    const double g = ci * fb;                                                      \
-    double v = w0 - g + gprev;                                                     \
+    const double fv = face_value2(w0, fp1, neg ? fp1 : w0, neg ? fneg : wm1, neg, ci, beta); \
+    const double u2 = (last && !in) ? 2.0 * w0 : fv; /* FBND(NR) = F(NR) on outflow lines */ \
+    const double h = ci * u2;                                                      \
+    double v = fma(0.5, hprev, fma(-0.5, h, w0));                                  \
     if (v < 0) v = 1E-15;                                                          \
-    gprev = g;                                                                     \
+    hprev = h;                                                                     \
     if (MODE == 2) {                                                               \
-      acc += sum_line ? ekk * (v * wek * wml) : 0.0;                               \
+      acc += v;                                                                    \
       fo[(size_t)i * di] = (r.w == 1.0) ? 1e-31 : v;                               \
       if (j == 0) fs[(size_t)i * di] = (mgt[i] == 1.0) ? 1e-31 : v;                \
     } else {                                                                       \
@@ -624,6 +619,7 @@ __global__ void __launch_bounds__(kLineThreads, 4) k_r(Launch L) {
 #undef RSTEP
 #undef RTERM
 #undef RSTERM
+      acc *= wsum;
     }
     if (MODE == 1) {
       const double m = block_max(cmax, red);
@@ -698,8 +694,8 @@ __global__ void __launch_bounds__(kLineThreads) k_p(Launch L) {
       CAZIM(NT, cN, mgN);
       if (MODE == 1 && mgN == 0.0) cmax = fmax(cmax, fmax(fabs(cN), 1E-10));
       // face NT: J1 = 2; upwind N = NT+2 -> 3 (:250-251)
-      const double gN = cN * face_value(FN, F2o, (cN < 0) ? F3 : FN, (cN < 0) ? F2o : FNm1, cN, cN, beta);
-      double gprev = gN;
+      const double hN = cN * face_value2(FN, F2o, (cN < 0) ? F2o : FN, (cN < 0) ? F3 : FNm1, cN < 0, cN, beta);
+      double hprev = hN;  // twice the flux: the factor 1/2 (exact) is in the update
       // step J with F(J+3) = FN_ (0 beyond NT); selects only
 #define PSTEP(JV, FN_)                                                          \
   {                                                                             \
@@ -710,13 +706,12 @@ __global__ void __launch_bounds__(kLineThreads) k_p(Launch L) {
     if (MODE == 1) cmax = (mg == 0.0) ? fmax(cmax, fmax(fabs(cp), 1E-10)) : cmax; \
     /* C<0: N = J+2, or at J = NT-1 N = NT+1 -> 2, N-1 = 1 */                   \
     const bool neg = cp < 0, inr = J + 2 <= NT;                                 \
-    const double fn = neg ? (inr ? w2 : F2o) : w0;                              \
-    const double fnm1 = neg ? (inr ? w1 : F1) : wm1;                            \
-    const double g = cp * face_value_sel(w0, w1, fn, fnm1, cp, cp, beta);      \
-    double v = w0 - g + gprev;                                                  \
+    const double fn = inr ? w2 : F2o, fnm1 = inr ? w1 : F1;                     \
+    const double h = cp * face_value2(w0, w1, neg ? fnm1 : w0, neg ? fn : wm1, neg, cp, beta); \
+    double v = fma(0.5, hprev, fma(-0.5, h, w0));                               \
     if (v < 0) v = 1E-15;                                                       \
     fo[(size_t)(J - 1) * P] = v;                                                \
-    gprev = g;                                                                  \
+    hprev = h;                                                                  \
     wm1 = w0;                                                                   \
     w0 = w1;                                                                    \
     w1 = w2;                                                                    \
@@ -738,7 +733,7 @@ __global__ void __launch_bounds__(kLineThreads) k_p(Launch L) {
       }
 #undef PSTEP
 #undef CAZIM
-      double v = FN - gN + gprev;
+      double v = fma(0.5, hprev, fma(-0.5, hN, FN));
       if (v < 0) v = 1E-15;
       fo[(size_t)(NT - 1) * P] = v;
       fo[0] = v;

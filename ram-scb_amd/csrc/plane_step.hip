@@ -28,21 +28,6 @@
 
 namespace ramgpu {
 
-// x formed here, in program order: without it the compiler sinks a row's
-// last operations below the next rows and holds their operands instead.
-__device__ __forceinline__ double row_done(double x) {
-  asm volatile("" : "+v"(x));
-  return x;
-}
-
-// A uniform pointer, hidden from the optimiser: what a phase reads through it
-// is read in the phase, not kept in scalar registers from the kernel's start.
-template <class P>
-__device__ __forceinline__ P fresh_uniform(P p) {
-  asm volatile("" : "+s"(p));
-  return p;
-}
-
 // LDS of the kernel (step_lds_doubles)
 struct StepLds {
   double *F;   // NPAP rows of NE+3 energy-stencil positions F(0) .. F(NE+2)
@@ -57,12 +42,6 @@ struct StepLds {
 };
 // slots of red per wave
 constexpr int kStepSums = 7, kStepXSums = kSumSlots;
-struct Yes {
-  static constexpr bool value = true;
-};
-struct No {
-  static constexpr bool value = false;
-};
 
 // Per-row terms of the Coulomb operators and the line solves: XNE(L) =
 // NECR(I,J)*BANE(L) with the bounce factor BANE(L) = (1-FNIS/2/FNHS)/(1-MU^2)

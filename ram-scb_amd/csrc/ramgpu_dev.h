@@ -136,6 +136,7 @@ struct Tab {
   int plane_chunks;
   int step_cells, step_apart;  // step_wave_cells, step_edges_apart of k_plane_step's shape
   int stepx_apart;             // step_edges_apart of SEQ_STEPX's
+  int r_rows, p_rows;          // rows of k_r_rows and k_p_rows; 0: k_r, k_p (lines too long)
   // state
   double *f2;
   double *partials;  // [slot][s][maxblk]
@@ -205,12 +206,37 @@ inline __host__ __device__ bool out_of_place(const Launch &L) { return L.dsl != 
 
 // block counts of the kernels, per (problem, species)
 template <class T>
-inline __host__ __device__ int blocks_r(const T &t) {
+inline __host__ __device__ int blocks_line_r(const T &t) {  // one thread per line: k_r, k_r_bwd
   return (t.nt * t.ne * t.npa + kLineThreads - 1) / kLineThreads;
 }
 template <class T>
-inline __host__ __device__ int blocks_p(const T &t) {
+inline __host__ __device__ int blocks_line_p(const T &t) {  // k_p, k_p_bwd
   return ((t.nr - 1) * t.ne * t.npa + kLineThreads - 1) / kLineThreads;
+}
+// The sweeps with a line's cells in registers (k_r_rows, k_p_rows): 64 lines
+// of one J or I per block, line_chunks waves of `rows` cells.
+inline __host__ __device__ int line_chunks(int n, int rows) { return (n + rows - 1) / rows; }
+inline __host__ __device__ size_t line_lds_bytes(int chunks, int rows) {
+  return (size_t)((4 * chunks + 2) * 64 + 16 + 6 * chunks * rows) * sizeof(double);
+}
+constexpr int kLineMaxChunks = 16;
+// waves per SIMD that the registers leave room for, by rows
+constexpr int line_simd_waves(int rows) { return rows <= 2 ? 8 : (rows <= 6 ? 5 : 4); }
+template <class T>
+inline __host__ __device__ int blocks_r(const T &t) {
+  return t.r_rows ? t.nt * ((t.ne * t.npa + 63) / 64) : blocks_line_r(t);
+}
+template <class T>
+inline __host__ __device__ int blocks_p(const T &t) {
+  return t.p_rows ? (t.nr - 1) * ((t.ne * t.npa + 63) / 64) : blocks_line_p(t);
+}
+// out of place DRIFTP also copies the unswept I=1 rows
+template <class T>
+inline __host__ __device__ int blocks_p_copy(const T &t, bool chunks = true) {
+  const int P = t.ne * t.npa;
+  if (!t.p_rows || !chunks) return ((t.nr - 1) * P + t.nt * P + kLineThreads - 1) / kLineThreads;
+  const int threads = 64 * line_chunks(t.nt, t.p_rows);
+  return blocks_p(t) + (t.nt * P + threads - 1) / threads;
 }
 template <class T>
 inline __host__ __device__ int blocks_kl(const T &t) { return (t.nr - 1) * t.nt; }

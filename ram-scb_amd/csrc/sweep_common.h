@@ -20,6 +20,14 @@ static constexpr double kRE = 6.371E6;      // src/ModRamConst.f90:14
 #define GEO2(A, I, J) (A)[((I)-1) + (size_t)(t.nr + 1) * ((J)-1)]
 #define MGNP(I, J) t.mgnp[((I)-1) + (size_t)t.nr * ((J)-1)]
 
+// a choice made at compile time, passed to a generic lambda
+struct Yes {
+  static constexpr bool value = true;
+};
+struct No {
+  static constexpr bool value = false;
+};
+
 // n/d for 0 <= n < 2^22, d >= 1, from rd = RN_float(1/d): the float
 // quotient is within one of the true one, and one remainder test fixes it.
 __device__ __forceinline__ int fast_div(int n, int d, float rd) {
@@ -192,6 +200,29 @@ __device__ __forceinline__ double4 ld_d4(gptr<const double> p, size_t n) {
 __device__ __forceinline__ double2 ld_d2(gptr<const double> p, size_t n) {
   const gptr<const double> q = p + 2 * n;
   return make_double2(q[0], q[1]);
+}
+
+// x formed here, in program order: without it the compiler sinks a row's
+// last operations below the next rows and holds their operands instead.
+__device__ __forceinline__ double row_done(double x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
+// A uniform pointer, hidden from the optimiser: what a phase reads through it
+// is read in the phase, not kept in scalar registers from the kernel's start.
+template <class P>
+__device__ __forceinline__ P fresh_uniform(P p) {
+  asm volatile("" : "+s"(p));
+  return p;
+}
+
+// Uniform values all in scalar registers here: descriptor fields named in one
+// call are loaded together, in one memory round trip, instead of one after
+// the other as the code reaches them.
+template <class... T>
+__device__ __forceinline__ void fetched(T... x) {
+  (([](auto v) __attribute__((always_inline)) { asm volatile("" ::"s"(v)); })(x), ...);
 }
 
 // x, hidden from the optimiser: row indices derived from it are formed

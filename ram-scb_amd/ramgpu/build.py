@@ -19,7 +19,7 @@ INCLUDE = REPO / "include"
 LIB = PKG / "libramgpu.so"
 
 HIP_SOURCES = ["kernels.hip", "api.hip", "batch.hip", "adjoint.hip", "adjoint_api.hip", "moments.hip",
-               "coulomb.hip", "pitch.hip", "bounce.hip", "hostio.hip"]
+               "coulomb.hip", "pitch.hip", "bounce.hip", "hostio.hip", "line_sweep.hip"]
 # sources compiled once per part: (source, macro, parts)
 HIP_PARTS = [("plane_step.hip", "STEP_PART", 5)]
 
