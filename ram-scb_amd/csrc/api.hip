@@ -186,7 +186,7 @@ bool takes_wave(const ramgpu_ctx *c) {
 // terms, then WAVELO's factors (one (S,I,J,K) per thread) when a species
 // takes it.
 int coef_units(const ramgpu_ctx *c, int threads) {
-  int n = (c->nr * c->nt + threads - 1) / threads;
+  int n = (c->nr * c->nt + kCoefCells - 1) / kCoefCells;
   if (takes_wave(c)) n += (int)(((long long)c->ns * c->nr * c->nt * c->ne + threads - 1) / threads);
   return n;
 }
@@ -246,7 +246,7 @@ int prepare(ramgpu_ctx *c) {
     if (stage_q1) lds += q1b;
     const Launch lc = launch_of(c, 0, 1, coef_units(c, kFinalizeThreads));
     const Launch lf = launch_of(c, 0, c->fin_mask >= 0 ? c->ns : 0, 1);
-    const Launch lg = launch_of(c, 0, c->ns, 1);
+    const Launch lg = launch_of(c, 0, c->ns, ghost_blocks(c->t));
     hipLaunchKernelGGL(k_step_head, dim3(lc.nv + lf.nv + lg.nv), dim3(kFinalizeThreads), lds, c->stream, lc,
                        c->step_kp, c->step_bs, lf, c->fin_mask, c->fin_mode, lg, nvt, stage_q1);
     c->fin_mask = -1;
@@ -259,7 +259,7 @@ int prepare(ramgpu_ctx *c) {
   }
   if (c->ghost_dirty) {
     tbeg(c, RAMGPU_KERNEL_PREPARE);
-    const Launch l = launch_of(c, 0, c->ns, 1);
+    const Launch l = launch_of(c, 0, c->ns, ghost_blocks(c->t));
     hipLaunchKernelGGL(k_ghost, dim3(l.nv), dim3(1024), (size_t)4 * c->nt * sizeof(double), c->stream, l);
     tend(c);
     if ((rc = launch_check("k_ghost"))) return rc;

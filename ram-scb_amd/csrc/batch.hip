@@ -98,6 +98,7 @@ int batch_alloc(ramgpu_batch *b, void **p, size_t bytes) {
 int blocks_of(const ramgpu_batch *b, int kind, const ramgpu_ctx *c) {
   switch (kind) {
     case BK_COEFIJ: return coef_units(c, 256);
+    case BK_GHOST: return ghost_blocks(c->t);
     case BK_R: return blocks_r(c->t);
     case BK_P: return b->chunks ? blocks_p(c->t) : blocks_line_p(c->t);
     case BK_PLANE: return blocks_kl(c->t);

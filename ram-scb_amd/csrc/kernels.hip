@@ -156,14 +156,14 @@ __device__ __forceinline__ double vs_vt(double avs, double lz, double phi) {
 // (AVS*(LZ*RE)^2)*sin(PHI) is the product vs_vt forms.  bs, when given, is
 // the step's boundary-flux scales, copied to the descriptor's.
 // (LZ*RE)^2 [NR+1] and sin(PHI) [NT] into svt, by the block
-__device__ inline void stage_vt_factors(const Tab &t, double *svt) {
+__device__ inline void stage_vt_factors(CTab &t, double *svt) {
   const int NR1 = t.nr + 1;
   for (int x = threadIdx.x; x < NR1 + t.nt; x += blockDim.x) {
     if (x < NR1) {
-      const double lre = t.lz[x] * kRE;
+      const double lre = as_global(t.lz)[x] * kRE;
       svt[x] = lre * lre;
     } else {
-      svt[x] = sin(t.phi[x - NR1] - 0.0);
+      svt[x] = sin(as_global(t.phi)[x - NR1] - 0.0);
     }
   }
   __syncthreads();
@@ -176,78 +176,87 @@ __device__ inline void stage_vt_factors(const Tab &t, double *svt) {
 // BNES(I+1,J), its reciprocal, outsideMGNP(I,J)} (src/ModRamDrift.f90:
 // 118-127) and rsi = {RLZ+MDR/2, its reciprocal}; one definition for the
 // table and for the ghost carry, which forms the face-NR row itself
-__device__ __forceinline__ double4 radial_rij(const Tab &t, int i, int j, const double *kp, double avs,
-                                              const double *svt) {
+__device__ __forceinline__ double4 radial_rij(CTab &t, int i, int j, const double *kp, double avs, const double *svt) {
   const int I = i + 1, J = j + 1, NT = t.nt;
   const double dts = t.dts, mdr = t.mdr, dphi = t.dphi;
-  const double rlz = t.rlz[i];
+  const gptr<const double> bnes = as_global(t.bnes), eip = as_global(t.eip);
+  const double rlz = as_global(t.rlz)[i];
   const int J0 = (J == 1) ? NT - 1 : J - 1;
   const int J1 = (J == NT) ? 2 : J + 1;
   const double vr = dts / mdr / (rlz + 0.5 * mdr) / 2.0 / dphi;  // :67
-  const double bsum = GEO2(t.bnes, I, J) + GEO2(t.bnes, I + 1, J);
+  const double bsum = GEO2(bnes, I, J) + GEO2(bnes, I + 1, J);
   const double dv = VTV(I, J0) + VTV(I + 1, J0) - VTV(I, J1) - VTV(I + 1, J1);
-  const double cr = vr * dv / bsum + (GEO2(t.eip, I, J) + GEO2(t.eip, I + 1, J)) / bsum * dts / mdr;
-  return make_double4(cr, bsum, 1.0 / bsum, (double)MGNP(I, J));
+  const double cr = vr * dv / bsum + (GEO2(eip, I, J) + GEO2(eip, I + 1, J)) / bsum * dts / mdr;
+  return make_double4(cr, bsum, 1.0 / bsum, (double)as_global(t.mgnp)[i + (size_t)t.nr * j]);
 }
-__device__ __forceinline__ double2 radial_rsi(const Tab &t, int i) {
-  const double rs = t.rlz[i] + 0.5 * t.mdr;
+__device__ __forceinline__ double2 radial_rsi(CTab &t, int i) {
+  const double rs = as_global(t.rlz)[i] + 0.5 * t.mdr;
   return make_double2(rs, 1.0 / rs);
 }
 
+// The (I,J) terms go kCoefCells to a block, one per thread: a cell's chain of
+// quotients is the launch's time, so the cells are spread over the CUs, and
+// the descriptor's fields and then the geometry come in one trip each (10.5 us
+// as they were reached, 500 cells to a block).
 __device__ inline void coef_ij_unit(const Launch &L, int vb, const double *kp, const double *bs, double avs,
                                     double *svt) {
   {
-    const Unit u = unit_of(L, vb);
-    const Tab &t = *u.t;
-    const int nbc = (t.nr * t.nt + blockDim.x - 1) / blockDim.x;  // units of the (I,J) terms
+    const CUnit u = const_unit(L, vb);
+    CTab &t = *u.t;
+    fetched(t.ns, t.nr, t.nt, t.ne, t.bnes, t.eip, t.eir, t.dbdt, t.vt, t.mgnp, t.rlz, t.lz, t.phi, t.dts, t.mdr, t.dphi,
+            t.rij, t.pij, t.kij, t.rsi, t.rrlz);
+    const int nbc = (t.nr * t.nt + kCoefCells - 1) / kCoefCells;  // units of the (I,J) terms
     if (u.b >= nbc) {
       // WAVELO's factors at the step's Kp, one (S,I,J,K) per thread, K >= 2,
       // I >= 2, for the species that take it (src/ModRamWPI.f90:596-630)
+      const Tab &tg = *(const Tab *)(unsigned long long)u.t;
       const int m = (u.b - nbc) * blockDim.x + threadIdx.x;
       const int NE = t.ne, NT = t.nt;
       if (m < t.ns * t.nr * NT * NE) {
         const int k = m % NE, r = m / NE, j = r % NT, r2 = r / NT, i = r2 % t.nr, s = r2 / t.nr;
-        if (t.wpi[s] && i >= 1 && k >= 1) t.wavef[m] = wave_factor(t, s, i, j, k, kp ? *kp : *t.kpnow);
+        if (tg.wpi[s] && i >= 1 && k >= 1) t.wavef[m] = wave_factor(tg, s, i, j, k, kp ? *kp : *t.kpnow);
       }
       return;
     }
     if (bs && u.b == 0)
       for (int s = threadIdx.x; s < t.ns; s += blockDim.x) t.bscale[s] = bs[s];
     if (kp && u.b == 0 && threadIdx.x == 0) *t.kpnow = *kp;  // WAVELO's KP of the step
+    const int n = u.b * kCoefCells + threadIdx.x;
+    const bool on = threadIdx.x < kCoefCells && n < t.nr * t.nt;
+    const int i = on ? n / t.nt : 0, j = on ? n - i * t.nt : 0;
+    const int I = i + 1, J = j + 1;
+    const int NT = t.nt;
+    const double dts = t.dts, mdr = t.mdr, dphi = t.dphi;
+    const gptr<const double> gb = as_global(t.bnes), gr = as_global(t.eir), gp = as_global(t.eip), gd = as_global(t.dbdt);
+    const int J1 = (J == NT) ? 2 : J + 1;
+    // the cell's geometry, in flight with the VT factors
+    const double rlz = as_global(t.rlz)[i];
+    const double bij = GEO2(gb, I, J), bij1 = GEO2(gb, I, J1);
+    const double erij = GEO2(gr, I, J), erij1 = GEO2(gr, I, J1), epij = GEO2(gp, I, J), dbij = GEO2(gd, I, J);
+    const double mg = (double)as_global(t.mgnp)[i + (size_t)t.nr * j];
     if (kp) stage_vt_factors(t, svt);
-    const int n = u.b * blockDim.x + threadIdx.x;
-    if (n < t.nr * t.nt) {
-      const int i = n / t.nt, j = n % t.nt;
-      const int I = i + 1, J = j + 1;
-      const int NT = t.nt;
-      const double dts = t.dts, mdr = t.mdr, dphi = t.dphi;
-      const double rlz = t.rlz[i];
+    if (on) {
       const size_t ij = (size_t)i * NT + j;
-      const double mg = (double)MGNP(I, J);
       if (j == 0) {
-        t.rrlz[i] = 1.0 / rlz;
+        as_global(t.rrlz)[i] = 1.0 / rlz;
         t.rsi[i] = radial_rsi(t, i);
       }
       t.rij[ij] = radial_rij(t, i, j, kp, avs, svt);
       double pa = 0.0, pce = 0.0, pbs = 1.0;
       double drd1 = 0.0, dpd1 = 0.0, drm1 = 0.0, dpm1 = 0.0, db2 = 0.0;
-      const double bij = GEO2(t.bnes, I, J);
       if (I >= 2) {
         if (J >= 2) {
-          const int J1 = (J == NT) ? 2 : J + 1;
           const double p1 = dts / dphi / 2.0 / mdr / rlz;  // :68
           pa = (VTV(I + 1, J) + VTV(I + 1, J1) - VTV(I - 1, J) - VTV(I - 1, J1)) * p1;
-          pce = (GEO2(t.eir, I, J1) + GEO2(t.eir, I, J)) / rlz * dts / dphi;
-          pbs = GEO2(t.bnes, I, J) + GEO2(t.bnes, I, J1);
+          pce = (erij1 + erij) / rlz * dts / dphi;
+          pbs = bij + bij1;
         }
         const int J0 = (J == 1) ? NT - 1 : J - 1;
-        const int J2 = (J == NT) ? 2 : J + 1;
-        drd1 = (GEO2(t.eip, I, J) * rlz - (VTV(I, J2) - VTV(I, J0)) / 2.0 / dphi) / bij;
-        dpd1 = kOME * rlz + ((VTV(I + 1, J) - VTV(I - 1, J)) / 2.0 / mdr - GEO2(t.eir, I, J)) / bij;
-        // DRIFTMU's DRM1/DPM1 (:415-416) are the same expressions as DRD1/DPD1
-        drm1 = (GEO2(t.eip, I, J) * rlz - (VTV(I, J2) - VTV(I, J0)) / 2.0 / dphi) / bij;
-        dpm1 = kOME * rlz + ((VTV(I + 1, J) - VTV(I - 1, J)) / 2.0 / mdr - GEO2(t.eir, I, J)) / bij;
-        db2 = GEO2(t.dbdt, I, J) / 2.0 / bij * rlz;  // :431
+        drd1 = (epij * rlz - (VTV(I, J1) - VTV(I, J0)) / 2.0 / dphi) / bij;
+        dpd1 = kOME * rlz + ((VTV(I + 1, J) - VTV(I - 1, J)) / 2.0 / mdr - erij) / bij;
+        drm1 = drd1;  // DRIFTMU's DRM1/DPM1 (:415-416) are the same expressions
+        dpm1 = dpd1;
+        db2 = dbij / 2.0 / bij * rlz;  // :431
       }
       t.pij[ij] = make_double4(pa, pce, pbs, 1.0 / pbs);
       double *k8 = t.kij + ij * 8;
@@ -407,28 +416,33 @@ __global__ void k_coef(Launch L) {
 // order, or 0 when no inflow line came before.  Whether a line is inflow
 // depends on geometry, fields and grid only, so the carry is precomputed:
 // carry[s][p] is the index p'*NT+(J'-1) of the last inflow line before plane
-// p=(K-1)*NPA+(L-1), or -1.  One block per (problem, species): each thread
-// finds the top inflow J of its planes (four J per memory round trip) into
-// LDS, then a block-wide exclusive max-scan over the planes in order (wave
-// shuffles, then the waves' totals).
-// One (problem, species) of the ghost carry.  The face-NR terms it tests
-// (rij(NR-1,.), rsi(NR-1)) are formed here with the table's own code, so the
-// carry does not wait for k_coef_ij; rrow holds them (4*NT doubles), svt the
-// VT factors when kp is given.  q1s (NPA*NT doubles, or null): LDS for the
-// face-NR row of q1, loaded in one pass so that the search for each line's
-// last inflow J reads no global memory.
+// p=(K-1)*NPA+(L-1), or -1.  A block takes kGhostPlanes planes of a species:
+// one half of its threads find the top inflow J of these (four J per step),
+// the other half of as many planes before them, whose maximum is the carry
+// into the first (the index of an inflow line grows with p, so the last one is
+// the maximum; while it finds none the block goes further back).  Then an
+// exclusive max-scan over the planes in order (wave shuffles, then the waves'
+// totals).  One block for a species' 2520 planes made three searches a thread
+// on one CU (9.1 us).
+// The face-NR terms it tests (rij(NR-1,.), rsi(NR-1)) are formed here with the
+// table's own code, so the carry does not wait for k_coef_ij; rrow holds them
+// (4*NT doubles), svt the VT factors when kp is given.  q1s (NPA*NT doubles, or
+// null): LDS for the face-NR row of q1, loaded in one pass so that the search
+// for each line's last inflow J reads no global memory.
 __device__ inline void ghost_unit(const Launch &L, int vb, const double *kp, double avs, double *svt, double *rrow,
-                                  int *s_last, int *s_wave, double *q1s = nullptr) {
-  const Unit u = unit_of(L, vb);
-  const Tab &t = *u.t;
+                                  int *s_wave, double *q1s = nullptr) {
+  const CUnit u = const_unit(L, vb);
+  CTab &t = *u.t;
+  fetched(t.ns, t.nr, t.nt, t.ne, t.npa, t.q1, t.p4, t.bnes, t.eip, t.vt, t.mgnp, t.rlz, t.lz, t.phi, t.carry, t.dts, t.mdr,
+          t.dphi);
   const int s = u.s, NR = t.nr, NT = t.nt, NPA = t.npa;
   const int P = t.ne * NPA, T = blockDim.x, tid = threadIdx.x;
-  if (kp) stage_vt_factors(t, svt);
   if (q1s)
     for (int x = tid; x < NPA * NT; x += T) {
       const int l = x / NT, j = x - l * NT;
-      q1s[x] = t.q1[((size_t)l * NR + NR - 1) * NT + j];
+      q1s[x] = as_global((const double *)t.q1)[((size_t)l * NR + NR - 1) * NT + j];
     }
+  if (kp) stage_vt_factors(t, svt);
   for (int j = tid; j < NT; j += T) {
     const double4 r = radial_rij(t, NR - 1, j, kp, avs, svt);
     rrow[4 * j] = r.x;
@@ -438,10 +452,10 @@ __device__ inline void ghost_unit(const Launch &L, int vb, const double *kp, dou
   }
   __syncthreads();
   const double2 rs = radial_rsi(t, NR - 1);
-  for (int p = tid; p < P; p += T) {
+  // the last inflow line of plane p, searched down from J=NT in groups of 4
+  auto last_inflow = [&](int p) {
     const int k = p / NPA, l = p - k * NPA;
-    const double p4k = t.p4[s * t.ne + k];
-    // the highest inflow J of the line, searched down from NT in groups of 4
+    const double p4k = as_global((const double *)t.p4)[s * t.ne + k];
     auto search = [&](auto q1) {
       int last = -1;
       for (int j0 = NT - 1; j0 >= 0 && last < 0; j0 -= 4) {
@@ -458,38 +472,42 @@ __device__ inline void ghost_unit(const Launch &L, int vb, const double *kp, dou
       }
       return last;
     };
-    s_last[p] = q1s ? search(q1s + (size_t)l * NT) : search(as_global(t.q1 + ((size_t)l * NR + NR - 1) * NT));
-  }
-  __syncthreads();
-  // planes [p0, p1) of this thread, in order
-  const int chunk = (P + T - 1) / T;
-  const int p0 = min(P, tid * chunk), p1 = min(P, p0 + chunk);
-  int v = -1;
-  for (int p = p0; p < p1; ++p) v = max(v, s_last[p]);
-  const int lane = tid & 63, w = tid >> 6;
+    return q1s ? search(q1s + (size_t)l * NT)
+               : search(as_global((const double *)t.q1 + ((size_t)l * NR + NR - 1) * NT));
+  };
+  const int p0 = u.b * kGhostPlanes, half = T >> 1;  // kGhostPlanes threads and as many
+  const int p = tid < half ? p0 + tid : p0 - 1 - (tid - half);
+  int v = (p >= 0 && p < P) ? last_inflow(p) : -1;
+  const int lane = tid & 63, w = tid >> 6, wh = half >> 6;
   for (int off = 1; off < 64; off <<= 1) {  // inclusive max-scan in the wave
     const int o = __shfl_up(v, off, 64);
     if (lane >= off) v = max(v, o);
   }
   if (lane == 63) s_wave[w] = v;
   __syncthreads();
+  int carry = -1;
+  for (int ww = wh; ww < 2 * wh; ++ww) carry = max(carry, s_wave[ww]);
   int run = __shfl_up(v, 1, 64);
   if (lane == 0) run = -1;
-  for (int ww = 0; ww < w; ++ww) run = max(run, s_wave[ww]);
-  // the index of an inflow line grows with p, so the last one is the maximum
-  for (int p = p0; p < p1; ++p) {
-    t.carry[(size_t)s * P + p] = run;
-    run = max(run, s_last[p]);
+  if (w < wh)
+    for (int ww = 0; ww < w; ++ww) run = max(run, s_wave[ww]);
+  for (int pe = p0 - half; carry < 0 && pe > 0; pe -= T) {  // planes before pe, a block's width at a time
+    int x = pe - 1 - tid >= 0 ? last_inflow(pe - 1 - tid) : -1;
+    for (int off = 32; off > 0; off >>= 1) x = max(x, __shfl_down(x, off, 64));
+    __syncthreads();  // s_wave is read
+    if (lane == 0) s_wave[w] = x;
+    __syncthreads();
+    for (int ww = 0; ww < 2 * wh; ++ww) carry = max(carry, s_wave[ww]);
   }
+  if (tid < half && p < P) t.carry[(size_t)s * P + p] = max(run, carry);
   __syncthreads();
 }
 #undef VTV
 
 __global__ void __launch_bounds__(1024) k_ghost(Launch L) {
   extern __shared__ double rrow[];  // 4*NT: ghost_rows_lds_bytes
-  __shared__ int s_last[kMaxPlaneCells];
-  __shared__ int s_wave[16];
-  for (int vb = blockIdx.x; vb < L.nv; vb += gridDim.x) ghost_unit(L, vb, nullptr, 0.0, nullptr, rrow, s_last, s_wave);
+  __shared__ int s_wave[kFinalizeThreads / 64];
+  for (int vb = blockIdx.x; vb < L.nv; vb += gridDim.x) ghost_unit(L, vb, nullptr, 0.0, nullptr, rrow, s_wave);
 }
 
 // ---------------------------------------------------------------------------
@@ -1279,95 +1297,81 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, 4) k_plane(Launch L, int rec
 // species that takes a line solve books every SUMRC that some species has:
 // FLCscatter has none of its own, so its loss goes to the next one.  One
 // block per (problem, species).
-constexpr int kFinNV = 2 + kSumSlots;  // the DtDriftE and DtDriftMu minima, then the SUMRC slot sums
-__device__ inline void finalize_unit(const Launch &L, int vb, int cflmask, int summode, double *red) {
-  constexpr int NV = kFinNV;
+//
+// What bounds it: latency alone.  A slot's sums are a wave's (two waves' when
+// eight slots are in use, sixteen's for one), by lane adds without LDS; with
+// every thread summing all slots the block reduction of sixteen values took
+// most of 14.0 us.  Now 5.1 (one species of 20x25x35x72), 3.6 for a DtDrift.
+constexpr int kFinRed = kFinalizeThreads / 64 + 2;  // the waves' sums, then the DtDriftE and DtDriftMu minima
+__device__ inline void finalize_unit(const Launch &L, int vb, int cflmask, int mode, double *red) {
   {
-    const Unit u = unit_of(L, vb);
-    const Tab &t = *u.t;
+    const CUnit u = const_unit(L, vb);
+    CTab &t = *u.t;
+    fetched(t.ns, t.nr, t.nt, t.ne, t.npa, t.maxblk, t.r_rows, t.coul, t.sum_any, t.fraccfl, t.dts, t.partials, t.energy,
+            t.lsx, t.cflmax, t.dtdrift, t.de, t.dmu);
     const int s = u.s, tid = threadIdx.x, T = blockDim.x;
+    const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), W = T >> 6;
     const int NE = t.ne, NPA = t.npa;
     const double a = t.fraccfl * t.dts;
-    unsigned long long *m = t.cflmax + (size_t)s * (2 + NE + NPA);
-    // every load of the block first: thread 0's scalars, the CFL maxima, the
-    // plane and radial blocks' partial sums
+    unsigned long long *const m = t.cflmax + (size_t)s * (2 + NE + NPA);
+    const gptr<const unsigned long long> gm = as_global((const unsigned long long *)m);
+    // thread 0's scalars
     double e0[4] = {0.0, 0.0, 0.0, 0.0}, lswae = 0.0, lscoe = 0.0, lscsc = 0.0;
     unsigned long long m01[2] = {0ull, 0ull};
-    int cex = 0, wpi = 0;
     const bool coul = t.coul != 0;
     const bool lines = t.pd_wpi[s] || t.pd_emic[s] || t.flc[s];
     const bool emic = lines && (t.sum_any & ANY_EMIC);
+    const int cex = lines ? t.sum_any & ANY_CEX : t.cex[s], wpi = lines ? t.sum_any & ANY_WPI : t.wpi[s];
     if (tid == 0) {
+      const gptr<const double> ge = as_global((const double *)t.energy) + s * 4, gl = as_global((const double *)t.lsx) + s * 3;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) e0[q] = t.energy[s * 4 + q];
-      lswae = t.lsx[s * 3];
-      lscoe = t.lsx[s * 3 + 1];
-      lscsc = t.lsx[s * 3 + 2];
-      m01[0] = m[0];
-      m01[1] = m[1];
-      cex = lines ? t.sum_any & ANY_CEX : t.cex[s];
-      wpi = lines ? t.sum_any & ANY_WPI : t.wpi[s];
+      for (int q = 0; q < 4; ++q) e0[q] = ge[q];
+      lswae = gl[0];
+      lscoe = gl[1];
+      lscsc = gl[2];
+      m01[0] = gm[0];
+      m01[1] = gm[1];
     }
-    double v[NV];
-    v[0] = 10000.0;
-    v[1] = 10000.0;
+    // the slots in use: 0..6 (and with the optional processes 8..13) from the
+    // plane blocks, 7 from the R blocks; a single SUMRC reads slot 0
+    const int nslot = mode == 0 ? 0 : mode == 1 ? 1 : 8 + (coul ? 4 : 0) + (emic ? 2 : 0);
+    const int per = nslot ? W / nslot : 0;  // waves of a slot
+    if (w < nslot * per) {
+      const int g = w / per, part = w - g * per;
+      const int id = (g >= kSumCoul && !coul) ? g + (kSumEmic - kSumCoul) : g;
+      const int n = id == kSumRadial ? blocks_r(t) : blocks_kl(t), st = 64 * per;
+      const gptr<const double> p = as_global((const double *)t.partials + ((size_t)id * t.ns + s) * t.maxblk);
+      double acc = 0.0;
+      for (int b0 = part * 64 + lane; b0 < n; b0 += 8 * st) {
+        double v[8];
 #pragma unroll
-    for (int q = 2; q < NV; ++q) v[q] = 0.0;
-    if (cflmask & 4)
-      for (int k = tid; k < NE; k += T) {
-        const double c = __longlong_as_double((long long)m[2 + k]);
-        if (c > 0) v[0] = fmin(v[0], a * t.de[k] / c);
-      }
-    if (cflmask & 8)
-      for (int l = 1 + tid; l < NPA; l += T) {
-        const double c = __longlong_as_double((long long)m[2 + NE + l]);
-        if (c > 0) v[1] = fmin(v[1], a * t.dmu[l] / c);
-      }
-    const int mode = summode;
-    if (mode != 0) {
-      // slots 0..6 (and with the optional processes 8..13) from the plane
-      // blocks, slot 7 from the R blocks; a single SUMRC reads slot 0
-      const int nbk = blocks_kl(t), nbr = blocks_r(t);
-      const double *pp = t.partials + (size_t)s * t.maxblk;
-      const size_t slot = (size_t)t.ns * t.maxblk;
-      const int nslot = (mode == 1) ? 1 : kSumRadial;
-      for (int b = tid; b < nbk; b += T)
-        for (int sl = 0; sl < nslot; ++sl) v[2 + sl] += pp[sl * slot + b];
-      if (mode == 2) {
-        for (int b = tid; b < nbr; b += T) v[2 + kSumRadial] += pp[kSumRadial * slot + b];
-        if (coul)
-          for (int b = tid; b < nbk; b += T)
+        for (int q = 0; q < 8; ++q) v[q] = (b0 + q * st < n) ? p[b0 + q * st] : 0.0;
 #pragma unroll
-            for (int sl = kSumCoul; sl < kSumCoul + 4; ++sl) v[2 + sl] += pp[sl * slot + b];
-        if (emic)
-          for (int b = tid; b < nbk; b += T) {
-            v[2 + kSumEmic] += pp[kSumEmic * slot + b];
-            v[3 + kSumEmic] += pp[(kSumEmic + 1) * slot + b];
-          }
+        for (int q = 0; q < 8; ++q) acc += v[q];
       }
+      acc = wave_sum(acc);
+      if (lane == 63) red[w] = acc;
     }
-    // one block reduction (fixed order): minima of v[0..1], sums of the rest
-    for (int off = 32; off > 0; off >>= 1) {
-      v[0] = fmin(v[0], __shfl_down(v[0], off, 64));
-      v[1] = fmin(v[1], __shfl_down(v[1], off, 64));
-#pragma unroll
-      for (int q = 2; q < NV; ++q) v[q] += __shfl_down(v[q], off, 64);
+    if (((cflmask & 4) && w == W - 2) || ((cflmask & 8) && w == W - 1)) {
+      const bool mu = w == W - 1;
+      const gptr<const unsigned long long> c0 = gm + (mu ? 2 + NE : 2);
+      const gptr<const double> d0 = as_global(mu ? (const double *)t.dmu : (const double *)t.de);
+      double v = 10000.0;
+      for (int x = (mu ? 1 : 0) + lane; x < (mu ? NPA : NE); x += 64) {
+        const double c = __longlong_as_double((long long)c0[x]);
+        if (c > 0) v = fmin(v, a * d0[x] / c);
+      }
+      for (int off = 32; off > 0; off >>= 1) v = fmin(v, __shfl_down(v, off, 64));
+      if (lane == 0) red[W + (mu ? 1 : 0)] = v;
     }
-    const int lane = tid & 63, w = tid >> 6, nw = (T + 63) >> 6;
-    if (lane == 0)
-#pragma unroll
-      for (int q = 0; q < NV; ++q) red[w * NV + q] = v[q];
     __syncthreads();
     if (tid == 0) {
-      double r[NV];
-#pragma unroll
-      for (int q = 0; q < NV; ++q) r[q] = red[q];
-      for (int ww = 1; ww < nw; ++ww) {
-        r[0] = fmin(r[0], red[ww * NV]);
-        r[1] = fmin(r[1], red[ww * NV + 1]);
-#pragma unroll
-        for (int q = 2; q < NV; ++q) r[q] += red[ww * NV + q];
-      }
+      auto sum = [&](int id) {
+        const int g = (id >= kSumCoul && !coul) ? id - (kSumEmic - kSumCoul) : id;
+        double v = red[g * per];
+        for (int q = 1; q < per; ++q) v += red[g * per + q];
+        return v;
+      };
       if (cflmask & 1) {
         const double c = __longlong_as_double((long long)m01[0]);
         t.dtdrift[s * 4 + 0] = (c > 0) ? fmin(100000.0, a / c) : 100000.0;
@@ -1376,10 +1380,22 @@ __device__ inline void finalize_unit(const Launch &L, int vb, int cflmask, int s
         const double c = __longlong_as_double((long long)m01[1]);
         t.dtdrift[s * 4 + 1] = (c > 0) ? fmin(100000.0, a / c) : 100000.0;
       }
-      if (cflmask & 4) t.dtdrift[s * 4 + 2] = r[0];
-      if (cflmask & 8) t.dtdrift[s * 4 + 3] = r[1];
+      if (cflmask & 4) t.dtdrift[s * 4 + 2] = red[W];
+      if (cflmask & 8) t.dtdrift[s * 4 + 3] = red[W + 1];
       if (mode != 0) {
-        const double *S = r + 2;
+        double S[kSumSlots];
+        S[0] = sum(0);
+        if (mode == 2) {
+#pragma unroll
+          for (int q = 1; q < kSumCoul; ++q) S[q] = sum(q);
+          if (coul)
+#pragma unroll
+            for (int q = kSumCoul; q < kSumEmic; ++q) S[q] = sum(q);
+          if (emic) {
+            S[kSumEmic] = sum(kSumEmic);
+            S[kSumEmic + 1] = sum(kSumEmic + 1);
+          }
+        }
         double *e = t.energy + s * 4;
         const double old = e0[0];
         if (mode == 1) {
@@ -1456,12 +1472,13 @@ __device__ inline void finalize_unit(const Launch &L, int vb, int cflmask, int s
 }
 
 __global__ void __launch_bounds__(kFinalizeThreads) k_finalize(Launch L, int cflmask, int summode) {
-  __shared__ double red[(kFinalizeThreads / 64) * kFinNV];
+  __shared__ double red[kFinRed];
   for (int vb = blockIdx.x; vb < L.nv; vb += gridDim.x) finalize_unit(L, vb, cflmask, summode, red);
 }
 
 // The head of a step in one launch (each part on its own is a latency-bound
-// launch of a few microseconds): blocks below Lc.nv form the step's
+// launch of a few microseconds; 14.0 -> 6.3 us for three species of
+// 9x13x11x17 with the parts as they are now): blocks below Lc.nv form the step's
 // Courant-number terms (k_coef_ij), the next Lf.nv finish the previous step
 // of a schedule (k_finalize, one block per species; none when Lf.nv = 0),
 // the last Lg.nv form the step's ghost carry (k_ghost).  The parts touch
@@ -1473,8 +1490,7 @@ __global__ void __launch_bounds__(kFinalizeThreads) k_step_head(Launch Lc, const
                                                                 Launch Lf, int cflmask, int summode, Launch Lg,
                                                                 int nvt, int stage_q1) {
   extern __shared__ double dyn[];
-  __shared__ double red[(kFinalizeThreads / 64) * kFinNV];
-  __shared__ int s_last[kMaxPlaneCells];
+  __shared__ double red[kFinRed];
   __shared__ int s_wave[kFinalizeThreads / 64];
   const double avs = kp ? vs_avs(*kp) : 0.0;
   int b = blockIdx.x;
@@ -1484,7 +1500,7 @@ __global__ void __launch_bounds__(kFinalizeThreads) k_step_head(Launch Lc, const
     finalize_unit(Lf, b, cflmask, summode, red);
   } else {
     const int nt = Lg.tabs[0].nt;
-    ghost_unit(Lg, b - Lf.nv, kp, avs, dyn, dyn + nvt, s_last, s_wave, stage_q1 ? dyn + nvt + 4 * nt : nullptr);
+    ghost_unit(Lg, b - Lf.nv, kp, avs, dyn, dyn + nvt, s_wave, stage_q1 ? dyn + nvt + 4 * nt : nullptr);
   }
 }
 

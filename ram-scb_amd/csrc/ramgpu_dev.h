@@ -38,7 +38,9 @@ constexpr int kSumEmic = 12;
 enum SumAny { ANY_WPI = 1, ANY_EMIC = 2, ANY_CEX = 4 };
 // k_finalize's summode: 0 none, 1 one SUMRC (slot 0), 2 the fused step's chain
 constexpr int kMuSpread = 4;           // LDS slots per pitch-angle row of DRIFTMU's CFL maximum (by K mod 4)
-constexpr int kFinalizeThreads = 1024;  // one block per (problem, species) of k_finalize (and of k_ghost)
+constexpr int kFinalizeThreads = 1024;  // one block per (problem, species) of k_finalize; also k_ghost's block
+constexpr int kGhostPlanes = kFinalizeThreads / 2;  // (K,L) planes per block of k_ghost
+constexpr int kCoefCells = 128;         // (I,J) cells per block of k_coef_ij
 
 // packed per-(I,J) terms of the plane sweeps, kij[(i*NT+j)*8 + ..]
 enum KijField { KIJ_DRD1, KIJ_DPD1, KIJ_BIJ, KIJ_RBIJ, KIJ_DRM1, KIJ_DPM1, KIJ_DB2, KIJ_MG };
@@ -237,6 +239,11 @@ inline __host__ __device__ int blocks_p_copy(const T &t, bool chunks = true) {
   if (!t.p_rows || !chunks) return ((t.nr - 1) * P + t.nt * P + kLineThreads - 1) / kLineThreads;
   const int threads = 64 * line_chunks(t.nt, t.p_rows);
   return blocks_p(t) + (t.nt * P + threads - 1) / threads;
+}
+// blocks of k_ghost, per species
+template <class T>
+inline __host__ __device__ int ghost_blocks(const T &t) {
+  return (t.ne * t.npa + kGhostPlanes - 1) / kGhostPlanes;
 }
 template <class T>
 inline __host__ __device__ int blocks_kl(const T &t) { return (t.nr - 1) * t.nt; }
