@@ -24,7 +24,7 @@ template <int BT>
 void set_bwd_lds_limit_t(size_t limit) {
   const void *fns[] = {(const void *)k_plane_bwd<SEQ_E, BT>,   (const void *)k_plane_bwd<SEQ_MU, BT>,
                        (const void *)k_plane_bwd<SEQ_CEX, BT>, (const void *)k_plane_bwd<SEQ_ATM, BT>,
-                       (const void *)k_plane_bwd<SEQ_LOSS, BT>, (const void *)k_plane_bwd<SEQ_STEP, BT>};
+                       (const void *)k_plane_bwd<SEQ_LOSS, BT>};
   for (const void *f : fns) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)limit);
 }
 
@@ -42,12 +42,49 @@ void launch_plane_bwd_t(int seq, dim3 grid, size_t lds, hipStream_t st, const La
     case SEQ_MU: hipLaunchKernelGGL((k_plane_bwd<SEQ_MU, BT>), grid, blk, lds, st, L, x, adj); break;
     case SEQ_CEX: hipLaunchKernelGGL((k_plane_bwd<SEQ_CEX, BT>), grid, blk, lds, st, L, x, adj); break;
     case SEQ_ATM: hipLaunchKernelGGL((k_plane_bwd<SEQ_ATM, BT>), grid, blk, lds, st, L, x, adj); break;
-    case SEQ_LOSS: hipLaunchKernelGGL((k_plane_bwd<SEQ_LOSS, BT>), grid, blk, lds, st, L, x, adj); break;
-    default: hipLaunchKernelGGL((k_plane_bwd<SEQ_STEP, BT>), grid, blk, lds, st, L, x, adj); break;
+    default: hipLaunchKernelGGL((k_plane_bwd<SEQ_LOSS, BT>), grid, blk, lds, st, L, x, adj); break;
+  }
+}
+
+// Rows per thread the step's plane adjoint is built for.
+#define ADJ_ROWS(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12)
+
+// Rows per thread of the step's plane adjoint: step_shape's rule with its own
+// threads and LDS (MI355X, us by rows: 475 planes of 35x72 4: 52, 5: 59, 6: 44,
+// 8: 54, 9: 53, 12: 51).
+StepShape adj_shape(int ne, int npa, long planes, int ncu, size_t lds_cu) {
+  StepShape best{0, 0};
+  double bcost = 0;
+#define TRY(r)                                                                                           \
+  {                                                                                                      \
+    const int threads = adj_threads(ne, npa, r), waves = threads / 64, simd = (waves + 3) / 4;           \
+    const size_t lds = adj_lds_bytes(ne, npa, r);                                                        \
+    if (npa % r != 1 && threads <= kPlaneMaxThreads && lds <= lds_cu && kStepSimdWaves / simd > 0) {     \
+      const long res = std::min<long>({kStepSimdWaves / simd, (long)(lds_cu / lds), (planes + ncu - 1) / ncu}); \
+      const double cost = 0.5 * (waves / 4.0 + simd) * (r + 4) * std::pow(16.0 / (res * waves), 0.4);    \
+      if (best.threads == 0 || cost < bcost) best = {threads, r}, bcost = cost;                          \
+    }                                                                                                    \
+  }
+  ADJ_ROWS(TRY)
+#undef TRY
+  return best;
+}
+
+void launch_plane_adj(StepShape sh, dim3 grid, size_t lds, hipStream_t st, const Launch &L, const double *x, double *adj) {
+  const dim3 blk(sh.threads);
+  switch (sh.rows) {
+#define ROWS(r) \
+  case r: hipLaunchKernelGGL((k_plane_adj<r>), grid, blk, lds, st, L, x, adj); break;
+    ADJ_ROWS(ROWS)
+#undef ROWS
   }
 }
 
 void set_plane_bwd_lds_limit(size_t limit) {
+#define ADJ_K(r) \
+  (void)hipFuncSetAttribute((const void *)k_plane_adj<r>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)limit);
+  ADJ_ROWS(ADJ_K)
+#undef ADJ_K
   set_bwd_lds_limit_t<kPlaneThreads>(limit);
   set_bwd_lds_limit_t<kPlaneMaxThreads>(limit);
 }
@@ -196,7 +233,10 @@ int bwd_plane(ramgpu_ctx *c, int seq, const double *x, double *adj, int s0, int 
   const Launch L = launch_of(c, s0, nsp, blocks_kl(c->t));
   const size_t lds = bwd_lds(c);
   tbeg(c, RAMGPU_KERNEL_PLANE_BWD);
-  launch_plane_bwd(seq, plane_bwd_threads(c->ne, c->npa), dim3(L.nv), lds, c->stream, L, x, adj);
+  if (seq == SEQ_STEP)
+    launch_plane_adj(c->adj, dim3(L.nv), adj_lds_bytes(c->ne, c->npa, c->adj.rows), c->stream, L, x, adj);
+  else
+    launch_plane_bwd(seq, plane_bwd_threads(c->ne, c->npa), dim3(L.nv), lds, c->stream, L, x, adj);
   tend(c);
   return launch_check("k_plane_bwd");
 }

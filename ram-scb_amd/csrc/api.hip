@@ -656,7 +656,8 @@ int ramgpu_create(ramgpu_ctx **out, int ns, int nr, int nt, int ne, int npa, int
   t.plane_chunks = plane_chunks_for(ne, npa, c->plane.threads);
   c->step = step_shape(ne, npa, (long)ns * (nr - 1) * nt, ncu, c->lds_limit, false);
   c->stepx = step_shape(ne, npa, (long)ns * (nr - 1) * nt, ncu, c->lds_limit, true);
-  if (c->step.threads == 0 || c->stepx.threads == 0)
+  c->adj = adj_shape(ne, npa, (long)ns * (nr - 1) * nt, ncu, c->lds_limit);
+  if (c->step.threads == 0 || c->stepx.threads == 0 || c->adj.threads == 0)
     return cleanup(fail(RAMGPU_EINVAL, "no plane kernel shape for %dx%d", ne, npa));
   t.step_cells = step_wave_cells(ne);
   t.step_apart = step_edges_apart(ne, npa, c->step.rows);

@@ -32,7 +32,8 @@ namespace {
 // plane out of place (with the copy lines / planes of the unswept I=1 rows),
 // one unit per member (misfit) and a whole-F2 copy per member
 enum BatchKind {
-  BK_SCHED, BK_COEFIJ, BK_GHOST, BK_R, BK_P, BK_PLANE, BK_FIN, BK_POOP, BK_PLOOP, BK_RB, BK_PB, BK_MEM, BK_COPY, BK_N
+  BK_SCHED, BK_COEFIJ, BK_GHOST, BK_R, BK_P, BK_PLANE, BK_FIN, BK_POOP, BK_PLOOP, BK_RB, BK_PB, BK_PLB, BK_MEM,
+  BK_COPY, BK_N
 };
 
 struct Plan {
@@ -101,7 +102,7 @@ int blocks_of(const ramgpu_batch *b, int kind, const ramgpu_ctx *c) {
     case BK_GHOST: return ghost_blocks(c->t);
     case BK_R: return blocks_r(c->t);
     case BK_P: return b->chunks ? blocks_p(c->t) : blocks_line_p(c->t);
-    case BK_PLANE: return blocks_kl(c->t);
+    case BK_PLANE: case BK_PLB: return blocks_kl(c->t);
     case BK_POOP: return blocks_p_copy(c->t, b->chunks);
     case BK_RB: return blocks_line_r(c->t);
     case BK_PB: return blocks_line_p(c->t);
@@ -119,13 +120,17 @@ int build_plan(ramgpu_batch *b, int kind) {
   std::vector<Job> jobs;
   std::vector<int> vmap;
   const bool plane = kind == BK_PLANE || kind == BK_PLOOP;
-  const bool grouped = plane || kind == BK_R || kind == BK_P || kind == BK_POOP;
+  const bool grouped = plane || kind == BK_PLB || kind == BK_R || kind == BK_P || kind == BK_POOP;
   std::vector<size_t> order(b->m.size());
   std::iota(order.begin(), order.end(), size_t(0));
   auto shape_of = [&](const ramgpu_ctx *c, size_t *lds) {
     if (plane) {
       *lds = step_lds_bytes(c->ne, c->npa, c->step.rows);
       return c->step;
+    }
+    if (kind == BK_PLB) {
+      *lds = adj_lds_bytes(c->ne, c->npa, c->adj.rows);
+      return c->adj;
     }
     const LineShape h = kind == BK_R ? r_shape(c) : p_shape(c, b->chunks);
     *lds = h.lds;
@@ -154,7 +159,7 @@ int build_plan(ramgpu_batch *b, int kind) {
       return fail(RAMGPU_EINVAL, "ensemble too large for the launch tables");
     const int j0 = (int)jobs.size();
     for (int s = 0; s < nsp; ++s) jobs.push_back(Job{(int)mi, s, (int)vmap.size(), nb});
-    if (kind == BK_PLANE) {
+    if (kind == BK_PLANE || kind == BK_PLB) {
       // the species of each run of 8 planes in turn: a plane's species land
       // on one XCD, whose L2 serves them the plane's tables (Launch::ilv)
       for (int g = 0; g < nb; g += 8)
@@ -386,15 +391,20 @@ void enq_taped_step(ramgpu_batch *b, int g, int dsl_out, bool bookkeeping = true
 }
 
 // adjoint of the step taped at group g: Tab::lam in place, Tab::bbar[step]
-void enq_step_bwd(ramgpu_batch *b, int g, int step, size_t bwd_lds, int bwd_threads) {
+void enq_step_bwd(ramgpu_batch *b, int g, int step) {
   hipStream_t st = b->stream;
   Launch L = slot_launch(b, BK_RB, g + T_R2 + 1, 0, step);
   hipLaunchKernelGGL(k_r_bwd<1>, dim3(grid_for(b, BK_RB)), dim3(kLineThreads), b->radial_lds, st, L, nullptr, nullptr,
                      nullptr);
   L = slot_launch(b, BK_PB, g + T_P2 + 1, 0);
   hipLaunchKernelGGL(k_p_bwd, dim3(grid_for(b, BK_PB)), dim3(kLineThreads), b->azim_lds, st, L, nullptr, nullptr);
-  L = slot_launch(b, BK_PLANE, g + T_E1 + 1, 0);
-  launch_plane_bwd(SEQ_STEP, bwd_threads, dim3(grid_for(b, BK_PLANE)), bwd_lds, st, L, nullptr, nullptr);
+  L = slot_launch(b, BK_PLB, g + T_E1 + 1, 0);
+  const int *vmap = L.vmap;
+  for (const Plan::Group &gr : b->plan[BK_PLB].groups) {
+    L.vmap = vmap + gr.v0;
+    L.nv = gr.nv;
+    launch_plane_adj(gr.sh, dim3((unsigned)gr.nv), gr.lds, st, L, nullptr, nullptr);
+  }
   L = slot_launch(b, BK_PB, g + T_P1 + 1, 0);
   hipLaunchKernelGGL(k_p_bwd, dim3(grid_for(b, BK_PB)), dim3(kLineThreads), b->azim_lds, st, L, nullptr, nullptr);
   L = slot_launch(b, BK_RB, g + T_R1 + 1, 0, step);
@@ -665,10 +675,8 @@ int ramgpu_batch_adjoint_run(ramgpu_batch *b, int nsteps, int ckpt_every, const 
   const int nseg = (nsteps + ckpt_every - 1) / ckpt_every, seglen = std::min(ckpt_every, nsteps);
   // plane adjoint LDS
   size_t bwd_lds = 0, lds_limit = b->m[0]->lds_limit;
-  int bwd_threads = kPlaneThreads;
   for (ramgpu_ctx *c : b->m) {
     bwd_lds = std::max(bwd_lds, plane_bwd_lds_bytes(c->ne, c->npa));
-    bwd_threads = std::max(bwd_threads, plane_bwd_threads(c->ne, c->npa));
   }
   if (bwd_lds > lds_limit) return fail(RAMGPU_EINVAL, "plane adjoint does not fit the device LDS");
   set_plane_bwd_lds_limit(lds_limit);
@@ -806,7 +814,7 @@ int ramgpu_batch_adjoint_run(ramgpu_batch *b, int nsteps, int ckpt_every, const 
         enq_sched(b, s);
       }
       enq_misfit(b, out < 0 ? 0 : out, s, 1);
-      enq_step_bwd(b, group(s, n0), s, bwd_lds, bwd_threads);
+      enq_step_bwd(b, group(s, n0), s);
     }
     if ((rc = launch_check("ensemble adjoint"))) {
       detach();

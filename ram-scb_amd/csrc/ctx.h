@@ -21,6 +21,7 @@ __global__ void k_pitch_diffusion(const Tab *tp, PitchJob job);
 template <int FINAL> __global__ void k_r_bwd(Launch L, const double *xin, double *adj, double *bbar);
 __global__ void k_p_bwd(Launch L, const double *xin, double *adj);
 template <int SEQ, int BT> __global__ void k_plane_bwd(Launch L, const double *xin, double *adj);
+template <int R> __global__ void k_plane_adj(Launch L, const double *xin, double *adj);
 __global__ void k_misfit(const double *f2, int nr, int nt, int ne, int npa, int npts, const int *pts,
                          const double *w, const double *target, double *loss_out, double *lam);
 __global__ void k_misfit_ens(Launch L, int step, int adjoint);
@@ -79,6 +80,7 @@ struct ramgpu_ctx {
   size_t lds_limit = 65536;
   PlaneShape plane{ramgpu::kPlaneThreads, 16, 0};
   StepShape step{0, 0}, stepx{0, 0};  // of SEQ_STEP and SEQ_TAPE; of SEQ_STEPX
+  StepShape adj{0, 0};                // of the step's plane adjoint
   Tab t{};            // host image of the problem descriptor
   Tab *d_tab = nullptr;  // its device copy, read by every kernel
   bool tab_dirty = true;
@@ -188,6 +190,9 @@ void launch_plane(int seq, PlaneShape sh, dim3 grid, size_t lds, hipStream_t st,
 enum TapeSlot { T_R1, T_P1, T_E1, T_MU1, T_LOSS, T_MU2, T_E2, T_P2, T_R2, T_CLAMP, T_N };
 // plane adjoint kernels
 int plane_bwd_threads(int ne, int npa);
+StepShape adj_shape(int ne, int npa, long planes, int ncu, size_t lds_cu);
+void launch_plane_adj(StepShape sh, dim3 grid, size_t lds, hipStream_t st, const ramgpu::Launch &L, const double *x,
+                      double *adj);
 void set_plane_bwd_lds_limit(size_t limit);
 void launch_plane_bwd(int seq, int threads, dim3 grid, size_t lds, hipStream_t st, const ramgpu::Launch &L,
                       const double *x, double *adj);

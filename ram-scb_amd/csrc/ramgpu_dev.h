@@ -320,6 +320,19 @@ inline __host__ __device__ int step_resident(size_t lds, int ne, int npa, int ro
   const int by_waves = kStepSimdWaves / simd, by_lds = (int)(kLdsCu / lds);
   return by_waves < by_lds ? by_waves : by_lds;
 }
+// The step's plane adjoint (k_plane_adj): a wave takes adj_wave_cells of the
+// columns, the two lanes at either end repeating its neighbours'; LDS as the
+// forward's with 7*Q*NE doubles at the chunks' edges, in the rows' place, and
+// without sums and CFL slots.
+inline __host__ __device__ int adj_wave_cells(int ne) { return 64 % ne == 0 ? 64 : 60; }
+inline __host__ __device__ int adj_threads(int ne, int npa, int rows) {
+  const int w = adj_wave_cells(ne);
+  return (step_chunks(npa, rows) * ne + w - 1) / w * 64;
+}
+inline __host__ __device__ size_t adj_lds_bytes(int ne, int npa, int rows) {
+  const size_t q = step_chunks(npa, rows), npap = q * rows, plane = npap * (ne + 3), edges = 7 * q * ne;
+  return ((plane > edges ? plane : edges) + 1 + 21 * npap + 5 + 10 * (size_t)ne + 64) * sizeof(double);
+}
 // SEQ_STEPX's further LDS: wider sums, the per-row terms of the line solves
 // and what they hand between chunks
 inline __host__ __device__ size_t step_extra_bytes(int ne, int npa, int rows) {

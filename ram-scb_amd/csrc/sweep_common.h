@@ -153,7 +153,7 @@ __device__ __forceinline__ FaceD face_d(double f0, double fp1, double fn, double
   const double x = fp1 - f0;
   const double fup = 0.5 * (f0 + fp1 - sg * x);
   const double u0 = 0.5 * (1.0 + sg), u1 = 0.5 * (1.0 - sg);
-  const double rr = (fn - fnm1) / x;
+  const double rr = div_fast(fn - fnm1, x);
   const bool lin = !(fabs(x) <= 1.E-27) && !(rr <= 0);
   const double A = fmin(beta * rr, 1.0), B = fmin(rr, beta);
   const double lim = fmax(A, B);
