@@ -642,7 +642,7 @@ int ramgpu_create(ramgpu_ctx **out, int ns, int nr, int nt, int ne, int npa, int
   t.ns = ns; t.nr = nr; t.nt = nt; t.ne = ne; t.npa = npa;
   t.r_rows = line_rows(nr, (long)ns * nt * ne * npa, ncu);
   t.p_rows = line_rows(nt, (long)ns * (nr - 1) * ne * npa, ncu);
-  t.maxblk = std::max(blocks_kl(t), blocks_r(t));  // partial sums per (slot, species)
+  t.maxblk = std::max({blocks_kl(t), blocks_r(t), blocks_line_r(t), blocks_p(t), blocks_line_p(t)});
   if (plane_bwd_lds_bytes(ne, npa) > c->lds_limit)
     return cleanup(fail(RAMGPU_EINVAL, "NE*NPA=%d plane does not fit the device LDS (%zu bytes)", ne * npa,
                         c->lds_limit));
@@ -689,7 +689,7 @@ int ramgpu_create(ramgpu_ctx **out, int ns, int nr, int nt, int ne, int npa, int
   A(t.dtdrift, (size_t)ns * 4);
   A(t.f2, nf2);
   A(c->d_stage, nf2);
-  A(t.partials, (size_t)(kSumSlots + 1) * ns * t.maxblk);  // + ELORC slot of ramgpu_sumrc
+  A(t.partials, (size_t)kSlots * ns * t.maxblk);
   A(t.energy, (size_t)ns * 4);
   A(t.wl, (size_t)3 * ns * nr * ne); A(t.rlpp, nt); A(t.lsx, (size_t)ns * 3);
   A(t.wavef, (size_t)ns * nr * nt * ne);
@@ -1090,7 +1090,7 @@ int ramgpu_sumrc(ramgpu_ctx *c, int s, double *setrc, double *elorc) {
   if ((rc = run_finalize(c, 0, 1, s - 1, 1))) return rc;
   double e[4], el;
   HIP_TRY(hipMemcpyAsync(e, c->t.energy + (s - 1) * 4, 4 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipMemcpyAsync(&el, c->t.partials + ((size_t)kSumSlots * c->ns + (s - 1)) * c->t.maxblk,
+  HIP_TRY(hipMemcpyAsync(&el, c->t.partials + ((size_t)kSlotElorc * c->ns + (s - 1)) * c->t.maxblk,
                          sizeof(double), hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
   if (setrc) *setrc = e[0];

@@ -641,7 +641,7 @@ __global__ void __launch_bounds__(kLineThreads, 4) k_r(Launch L) {
     }
     if (MODE == 1) {
       const double m = block_max(cmax, red);
-      if (threadIdx.x == 0 && m > 0) atomic_max_pos(&t.cflmax[(size_t)s * (2 + NE + t.npa) + 0], m);
+      if (threadIdx.x == 0) t.partials[((size_t)kSlotCflR * t.ns + s) * t.maxblk + u.b] = m;
     }
     if (MODE == 2) {
       double a[1] = {acc}, tot[1];
@@ -758,7 +758,7 @@ __global__ void __launch_bounds__(kLineThreads) k_p(Launch L) {
     }
     if (MODE == 1) {
       const double m = block_max(cmax, red);
-      if (threadIdx.x == 0 && m > 0) atomic_max_pos(&t.cflmax[(size_t)s * (2 + NE + t.npa) + 1], m);
+      if (threadIdx.x == 0) t.partials[((size_t)kSlotCflP * t.ns + s) * t.maxblk + u.b] = m;
     }
     __syncthreads();  // the block's face terms are read
   }
@@ -1302,7 +1302,7 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, 4) k_plane(Launch L, int rec
 // eight slots are in use, sixteen's for one), by lane adds without LDS; with
 // every thread summing all slots the block reduction of sixteen values took
 // most of 14.0 us.  Now 5.1 (one species of 20x25x35x72), 3.6 for a DtDrift.
-constexpr int kFinRed = kFinalizeThreads / 64 + 2;  // the waves' sums, then the DtDriftE and DtDriftMu minima
+constexpr int kFinRed = kFinalizeThreads / 64 + 4;  // the waves' sums, DtDriftE and DtDriftMu, the R and P maxima
 __device__ inline void finalize_unit(const Launch &L, int vb, int cflmask, int mode, double *red) {
   {
     const CUnit u = const_unit(L, vb);
@@ -1317,7 +1317,6 @@ __device__ inline void finalize_unit(const Launch &L, int vb, int cflmask, int m
     const gptr<const unsigned long long> gm = as_global((const unsigned long long *)m);
     // thread 0's scalars
     double e0[4] = {0.0, 0.0, 0.0, 0.0}, lswae = 0.0, lscoe = 0.0, lscsc = 0.0;
-    unsigned long long m01[2] = {0ull, 0ull};
     const bool coul = t.coul != 0;
     const bool lines = t.pd_wpi[s] || t.pd_emic[s] || t.flc[s];
     const bool emic = lines && (t.sum_any & ANY_EMIC);
@@ -1329,8 +1328,6 @@ __device__ inline void finalize_unit(const Launch &L, int vb, int cflmask, int m
       lswae = gl[0];
       lscoe = gl[1];
       lscsc = gl[2];
-      m01[0] = gm[0];
-      m01[1] = gm[1];
     }
     // the slots in use: 0..6 (and with the optional processes 8..13) from the
     // plane blocks, 7 from the R blocks; a single SUMRC reads slot 0
@@ -1364,6 +1361,26 @@ __device__ inline void finalize_unit(const Launch &L, int vb, int cflmask, int m
       for (int off = 32; off > 0; off >>= 1) v = fmin(v, __shfl_down(v, off, 64));
       if (lane == 0) red[W + (mu ? 1 : 0)] = v;
     }
+    // DRIFTR's and DRIFTP's: the maxima of their blocks, however many the
+    // recording launch had (entries beyond are 0)
+    if (((cflmask & 1) && w == W - 4) || ((cflmask & 2) && w == W - 3)) {
+      const bool pz = w == W - 3;
+      const int n = pz ? max(blocks_p(t), blocks_line_p(t)) : max(blocks_r(t), blocks_line_r(t));
+      const gptr<double> p = as_global(t.partials + ((size_t)(pz ? kSlotCflP : kSlotCflR) * t.ns + s) * t.maxblk);
+      double mx = 0.0;
+      for (int b0 = lane; b0 < n; b0 += 8 * 64) {
+        double v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = (b0 + q * 64 < n) ? p[b0 + q * 64] : 0.0;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) mx = fmax(mx, v[q]);
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+          if (b0 + q * 64 < n) p[b0 + q * 64] = 0.0;
+      }
+      for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_down(mx, off, 64));
+      if (lane == 0) red[W + (pz ? 3 : 2)] = mx;
+    }
     __syncthreads();
     if (tid == 0) {
       auto sum = [&](int id) {
@@ -1372,14 +1389,8 @@ __device__ inline void finalize_unit(const Launch &L, int vb, int cflmask, int m
         for (int q = 1; q < per; ++q) v += red[g * per + q];
         return v;
       };
-      if (cflmask & 1) {
-        const double c = __longlong_as_double((long long)m01[0]);
-        t.dtdrift[s * 4 + 0] = (c > 0) ? fmin(100000.0, a / c) : 100000.0;
-      }
-      if (cflmask & 2) {
-        const double c = __longlong_as_double((long long)m01[1]);
-        t.dtdrift[s * 4 + 1] = (c > 0) ? fmin(100000.0, a / c) : 100000.0;
-      }
+      if (cflmask & 1) t.dtdrift[s * 4 + 0] = (red[W + 2] > 0) ? fmin(100000.0, a / red[W + 2]) : 100000.0;
+      if (cflmask & 2) t.dtdrift[s * 4 + 1] = (red[W + 3] > 0) ? fmin(100000.0, a / red[W + 3]) : 100000.0;
       if (cflmask & 4) t.dtdrift[s * 4 + 2] = red[W];
       if (cflmask & 8) t.dtdrift[s * 4 + 3] = red[W + 1];
       if (mode != 0) {
@@ -1401,7 +1412,7 @@ __device__ inline void finalize_unit(const Launch &L, int vb, int cflmask, int m
         if (mode == 1) {
           const double elorc = old - S[0];
           e[0] = S[0];
-          t.partials[((size_t)kSumSlots * t.ns + s) * t.maxblk] = elorc;  // ELORC
+          t.partials[((size_t)kSlotElorc * t.ns + s) * t.maxblk] = elorc;
         } else {
           // the accumulators of src/ModRamRun.f90:77-175 from consecutive
           // slot sums, each operator's only where the reference runs it
@@ -1465,7 +1476,7 @@ __device__ inline void finalize_unit(const Launch &L, int vb, int cflmask, int m
       }
     }
     __syncthreads();  // every read of the maxima is done
-    if (cflmask)
+    if (cflmask & 12)
       for (int e = tid; e < 2 + NE + NPA; e += T) m[e] = 0ull;
     __syncthreads();  // red is reused by the block's next unit
   }

@@ -32,6 +32,9 @@ constexpr int kMaxPlaneCells = kPlaneThreads * kMaxCellsPerThread;  // NE*NPA bo
 // (plane blocks: after the first drift half, after COULEN; after the second
 // COULMU, after the second COULEN), 12, 13 after the EMIC WPADIFs
 constexpr int kSumSlots = 14;
+// further slots of partials: ramgpu_sumrc's ELORC, and the blocks' CFL maxima
+// of DRIFTR and DRIFTP (cleared by k_finalize)
+constexpr int kSlotElorc = kSumSlots, kSlotCflR = kSumSlots + 1, kSlotCflP = kSumSlots + 2, kSlots = kSumSlots + 3;
 constexpr int kSumRadial = 7;
 constexpr int kSumCoul = 8;
 constexpr int kSumEmic = 12;
@@ -127,7 +130,7 @@ struct Tab {
   double *ex64;   // [j] 2^(j/64), the table of the loss factors' exponential
   // CFL maxima of max(|C|,floor) over cells inside the magnetopause, as the
   // bit patterns of non-negative doubles (atomicMax order = double order):
-  // [s][0] R, [s][1] P, [s][2+K] E per K, [s][2+NE+L] Mu per L
+  // [s][2+K] E, [s][2+NE+L] Mu (R's and P's: slots kSlotCflR, kSlotCflP)
   unsigned long long *cflmax;
   double *dtdrift;      // [s][4]
   // float reciprocals for exact small-integer division (fast_div)
