@@ -758,7 +758,8 @@ __global__ void __launch_bounds__(kLineThreads) k_p(Launch L) {
     }
     if (MODE == 1) {
       const double m = block_max(cmax, red);
-      if (threadIdx.x == 0) t.partials[((size_t)kSlotCflP * t.ns + s) * t.maxblk + u.b] = m;
+      // (not the blocks beyond the rings, which only copy)
+      if (threadIdx.x == 0 && line0 < nring) t.partials[((size_t)kSlotCflP * t.ns + s) * t.maxblk + u.b] = m;
     }
     __syncthreads();  // the block's face terms are read
   }

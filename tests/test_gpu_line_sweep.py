@@ -46,3 +46,18 @@ def test_line_sweeps_at_mapping_edges(grid):
         for k in ("setrc", "lsdr"):
             assert abs(out[s][k] - o.arr(k)[s]) <= RTOL * abs(o.arr("setrc")[s]), (s, k)
     g.close()
+
+
+def test_recording_out_of_place_sweep_keeps_every_species_limit():
+    # out of place (the taped step), DRIFTP's launch has more blocks than any
+    # other kernel, those that copy the I=1 rows; the CFL maxima it records
+    # must be the in-place sweep's
+    p = random_problem(4, 48, 64, 90, species=(sp.ELECTRON, sp.HYDROGEN, sp.HELIUM, sp.OXYGEN), seed=7)
+    a, b = RamGpu.from_problem(p), RamGpu.from_problem(p)
+    a.ram_run_bwd(np.ones_like(p.f2))  # records the limits on its taped step
+    ra, rb = a.ram_run(1), b.ram_run(1)
+    for s in range(4):
+        for k in ("dtdrift_r", "dtdrift_p", "dtdrift_e", "dtdrift_mu"):
+            assert ra[s][k] == rb[s][k], (s, k)
+    a.close()
+    b.close()
