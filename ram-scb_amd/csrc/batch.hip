@@ -230,7 +230,8 @@ void enq_r(ramgpu_batch *b, Launch L, int mode) {
   L.jobs = p.jobs;
   L.vmap = p.vmap;
   L.nv = p.nv;
-  launch_r(mode, {0, kLineThreads, b->radial_lds}, dim3(grid_for(b, BK_RB)), b->stream, L);
+  const int cap = b->plan[BK_R].cap, grid = (cap > 0 && cap < p.nv) ? cap : p.nv;
+  launch_r(mode, {0, kLineThreads, b->radial_lds}, dim3((unsigned)grid), b->stream, L);
 }
 
 void destroy_graphs(ramgpu_batch *b) {

@@ -12,8 +12,9 @@
 //   k_ghost     DRIFTR outer-ghost carry between lines (see k_ghost)
 //   k_r         DRIFTR, one thread per radial line (J,K,L)
 //   k_p         DRIFTP, one thread per azimuthal ring (I,K,L)
-//   k_plane     DRIFTE / DRIFTMU sweeps, loss operators and SUMRC on whole
-//               (K,L) planes in LDS
+//               (k_r_rows, k_p_rows for few lines: line_sweep.hip)
+//   k_plane     DRIFTE, DRIFTMU, a loss operator, SUMRC, COULEN or COULMU on
+//               whole (K,L) planes in LDS (the step's: plane_step.hip)
 //   k_finalize  DtDrift* from the CFL partial maxima; SUMRC bookkeeping
 //   k_vs        Volland-Stern VT from Kp
 //
@@ -945,7 +946,7 @@ __device__ void plane_e(const Tab &t, const FwdCtx &c, const PlaneFwd &d, bool r
       const double f0 = p[1], fp1 = p[2];
       const double a = p[neg ? 3 : 0];
       const double fn = neg ? a : f0, fnm1 = neg ? fp1 : a;
-      const double fb = face_value_sel(f0, fp1, fn, fnm1, ce, div_rn(ce, de, rde), beta);
+      const double fb = face_value(f0, fp1, fn, fnm1, ce, div_rn(ce, de, rde), beta);
       const double h = div_rn(ce, we1, rwe1) * fb;
       // the lower neighbour is lane-1 of the same chunk (same rows), or for
       // lane 0 the last lane of the wave before, whose term comes after the
@@ -1028,7 +1029,7 @@ __device__ void plane_mu(const Tab &t, const FwdCtx &c, const PlaneFwd &d, bool 
       const double a = neg ? f2 : (L1 <= 2 ? f0 : fm);  // F(1) = F(2)
       const double fn = neg ? a : f0, fnm1 = neg ? f1 : a;
       const int lw = (L1 <= NPA - 1) ? l + 1 : l;  // WMU(L+1) of the face's upper cell (in range)
-      const double fl = face_value_sel(f0, f1, fn, fnm1, cm, div_rn(cm, d.lt[LT_DMU * NPA + l], d.lt[LT_RDMU * NPA + l]), beta);
+      const double fl = face_value(f0, f1, fn, fnm1, cm, div_rn(cm, d.lt[LT_DMU * NPA + l], d.lt[LT_RDMU * NPA + l]), beta);
       const double fb = (L1 == NPA - 1) ? f1 : fl;  // FBND(NPA-1) = F(NPA)
       // faces 1 and NPA carry nothing: face 1 has CDriftMu(1)=0, FBND(1)=0
       // (its term 0/WMU(2)*0 = 0); row NPA is the top cell

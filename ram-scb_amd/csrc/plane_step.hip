@@ -12,8 +12,9 @@
 // stencil, and the flux terms handed over between chunks.
 //
 // What bounds it: VALU issue.  A cell takes about 430 vector instructions a
-// step (72 a DRIFTE row, 80 a DRIFTMU row, two table-driven exponentials; the
-// kernel with the plane in LDS that this one replaces took 637), two thirds
+// step (72 a DRIFTE row, 80 a DRIFTMU row, two table-driven exponentials; 522
+// by the counters, with the lanes that a 35x72 plane leaves idle; the kernel
+// with the plane in LDS that this one replaces took 637), two thirds
 // of the issue slots over a launch of 1900 35x72 planes.  Rows in registers
 // took the LDS round trips between the pitch-angle sweeps and the loss chain
 // out, and with whole chunks per thread six barriers a plane are left of

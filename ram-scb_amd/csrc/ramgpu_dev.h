@@ -141,7 +141,7 @@ struct Tab {
   int plane_chunks;
   int step_cells, step_apart;  // step_wave_cells, step_edges_apart of k_plane_step's shape
   int stepx_apart;             // step_edges_apart of SEQ_STEPX's
-  int r_rows, p_rows;          // rows of k_r_rows and k_p_rows; 0: k_r, k_p (lines too long)
+  int r_rows, p_rows;          // rows of k_r_rows and k_p_rows; 0: k_r, k_p (line_rows)
   // state
   double *f2;
   double *partials;  // [slot][s][maxblk]

@@ -66,39 +66,6 @@ __host__ __device__ inline double exp_tab(double x, const double *tab) {
   return ldexp(fma(tab[j], p, tab[j]), m);
 }
 
-// Limited face value of the reference's upwind scheme (src/ModRamDrift.f90:
-// 169-183) for the face between F(I) = f0 and F(I+1) = fp1.  fn and fnm1 are
-// F(N) and F(N-1) with N = I+1-sgn as the reference forms it (including its
-// periodic wrap in DRIFTP); cn is the Courant number as the limiter's CORR
-// term sees it (C, C/DE(K) or C/DMU(L)).
-__device__ __forceinline__ double face_value(double f0, double fp1, double fn, double fnm1,
-                                             double c, double cn, double beta) {
-  const double sg = (c < 0) ? -1.0 : 1.0;
-  const double x = fp1 - f0;
-  const double fup = 0.5 * (f0 + fp1 - sg * x);
-  if (fabs(x) <= 1.E-27) return fup;
-  const double r = (fn - fnm1) / x;
-  if (r <= 0) return fup;
-  const double lim = fmax(fmin(beta * r, 1.0), fmin(r, beta));
-  const double corr = -0.5 * (cn - sg) * x;
-  return fup + lim * corr;
-}
-
-// face_value without branches: every lane forms the ratio and the limited
-// value, then keeps FUP where the reference returns early (|X| <= 1e-27 or
-// R <= 0); the arithmetic of the value kept is face_value's.
-__device__ __forceinline__ double face_value_sel(double f0, double fp1, double fn, double fnm1,
-                                                 double c, double cn, double beta) {
-  const double sg = (c < 0) ? -1.0 : 1.0;
-  const double x = fp1 - f0;
-  const double fup = 0.5 * (f0 + fp1 - sg * x);
-  const double r = (fn - fnm1) / x;
-  const double lim = fmax(fmin(beta * r, 1.0), fmin(r, beta));
-  const double corr = -0.5 * (cn - sg) * x;
-  const double v = fup + lim * corr;
-  return (fabs(x) <= 1.E-27 || r <= 0) ? fup : v;
-}
-
 // a/x, correctly rounded: the reciprocal from the hardware's by one cubic
 // iteration, the quotient by the residual correction of div_rn.  It is the
 // compiler's own division without its scaling of extreme exponents, so the
@@ -112,6 +79,25 @@ __device__ __forceinline__ double div_fast(double a, double x) {
   double q = a * y;
   q = fma(fma(-x, q, a), y, q);
   return __builtin_amdgcn_div_fixup(q, x, a);
+}
+
+// Limited face value of the reference's upwind scheme (src/ModRamDrift.f90:
+// 169-183) for the face between F(I) = f0 and F(I+1) = fp1.  fn and fnm1 are
+// F(N) and F(N-1) with N = I+1-sgn as the reference forms it (including its
+// periodic wrap in DRIFTP); cn is the Courant number as the limiter's CORR
+// term sees it (C, C/DE(K) or C/DMU(L)).  Without branches: every lane forms
+// the ratio and the limited value, then keeps FUP where the reference returns
+// early (|X| <= 1e-27 or R <= 0).
+__device__ __forceinline__ double face_value(double f0, double fp1, double fn, double fnm1, double c, double cn,
+                                             double beta) {
+  const double sg = (c < 0) ? -1.0 : 1.0;
+  const double x = fp1 - f0;
+  const double fup = 0.5 * (f0 + fp1 - sg * x);
+  const double r = div_fast(fn - fnm1, x);
+  const double lim = fmax(fmin(beta * r, 1.0), fmin(r, beta));
+  const double corr = -0.5 * (cn - sg) * x;
+  const double v = fup + lim * corr;
+  return (fabs(x) <= 1.E-27 || r <= 0) ? fup : v;
 }
 
 // Twice the face value of face_value, for callers that fold the factor 1/2
@@ -230,14 +216,6 @@ __device__ __forceinline__ void fetched(T... x) {
 __device__ __forceinline__ int fresh(int x) {
   asm volatile("" : "+v"(x));
   return x;
-}
-
-// The value of x in lane `lane` of the wave (a wave-uniform value).
-__device__ __forceinline__ double lane_value(double x, int lane) {
-  const long long b = __double_as_longlong(x);
-  const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffLL), lane);
-  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
 // A block-uniform x (read from LDS) held in scalar registers.
@@ -470,19 +448,6 @@ __device__ inline double block_max(double v, double *red) {
   return m;
 }
 
-__device__ inline double block_min(double v, double *red) {
-  for (int off = 32; off > 0; off >>= 1) v = fmin(v, __shfl_down(v, off, 64));
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  __syncthreads();
-  if (lane == 0) red[wid] = v;
-  __syncthreads();
-  double m = v;
-  const int nw = (blockDim.x + 63) >> 6;
-  for (int w = 0; w < nw; ++w) m = fmin(m, red[w]);
-  __syncthreads();
-  return m;
-}
-
 __device__ __forceinline__ void atomic_max_pos(unsigned long long *slot, double v) {
   atomicMax(slot, (unsigned long long)__double_as_longlong(v));  // v >= 0
 }
@@ -585,9 +550,6 @@ enum PlaneSeq : int {
 __host__ __device__ constexpr bool seq_coul(int seq) {
   return seq == SEQ_COULEN || seq == SEQ_COULMU;
 }
-
-// Elements of one F2-sized buffer (all species) of the problem t.
-__device__ __forceinline__ size_t f2_elems(const Tab &t) { return (size_t)t.ns * f2_species_stride(t); }
 
 // LDS layout of the plane kernel (doubles)
 struct PlaneLds {
