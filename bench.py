@@ -37,7 +37,7 @@ More objects in the same line:
     Coulomb collisions on (COULEN and COULMU twice a step in the plane
     kernel);
   "multi_species_all_processes": a sixth of the steps with every optional
-    process on (Coulomb, e- WPADIF, H+ EMIC, He+ FLC): the composed step;
+    process on (Coulomb, e- WPADIF, H+ EMIC, He+ FLC), in the plane kernel;
   "adjoint": H+ on 20x25x35x72, 60 steps, virtual-satellite misfit at 8
     points, gradient w.r.t. the initial F2 and every step's FGEOS with
     checkpoints every 10 steps, against the 60-step forward alone;
@@ -71,10 +71,10 @@ import numpy as np  # noqa: E402
 HBM_PEAK_GBPS = 8000.0       # MI355X HBM3E, AMD specification
 SWEEP_BYTES = 16             # one FP64 read + one FP64 write of F2 per cell and sweep
 # algorithmic sweeps per launch: k_r one (DRIFTR), k_p one (DRIFTP, rows
-# I>=2), k_plane four (DRIFTE, DRIFTMU, DRIFTMU, DRIFTE on rows I>=2)
+# I>=2), k_plane_step four (DRIFTE, DRIFTMU, DRIFTMU, DRIFTE on rows I>=2)
 SWEEPS_PER_LAUNCH = {"r": 1, "p": 1, "plane": 4}
 KERNEL_NAMES = {"r": "k_r (radial sweep, DRIFTR)", "p": "k_p (azimuthal sweep, DRIFTP)",
-                "plane": "k_plane (energy + pitch-angle sweeps and loss chain, one (K,L) plane per block)"}
+                "plane": "k_plane_step (energy + pitch-angle sweeps and loss chain, one (K,L) plane per block)"}
 ALGO_BYTES_PER_CELL_UPDATE = 128  # 8 directional sweeps x (read + write) of F2
 METRIC = "FP64 RAM split-step cell-updates/s + HBM roofline %; batched & adjoint vs plain"
 TRAFFIC_FILE = REPO / "profiles" / "traffic_c3_ensemble.txt"
@@ -327,7 +327,7 @@ def bench_multi_species(steps: int, warmup: int, seed: int, coulomb: bool = Fals
     scale LogNormal(0,0.3) per step; with coulomb, Coulomb collisions on
     (synthetic plasmasphere of Kp=2, TimeRamElapsed from 0); with pitch also
     WPADIF for e- in place of WAVELO, EMIC WPADIF for H+ and FLC scattering
-    for He+ (synthetic coefficients), which takes the composed step."""
+    for He+ (synthetic coefficients)."""
     from ramgpu import inputs
     from ramgpu.capi import RamGpu, copy_probe
 
@@ -362,13 +362,12 @@ def bench_multi_species(steps: int, warmup: int, seed: int, coulomb: bool = Fals
     ev_ms = dev.last_run_ms()
     ktimes = dev.kernel_times()
     dev.kernel_timing(False)
-    if pitch:  # one launch per operator: device time per step by kernel kind instead of a roofline
+    if pitch:  # the plane launch holds the line solves too: device time per step by kernel kind instead of a roofline
         value = cells * steps / (dev_ms * 1e-3)
         per = {k: {"ms_per_step": v[0] / steps, "launches_per_step": v[1] / steps} for k, v in ktimes.items() if v[1]}
         log(f"bench: all processes {dev_ms / steps * 1e3:.1f} us/step, {value:.3e} cell-updates/s")
         res = {"workload": "e-(WPADIF),H+(EMIC),He+(FLC),O+ (1:0.7:0.05:0.25) on 20x25x35x72 with Coulomb "
-                           "collisions, dt=5 s, Kp 2->6 ramp, boundary scale LogNormal(0,0.3) per step; the "
-                           "composed step (one launch per operator)",
+                           "collisions, dt=5 s, Kp 2->6 ramp, boundary scale LogNormal(0,0.3) per step",
                "cells": cells, "steps": steps, "value": value, "unit": "cell-updates/s",
                "ms_per_step": dev_ms / steps, "ms_per_step_with_kernel_events": ev_ms / steps,
                "kernels": per}
@@ -560,7 +559,7 @@ def main():
                     help="run only the multi-species leg and print its object (profiling)")
     ap.add_argument("--coulomb", action="store_true", help="with --multi-only: Coulomb collisions on")
     ap.add_argument("--all-processes", action="store_true",
-                    help="with --multi-only: every optional process on (the composed step)")
+                    help="with --multi-only: every optional process on")
     ap.add_argument("--no-coulomb", action="store_true", help="skip the multi-species leg with Coulomb collisions")
     ap.add_argument("--hi-only", action="store_true", help="only the computehI leg")
     args = ap.parse_args()

@@ -294,9 +294,8 @@ int ramgpu_moments(ramgpu_ctx *ctx, double *ppert, double *ppart, double *edent,
  * periodic local-time copy and the magnetopause mask.  Each optional
  * process as its set-up call switches it on: WAVELO (ramgpu_set_wavelo),
  * Coulomb collisions (ramgpu_set_coulomb), WPADIF and EMIC
- * (ramgpu_set_wpadif), FLC scattering (ramgpu_set_flc).  Without WPADIF and
- * FLC the middle of the step is one fused plane kernel; with them the step
- * runs one launch per operator for all species at once (the same results).
+ * (ramgpu_set_wpadif), FLC scattering (ramgpu_set_flc).  The middle of the
+ * step, from DRIFTE to DRIFTE, is one plane kernel.
  * out (may be NULL) receives NS records for the last step. */
 int ramgpu_ram_run(ramgpu_ctx *ctx, int nsteps, ramgpu_species_out *out);
 
@@ -332,7 +331,8 @@ int ramgpu_last_run_ms(ramgpu_ctx *ctx, double *ms);
  * device time and the launch count since the last query, then resets. */
 #define RAMGPU_KERNEL_PREPARE 0  /* species tables, Courant terms, ghost carry */
 #define RAMGPU_KERNEL_R 1        /* radial sweeps (DRIFTR)                    */
-#define RAMGPU_KERNEL_PLANE 2    /* energy / pitch-angle sweeps, losses, SUMRC */
+#define RAMGPU_KERNEL_PLANE 2    /* energy / pitch-angle sweeps, losses, SUMRC; in
+                                     ram_run also WPADIF and FLCscatter     */
 #define RAMGPU_KERNEL_FINALIZE 3 /* DtDrift* and SUMRC bookkeeping            */
 #define RAMGPU_KERNEL_VS 4       /* Volland-Stern VT from Kp; a schedule forms
                                      it with the Courant-number terms, timed
@@ -342,7 +342,7 @@ int ramgpu_last_run_ms(ramgpu_ctx *ctx, double *ms);
 #define RAMGPU_KERNEL_P_BWD 7    /* adjoint of DRIFTP                         */
 #define RAMGPU_KERNEL_PLANE_BWD 8 /* adjoints of DRIFTE, DRIFTMU, losses      */
 #define RAMGPU_KERNEL_MOMENTS 9  /* ANISCH pressure moments and FLUX          */
-#define RAMGPU_KERNEL_PITCH 10   /* WPADIF and FLCscatter line solves          */
+#define RAMGPU_KERNEL_PITCH 10   /* WPADIF and FLCscatter on their own         */
 #define RAMGPU_KERNEL_KINDS 11
 int ramgpu_kernel_timing(ramgpu_ctx *ctx, int enable);
 /* Measurement support: a plain device copy of `bytes` (read + write) run
