@@ -102,14 +102,14 @@ int upload_f2(ramgpu_ctx *c, double *dst, const double *host) {
   const size_t n = (size_t)c->ns * c->nr * c->nt * c->ne * c->npa;
   const int rc = copy_to_device(c->device, c->stream, c->d_stage, host, n * sizeof(double));
   if (rc) return rc;
-  hipLaunchKernelGGL(k_f2_in, dim3(1024), dim3(256), 0, c->stream, dst, (const double *)c->d_stage, c->ns, c->nr,
+  hipLaunchKernelGGL(k_f2_in, dim3(2048), dim3(256), 0, c->stream, dst, (const double *)c->d_stage, c->ns, c->nr,
                      c->nt, c->ne, c->npa);
   return launch_check("k_f2_in");
 }
 
 int download_f2(ramgpu_ctx *c, double *host, const double *src) {
   const size_t n = (size_t)c->ns * c->nr * c->nt * c->ne * c->npa;
-  hipLaunchKernelGGL(k_f2_out, dim3(1024), dim3(256), 0, c->stream, c->d_stage, src, c->ns, c->nr, c->nt, c->ne,
+  hipLaunchKernelGGL(k_f2_out, dim3(2048), dim3(256), 0, c->stream, c->d_stage, src, c->ns, c->nr, c->nt, c->ne,
                      c->npa);
   int rc = launch_check("k_f2_out");
   if (rc) return rc;

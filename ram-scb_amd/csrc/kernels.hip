@@ -1681,39 +1681,71 @@ __global__ void k_copy(double2 *__restrict__ dst, const double2 *__restrict__ sr
     dst[x] = src[x];
 }
 
-// Fortran F2(NS,NR,NT,NE,NPA) <-> device [S][I][J][L][K]
-__global__ void k_f2_in(double *dst, const double *src, int ns, int nr, int nt, int ne, int npa) {
-  const size_t n = (size_t)ns * nr * nt * ne * npa;
-  for (size_t x = blockIdx.x * (size_t)blockDim.x + threadIdx.x; x < n; x += (size_t)gridDim.x * blockDim.x) {
-    size_t r = x;  // device index: k fastest, then l, j, i, s
-    const int k = r % ne;
-    r /= ne;
-    const int l = r % npa;
-    r /= npa;
-    const int j = r % nt;
-    r /= nt;
-    const int i = r % nr;
-    r /= nr;
-    const int s = (int)r;
-    dst[x] = src[s + (size_t)ns * (i + (size_t)nr * (j + (size_t)nt * (k + (size_t)ne * l)))];
+// Fortran F2(NS,NR,NT,NE,NPA) <-> device [S][I][J][L][K], for one (J,L) at a
+// time: its (S,I) rows are runs of NE on the device, its K columns runs of
+// NS*NR in the Fortran array.  Bound by memory, and before that by the side
+// that a thread per cell moved in single doubles, each its own line.  Tiles of
+// at most 2048 cells (64 columns, 128 rows; 17 KB, eight blocks a CU), as even
+// as the sizes allow (fixed 64x32 tiles left 35 energies a second tile of
+// three: 45 us against 25), pass through LDS: both sides move whole runs, eight
+// cells a thread in flight.  In / out, a thread per cell -> tiles:
+// 4x20x25x35x72 (40 MB) 98 / 65 -> 25 / 22 us (3.2 and 3.7 TB/s moved),
+// 4x40x49x35x72 (158 MB) 385 / 525 -> 70 / 81 us, 1x20x25x35x72 21 / 22 ->
+// 14 / 13 us; at 0.3 MB the second trip through LDS costs 2 us.
+template <bool IN>
+__device__ __forceinline__ void f2_tiles(double *dst, const double *src, int ns, int nr, int nt, int ne, int npa) {
+  constexpr int TR = 128, TK = 64, T = 2048, U = T / 256;  // blocks of 256 threads
+  __shared__ double tile[T + TR];
+  const int rows = ns * nr, tid = threadIdx.x;
+  const int nkt = (ne + TK - 1) / TK, kw = (ne + nkt - 1) / nkt, S = kw | 1, rm = min(TR, T / kw);
+  const int nrt = (rows + rm - 1) / rm, rw = (rows + nrt - 1) / nrt;
+  const unsigned units = (unsigned)nt * npa * nrt * nkt;
+  for (unsigned u = blockIdx.x; u < units; u += gridDim.x) {
+    const unsigned w = u / (unsigned)nkt, jl = w / (unsigned)nrt;
+    const int kt = (int)(u - w * nkt), rt = (int)(w - jl * nrt), l = (int)(jl / (unsigned)nt), j = (int)jl - l * nt;
+    const int r0 = rt * rw, k0 = kt * kw;
+    const int rc = min(rw, rows - r0), kc = min(kw, ne - k0), n = rc * kc;
+    if (rc <= 0 || kc <= 0) continue;  // even tiles can leave none to the last: the whole block
+    const float rrc = 1.0f / (float)rc, rkc = 1.0f / (float)kc, rns = 1.0f / (float)ns;
+    // cell e of the tile as the device orders it and as Fortran does
+    auto dev = [&](int e, int &t) {
+      const int r = fast_div(e, kc, rkc), k = e - r * kc, i = fast_div(r0 + r, ns, rns), s = r0 + r - i * ns;
+      t = r * S + k;
+      return (((size_t)s * nr + i) * nt + j) * ((size_t)ne * npa) + (size_t)l * ne + k0 + k;
+    };
+    auto host = [&](int e, int &t) {
+      const int k = fast_div(e, rc, rrc), r = e - k * rc;
+      t = r * S + k;
+      return r0 + r + (size_t)rows * (j + (size_t)nt * (k0 + k + (size_t)ne * l));
+    };
+    double v[U];
+    int t[U];
+#pragma unroll
+    for (int m = 0; m < U; ++m) {
+      const int x = min(tid + m * 256, n - 1);
+      v[m] = src[IN ? host(x, t[m]) : dev(x, t[m])];
+    }
+#pragma unroll
+    for (int m = 0; m < U; ++m)
+      if (tid + m * 256 < n) tile[t[m]] = v[m];
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < U; ++m) {
+      const int x = tid + m * 256;
+      if (x < n) {
+        int tt;
+        const size_t o = IN ? dev(x, tt) : host(x, tt);
+        dst[o] = tile[tt];
+      }
+    }
+    __syncthreads();  // the tile is read
   }
 }
-
-__global__ void k_f2_out(double *dst, const double *src, int ns, int nr, int nt, int ne, int npa) {
-  const size_t n = (size_t)ns * nr * nt * ne * npa;
-  for (size_t x = blockIdx.x * (size_t)blockDim.x + threadIdx.x; x < n; x += (size_t)gridDim.x * blockDim.x) {
-    size_t r = x;
-    const int k = r % ne;
-    r /= ne;
-    const int l = r % npa;
-    r /= npa;
-    const int j = r % nt;
-    r /= nt;
-    const int i = r % nr;
-    r /= nr;
-    const int s = (int)r;
-    dst[s + (size_t)ns * (i + (size_t)nr * (j + (size_t)nt * (k + (size_t)ne * l)))] = src[x];
-  }
+__global__ void __launch_bounds__(256) k_f2_in(double *dst, const double *src, int ns, int nr, int nt, int ne, int npa) {
+  f2_tiles<true>(dst, src, ns, nr, nt, ne, npa);
+}
+__global__ void __launch_bounds__(256) k_f2_out(double *dst, const double *src, int ns, int nr, int nt, int ne, int npa) {
+  f2_tiles<false>(dst, src, ns, nr, nt, ne, npa);
 }
 
 // explicit instantiations used by the host code
