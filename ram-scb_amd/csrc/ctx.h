@@ -205,9 +205,10 @@ int coul_check_lds(const ramgpu_ctx *c, int threads);
 int forward_only(const ramgpu_ctx *c);
 // whether a species takes WPADIF or FLCscatter in ram_run
 int takes_pitch(const ramgpu_ctx *c);
-// Bulk copies between pageable host memory and the device, in stream order,
-// complete on return (hostio.hip); threads share one bounded ring of pinned
-// memory per process
+// Bulk copies between pageable host memory and the device, in stream order
+// (hostio.hip); threads share one bounded ring of pinned memory per process.
+// To the host it is complete on return; to the device the caller waits for the
+// stream before it gives the host array back
 int copy_to_host(int device, hipStream_t stream, void *host, const void *dev, size_t bytes);
 int copy_to_device(int device, hipStream_t stream, void *dev, const void *host, size_t bytes);
 // hipMalloc, giving the kept blocks back first when it fails

@@ -164,13 +164,14 @@ struct Transfer {
   }
 };
 
-// Synchronous copy of `bytes` in stream order; dev is a device pointer.
+// Copy of `bytes` in stream order; dev is a device pointer.
 int bulk_copy(int device, hipStream_t stream, void *host, void *dev, size_t bytes, bool to_host) {
-  const int cpus = (int)std::thread::hardware_concurrency();
-  const int threads = std::min(kMaxThreads, std::max(1, cpus / 2));
-  if (bytes >= (to_host ? kPipeMinToHost : kPipeMinToDevice) && threads > 1) {
-    std::unique_lock<std::mutex> lk(g_pipe.mu, std::try_to_lock);
-    if (lk.owns_lock() && g_pipe.ready(device)) {
+  if (bytes >= (to_host ? kPipeMinToHost : kPipeMinToDevice)) {
+    // asked for here only: the count is read from the system, 10 us
+    const int cpus = (int)std::thread::hardware_concurrency();
+    const int threads = std::min(kMaxThreads, std::max(1, cpus / 2));
+    std::unique_lock<std::mutex> lk(g_pipe.mu, std::defer_lock);
+    if (threads > 1 && lk.try_lock() && g_pipe.ready(device)) {
       // four chunks a thread, so that the last ones end together
       size_t chunk = bytes / ((size_t)threads * 4);
       chunk = std::min(kSlotBytes, std::max(size_t(512) << 10, chunk)) & ~size_t(4095);
@@ -183,8 +184,11 @@ int bulk_copy(int device, hipStream_t stream, void *host, void *dev, size_t byte
       return RAMGPU_OK;
     }
   }
-  if (to_host) HIP_TRY(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, stream));
-  else HIP_TRY(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, stream));
+  if (!to_host) {
+    HIP_TRY(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, stream));
+    return RAMGPU_OK;
+  }
+  HIP_TRY(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, stream));
   HIP_TRY(hipStreamSynchronize(stream));
   return RAMGPU_OK;
 }
