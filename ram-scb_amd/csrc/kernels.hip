@@ -566,8 +566,8 @@ __global__ void __launch_bounds__(kLineThreads, 4) k_r(Launch L) {
         gh1 = ghost_value(t, s, j, k, l, t.conf1);
         gh2 = ghost_value(t, s, j, k, l, t.conf2);
       }
-      double wsum = 0.0;  // EKEV*WE*WMU of the line in SUMRC
-      if (MODE == 2 && k >= 1 && l >= 1 && j <= NT - 2) wsum = t.ekev[k] * t.we[k] * t.wmu[l];
+      const bool sum_line = MODE == 2 && k >= 1 && l >= 1 && j <= NT - 2;
+      const double wsum = sum_line ? t.ekev[k] * t.we[k] * t.wmu[l] : 0.0;  // EKEV*WE*WMU of the line in SUMRC
       // face 1: FBND(1) = F(2) on inflow lines, 0 otherwise (:156,164)
       const double f1 = fw[0], f2v = fw[1], f3 = fw[2];
       double fnext = fw[3];  // F(4)
@@ -638,7 +638,7 @@ __global__ void __launch_bounds__(kLineThreads, 4) k_r(Launch L) {
 #undef RSTEP
 #undef RTERM
 #undef RSTERM
-      acc *= wsum;
+      acc = sum_line ? acc * wsum : 0.0;  // a line outside SUMRC leaves it alone whatever its cells hold
     }
     if (MODE == 1) {
       const double m = block_max(cmax, red);

@@ -429,16 +429,17 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step
           const double qw = (row1 || l >= NPA) ? 0.0 : ekw * lt[4 * n + 2];  // EKEV*WE*WMU
           const double wf = row1 ? 1.0 : wave;
           double x = f[n];
-          a[0] = fma(x, qw, a[0]);
+          auto in_sum = [&]() __attribute__((always_inline)) { return (X && row1) ? 0.0 : x; };
+          a[0] = fma(in_sum(), qw, a[0]);
           x = x * wf;
           x = x * cxf[g];
-          a[1] = fma(x, qw, a[1]);
+          a[1] = fma(in_sum(), qw, a[1]);
           x = x * af[g];
-          a[2] = fma(x, qw, a[2]);
+          a[2] = fma(in_sum(), qw, a[2]);
           x = x * af[g];
-          a[3] = fma(x, qw, a[3]);
+          a[3] = fma(in_sum(), qw, a[3]);
           x = x * cxf[g];
-          a[4] = fma(x, qw, a[4]);
+          a[4] = fma(in_sum(), qw, a[4]);
           f[n] = row_done(x * wf);
 #pragma unroll
           for (int m = 0; m < 5; ++m) a[m] = row_done(a[m]);
@@ -446,6 +447,9 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step
       }
       // slots: before WAVELO, after it, after CEX, ATMOL, ATMOL, CEX, after
       // WAVELO; each wave's sums in a fixed order, the waves' added up below
+      if constexpr (X)
+#pragma unroll
+        for (int m = 0; m < 5; ++m) a[m] = ekw != 0.0 ? a[m] : 0.0;
       double s7[7] = {a[0], a[0] * wave, a[1], a[2], a[3], a[4], a[4] * wave};
 #pragma unroll
       for (int m = 0; m < 7; ++m) s7[m] = wave_sum(s7[m]);
@@ -455,16 +459,19 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step
     };
 
     // ---- SEQ_STEPX: the optional processes ---------------------------------
-    // SUMRC's partial of the plane as it stands, slot m
+    // SUMRC's partial of the plane as it stands, slot m.  A cell outside the
+    // sum is left out of it, not weighed by 0: it may hold anything
     auto sum_slot = [&](int m) __attribute__((always_inline)) {
       THREAD_CELLS;
       const double ekw = sum_factor(k);
       const double *const lt = d.lt + 4 * l0;
       double a = 0.0;
 #pragma unroll
-      for (int n = 0; n < R; ++n)
-        a = fma(f[n], ((n == 0 && l0 == 0) || l0 + n >= NPA) ? 0.0 : ekw * lt[4 * n + 2], a);
-      a = wave_sum(a);
+      for (int n = 0; n < R; ++n) {
+        const bool row1 = n == 0 && l0 == 0;
+        a = fma(row1 ? 0.0 : f[n], (row1 || l0 + n >= NPA) ? 0.0 : ekw * lt[4 * n + 2], a);
+      }
+      a = wave_sum(ekw != 0.0 ? a : 0.0);
       if (lane == 63) d.red[wv * kSums + m] = a;
     };
     // The implicit pitch-angle step of every line (I,J,K>=2): the reference's
@@ -616,17 +623,17 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step
           const double af = (l + 1 >= upa) ? exp_tab(row_done(latl) * d.cf[8 * l + KLE_RHS], d.ex) : 1.0;
           const double qw = (row1 || l >= NPA) ? 0.0 : ekw * d.lt[4 * l + 2];
           double x = f[n] * af;
-          a3 = fma(x, qw, a3);
+          a3 = fma(row1 ? 0.0 : x, qw, a3);
           x = x * af;
-          a4 = row_done(fma(x, qw, a4));
+          a4 = row_done(fma(row1 ? 0.0 : x, qw, a4));
           f[n] = row_done(x);
         } else {
           f[n] = row_done(row1 ? f[n] : f[n] * wave);
         }
       }
       if (op == 1) {
-        a3 = wave_sum(a3);
-        a4 = wave_sum(a4);
+        a3 = wave_sum(ekw != 0.0 ? a3 : 0.0);
+        a4 = wave_sum(ekw != 0.0 ? a4 : 0.0);
         if (lane == 63) {
           d.red[wv * kSums + 3] = a3;
           d.red[wv * kSums + 4] = a4;
