@@ -11,8 +11,9 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -155,7 +156,7 @@ struct Transfer {
           check(hipSetDevice(device));
           work(false);
         });
-    } catch (const std::system_error &) {  // no more threads: those there, and this one, do it
+    } catch (const std::exception &) {  // no more threads, or no memory for one: those there, and this one, do it
     }
     work(true);
     for (std::thread &t : helpers) t.join();
@@ -175,13 +176,13 @@ int bulk_copy(int device, hipStream_t stream, void *host, void *dev, size_t byte
       // four chunks a thread, so that the last ones end together
       size_t chunk = bytes / ((size_t)threads * 4);
       chunk = std::min(kSlotBytes, std::max(size_t(512) << 10, chunk)) & ~size_t(4095);
-      hipError_t e;
-      {
+      try {
         Transfer t(g_pipe, device, stream, (char *)host, (char *)dev, bytes, chunk, to_host);
-        e = t.run(std::min(threads, t.n));
+        const hipError_t e = t.run(std::min(threads, t.n));
+        if (e != hipSuccess) return fail(RAMGPU_EHIP, "transfer of %zu bytes: %s", bytes, hipGetErrorString(e));
+        return RAMGPU_OK;
+      } catch (const std::bad_alloc &) {  // the transfer's own tables, before its first copy
       }
-      if (e != hipSuccess) return fail(RAMGPU_EHIP, "transfer of %zu bytes: %s", bytes, hipGetErrorString(e));
-      return RAMGPU_OK;
     }
   }
   if (!to_host) {
