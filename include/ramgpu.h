@@ -65,7 +65,12 @@ const char *ramgpu_last_error(void);
  * LDS; NT*NE*NPA and NR*NT below 2^22; and NR, NT small enough that the
  * face terms a sweep block stages in LDS fit the device (160 KB on MI355X:
  * NR <= 149 and NT <= 62 at NE = NPA = 4, NR <= 1017 and NT <= 462 at
- * 35 x 72).  Returns RAMGPU_EINVAL otherwise. */
+ * 35 x 72).  Returns RAMGPU_EINVAL otherwise.
+ * The library keeps device blocks that a call needed (tapes, schedules,
+ * computehI's workspace) for later calls: 4 GiB per process at most, the
+ * latest ones, given back before an allocation of this library fails and when
+ * the process's last context is destroyed.  Device memory that other
+ * libraries of the process find free is less by that much. */
 int ramgpu_create(ramgpu_ctx **ctx, int ns, int nr, int nt, int ne, int npa, int device);
 int ramgpu_destroy(ramgpu_ctx *ctx);
 

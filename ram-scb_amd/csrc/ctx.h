@@ -215,8 +215,8 @@ int copy_to_device(int device, hipStream_t stream, void *dev, const void *host, 
 bool dev_malloc(int device, void **p, size_t bytes);
 // A device block of exactly `bytes` for the length of a call: one kept from an
 // earlier call or a new one; given back (its device work done) it is kept for
-// a later call, 4 GiB per process at most, until the last context goes or an
-// allocation needs the room
+// a later call, the latest 4 GiB per process at most, until the last context
+// goes or an allocation needs the room
 bool dev_take(int device, void **p, size_t bytes);
 void dev_give(int device, void *p, size_t bytes);
 size_t dev_cached(int device);

@@ -82,7 +82,7 @@ struct Block {
   void *p;
 };
 std::mutex g_cache_mu;
-std::vector<Block> g_cache;
+std::vector<Block> g_cache;  // in the order they were given back
 size_t g_cached = 0;
 
 // One transfer through the ring (mu held).  Chunk i uses slot i mod kSlots.
@@ -194,17 +194,21 @@ int bulk_copy(int device, hipStream_t stream, void *host, void *dev, size_t byte
   return RAMGPU_OK;
 }
 
+// with g_cache_mu held: kept block i out of the list
+Block unkeep_locked(size_t i) {
+  const Block b = g_cache[i];
+  g_cache.erase(g_cache.begin() + i);
+  g_cached -= b.bytes;
+  return b;
+}
+
 // with g_cache_mu held
 void trim_locked(int device) {
   for (size_t i = 0; i < g_cache.size();) {
-    if (device >= 0 && g_cache[i].device != device) {
+    if (device < 0 || g_cache[i].device == device)
+      (void)hipFree(unkeep_locked(i).p);
+    else
       ++i;
-      continue;
-    }
-    (void)hipFree(g_cache[i].p);
-    g_cached -= g_cache[i].bytes;
-    g_cache[i] = g_cache.back();
-    g_cache.pop_back();
   }
 }
 
@@ -237,10 +241,7 @@ bool dev_take(int device, void **p, size_t bytes) {
     std::lock_guard<std::mutex> lk(g_cache_mu);
     for (size_t i = 0; i < g_cache.size(); ++i)
       if (g_cache[i].device == device && g_cache[i].bytes == bytes) {
-        *p = g_cache[i].p;
-        g_cached -= bytes;
-        g_cache[i] = g_cache.back();
-        g_cache.pop_back();
+        *p = unkeep_locked(i).p;
         return true;
       }
   }
@@ -249,7 +250,9 @@ bool dev_take(int device, void **p, size_t bytes) {
 
 void dev_give(int device, void *p, size_t bytes) {
   std::lock_guard<std::mutex> lk(g_cache_mu);
-  if (g_cached + bytes <= kCacheMax) {
+  if (bytes <= kCacheMax) {
+    // the oldest make room: a size that is no longer asked for leaves in time
+    while (g_cached + bytes > kCacheMax) (void)hipFree(unkeep_locked(0).p);
     try {
       g_cache.push_back({device, bytes, p});
       g_cached += bytes;

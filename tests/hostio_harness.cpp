@@ -14,6 +14,7 @@
 #include "ctx.h"
 
 static std::atomic<long> g_news_left{-1};  // allocations that still succeed (< 0: all)
+static std::atomic<long> g_mallocs{0}, g_frees{0};
 
 static void *counted(size_t n) {
   if (g_news_left.load() >= 0 && g_news_left.fetch_sub(1) <= 0) {
@@ -32,10 +33,12 @@ void operator delete[](void *p, size_t) noexcept { std::free(p); }
 
 extern "C" {
 hipError_t hipMalloc(void **p, size_t) {
+  ++g_mallocs;
   *p = std::malloc(1);
   return hipSuccess;
 }
 hipError_t hipFree(void *p) {
+  ++g_frees;
   std::free(p);
   return hipSuccess;
 }
@@ -104,7 +107,32 @@ static int no_memory() {
   return 0;
 }
 
+// kept blocks: those of sizes no longer asked for make room for the latest
+static int kept_blocks() {
+  const size_t MB = size_t(1) << 20;
+  void *p[8], *q;
+  for (int i = 0; i < 8; ++i) EXPECT(dev_take(0, &p[i], (900 + i) * MB));
+  for (int i = 0; i < 8; ++i) dev_give(0, p[i], (900 + i) * MB);
+  EXPECT(dev_cached(0) <= 4096 * MB);
+  long m = g_mallocs;
+  for (int i = 4; i < 8; ++i) EXPECT(dev_take(0, &p[i], (900 + i) * MB));  // the last four given
+  EXPECT(g_mallocs == m && dev_cached(0) == 0);
+  for (int i = 4; i < 8; ++i) dev_give(0, p[i], (900 + i) * MB);
+  EXPECT(dev_take(0, &q, 5000 * MB));  // more than is ever kept: the others stay
+  dev_give(0, q, 5000 * MB);
+  EXPECT(dev_cached(0) == (904 + 905 + 906 + 907) * MB);
+  EXPECT(dev_take(1, &q, 907 * MB));  // another device's block is not this one's
+  EXPECT(dev_cached(0) == (904 + 905 + 906 + 907) * MB);
+  dev_give(1, q, 907 * MB);
+  EXPECT(dev_cached(0) + dev_cached(1) <= 4096 * MB && dev_cached(1) == 907 * MB);
+  context_opened();
+  context_closed();
+  EXPECT(dev_cached(0) == 0 && dev_cached(1) == 0 && g_mallocs == g_frees);
+  return 0;
+}
+
 int main(int argc, char **argv) {
   if (argc > 1 && !std::strcmp(argv[1], "no_memory")) return no_memory();
+  if (argc > 1 && !std::strcmp(argv[1], "kept_blocks")) return kept_blocks();
   return 2;
 }

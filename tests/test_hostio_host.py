@@ -1,6 +1,8 @@
-"""The host side of bulk transfers (csrc/hostio.hip), run without a device:
-hostio_harness.cpp stands in for the HIP calls.  no_memory: a transfer that
-cannot allocate still moves the data, with no exception out of the C ABI."""
+"""The host side of bulk transfers and kept device blocks (csrc/hostio.hip),
+run without a device: hostio_harness.cpp stands in for the HIP calls.
+no_memory: a transfer that cannot allocate still moves the data, with no
+exception out of the C ABI.  kept_blocks: at most 4 GiB stay, the blocks given
+back last, and all go with the last context."""
 import shutil
 import subprocess
 from pathlib import Path
@@ -30,7 +32,7 @@ def harness(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["no_memory"])
+@pytest.mark.parametrize("check", ["no_memory", "kept_blocks"])
 def test_hostio(harness, check):
     r = subprocess.run([str(harness), check], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, f"{r.returncode}: {r.stdout}{r.stderr}"
