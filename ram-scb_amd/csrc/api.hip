@@ -1215,8 +1215,8 @@ int ramgpu_copy_probe(int device, size_t bytes, int reps, double *gbps) {
   HIP_TRY(hipSetDevice(device));
   const size_t n2 = bytes / 16;
   double2 *a = nullptr, *b = nullptr;
-  HIP_TRY(hipMalloc(&a, n2 * 16));
-  if (hipMalloc(&b, n2 * 16) != hipSuccess) {
+  if (!dev_malloc(device, (void **)&a, n2 * 16)) return fail(RAMGPU_EHIP, "copy probe: hipMalloc of %zu bytes failed", n2 * 16);
+  if (!dev_malloc(device, (void **)&b, n2 * 16)) {
     (void)hipFree(a);
     return fail(RAMGPU_ENOMEM, "copy probe allocation failed");
   }
