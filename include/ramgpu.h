@@ -399,6 +399,11 @@ int ramgpu_ram_run_bwd(ramgpu_ctx *ctx, double *adj, double *fgeos_adj);
 int ramgpu_adjoint_run(ramgpu_ctx *ctx, int nsteps, int ckpt_every, const double *kp,
                        const double *bscale, int npts, const int *pts, const double *w,
                        const double *target, double *loss, double *grad_f2, double *grad_fgeos);
+/* The same with grad_fgeos in C's order, [nsteps][NS][NT][NE][NPA] with NPA
+ * contiguous (reordered on the device), for hosts whose arrays are. */
+int ramgpu_adjoint_run_rows(ramgpu_ctx *ctx, int nsteps, int ckpt_every, const double *kp,
+                            const double *bscale, int npts, const int *pts, const double *w,
+                            const double *target, double *loss, double *grad_f2, double *grad_fgeos);
 
 /* ---- ensembles ------------------------------------------------------- */
 

@@ -718,6 +718,38 @@ __global__ void k_misfit_ens(Launch L, int step, int adjoint) {
   }
 }
 
+// n arrays (NS,NT,NE,NPA) from Fortran's order to C's: of one array the
+// columns (S,J,K), contiguous in src for each L, become rows of NPA, placed by
+// S, J, K.  Bound by memory; 64x32 tiles through LDS, so that both sides move
+// whole runs (30 of 1x25x35x72, 15 MB, in two launches: 24 us, where NumPy took
+// 8 ms on the host).
+__global__ void __launch_bounds__(256) k_fgeos_rows(double *__restrict__ dst, const double *__restrict__ src, int n, int ns,
+                                                    int nt, int ne, int npa) {
+  constexpr int TC = 64, TL = 32;
+  __shared__ double tile[TC * (TL + 1)];
+  const int cols = ns * nt * ne, nct = (cols + TC - 1) / TC, nlt = (npa + TL - 1) / TL;
+  const size_t ng = (size_t)cols * npa, units = (size_t)n * nct * nlt;
+  for (size_t u = blockIdx.x; u < units; u += gridDim.x) {
+    const size_t a = u / ((size_t)nct * nlt);
+    const int r = (int)(u - a * ((size_t)nct * nlt)), ct = r / nlt, c0 = ct * TC, l0 = (r - ct * nlt) * TL;
+    const double *const x = src + a * ng;
+    double *const y = dst + a * ng;
+    for (int e = threadIdx.x; e < TC * TL; e += 256) {
+      const int c = e & (TC - 1), l = e / TC;
+      if (c0 + c < cols && l0 + l < npa) tile[c * (TL + 1) + l] = x[(size_t)(l0 + l) * cols + c0 + c];
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < TC * TL; e += 256) {
+      const int l = e & (TL - 1), c = e / TL, col = c0 + c;
+      if (col < cols && l0 + l < npa) {
+        const int q = col / ns, s = col - q * ns, k = q / nt, j = q - k * nt;
+        y[((size_t)(s * nt + j) * ne + k) * npa + l0 + l] = tile[c * (TL + 1) + l];
+      }
+    }
+    __syncthreads();  // the tile is read
+  }
+}
+
 // y += a*x (n doubles)
 __global__ void k_axpy(double *y, const double *x, double a, size_t n) {
   for (size_t m = blockIdx.x * (size_t)blockDim.x + threadIdx.x; m < n; m += (size_t)gridDim.x * blockDim.x)

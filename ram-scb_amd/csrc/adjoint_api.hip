@@ -361,9 +361,29 @@ int ramgpu_ram_run_bwd(ramgpu_ctx *c, double *adj, double *fgeos_adj) {
   return RAMGPU_OK;
 }
 
-int ramgpu_adjoint_run(ramgpu_ctx *c, int nsteps, int ckpt_every, const double *kp, const double *bscale,
-                       int npts, const int *pts, const double *w, const double *target, double *loss,
-                       double *grad_f2, double *grad_fgeos) {
+}  // extern "C"
+
+namespace {
+
+// the nsteps adjoints of FGEOS at bbar to the host, each array in C's order:
+// NR of them at a time through the context's stage (NR of FGEOS's size)
+int download_fgeos_rows(ramgpu_ctx *c, double *host, const double *bbar, int nsteps) {
+  const size_t ng = nfg(c);
+  for (int n0 = 0; n0 < nsteps; n0 += c->nr) {
+    const int m = std::min(c->nr, nsteps - n0);
+    hipLaunchKernelGGL(k_fgeos_rows, dim3(2048), dim3(256), 0, c->stream, c->d_stage, bbar + (size_t)n0 * ng, m, c->ns,
+                       c->nt, c->ne, c->npa);
+    int rc = launch_check("k_fgeos_rows");
+    if (rc || (rc = copy_to_host(c->device, c->stream, host + (size_t)n0 * ng, c->d_stage, (size_t)m * ng * sizeof(double))))
+      return rc;
+  }
+  return RAMGPU_OK;
+}
+
+// rows: grad_fgeos in C's order (ramgpu_adjoint_run_rows)
+int adjoint_run(ramgpu_ctx *c, int nsteps, int ckpt_every, const double *kp, const double *bscale,
+                int npts, const int *pts, const double *w, const double *target, double *loss,
+                double *grad_f2, double *grad_fgeos, bool rows) {
   int rc = check_ctx(c);
   if (rc || (rc = ready(c)) || (rc = forward_only(c))) return rc;
   if (nsteps < 1 || ckpt_every < 1) return fail(RAMGPU_EINVAL, "nsteps and ckpt_every must be >= 1");
@@ -524,9 +544,26 @@ int ramgpu_adjoint_run(ramgpu_ctx *c, int nsteps, int ckpt_every, const double *
   }
   if (grad_f2 && (rc = download_f2(c, grad_f2, lam))) return rc;
   if (grad_fgeos) {
+    if (rows) return download_fgeos_rows(c, grad_fgeos, bbar, nsteps);
     if ((rc = copy_to_host(c->device, c->stream, grad_fgeos, bbar, (size_t)nsteps * ng * sizeof(double)))) return rc;
   }
   return RAMGPU_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int ramgpu_adjoint_run(ramgpu_ctx *c, int nsteps, int ckpt_every, const double *kp, const double *bscale,
+                       int npts, const int *pts, const double *w, const double *target, double *loss,
+                       double *grad_f2, double *grad_fgeos) {
+  return adjoint_run(c, nsteps, ckpt_every, kp, bscale, npts, pts, w, target, loss, grad_f2, grad_fgeos, false);
+}
+
+int ramgpu_adjoint_run_rows(ramgpu_ctx *c, int nsteps, int ckpt_every, const double *kp, const double *bscale,
+                            int npts, const int *pts, const double *w, const double *target, double *loss,
+                            double *grad_f2, double *grad_fgeos) {
+  return adjoint_run(c, nsteps, ckpt_every, kp, bscale, npts, pts, w, target, loss, grad_f2, grad_fgeos, true);
 }
 
 }  // extern "C"

@@ -25,6 +25,7 @@ template <int R> __global__ void k_plane_adj(Launch L, const double *xin, double
 __global__ void k_misfit(const double *f2, int nr, int nt, int ne, int npa, int npts, const int *pts,
                          const double *w, const double *target, double *loss_out, double *lam);
 __global__ void k_misfit_ens(Launch L, int step, int adjoint);
+__global__ void k_fgeos_rows(double *dst, const double *src, int n, int ns, int nt, int ne, int npa);
 __global__ void k_axpy(double *y, const double *x, double a, size_t n);
 __global__ void k_fill(double *y, double v, size_t n);
 __global__ void k_species(Launch L);

@@ -33,6 +33,7 @@ EXPORTS = (
     "ramgpu_batch_autotune", "ramgpu_batch_get_shapes", "ramgpu_batch_set_shapes",
     "ramgpu_driftr_bwd", "ramgpu_driftp_bwd", "ramgpu_drifte_bwd", "ramgpu_driftmu_bwd",
     "ramgpu_charexchange_bwd", "ramgpu_atmol_bwd", "ramgpu_ram_run_bwd", "ramgpu_adjoint_run",
+    "ramgpu_adjoint_run_rows",
     "ramgpu_batch_adjoint_run", "ramgpu_set_plane_shape", "ramgpu_get_plane_shape",
     "ramgpu_set_moment_factors", "ramgpu_anisch", "ramgpu_flux", "ramgpu_moments",
     "ramgpu_ram_run_schedule_noalloc", "ramgpu_set_loss_state", "ramgpu_get_loss_state",
@@ -143,8 +144,8 @@ def load_library(path: Path | None = None):
     for n in ("driftp", "drifte", "driftmu", "charexchange", "atmol"):
         getattr(lib, f"ramgpu_{n}_bwd").argtypes = [v, C.c_int, _dp]
     lib.ramgpu_ram_run_bwd.argtypes = [v, _dp, _dp]
-    lib.ramgpu_adjoint_run.argtypes = [v, C.c_int, C.c_int, _dp, _dp, C.c_int, _ip, _dp, _dp, _dp,
-                                       _dp, _dp]
+    for n in ("ramgpu_adjoint_run", "ramgpu_adjoint_run_rows"):
+        getattr(lib, n).argtypes = [v, C.c_int, C.c_int, _dp, _dp, C.c_int, _ip, _dp, _dp, _dp, _dp, _dp]
     lib.ramgpu_set_plane_shape.argtypes = [v, C.c_int, C.c_int]
     lib.ramgpu_get_plane_shape.argtypes = [v, _ip, _ip]
     _pp = C.POINTER(C.c_void_p)
@@ -533,7 +534,8 @@ class RamGpu:
     def adjoint_run(self, nsteps, pts, w, target, ckpt_every=10, kp=None, bscale=None):
         """Loss and gradients of the virtual-satellite misfit over nsteps.
         pts: (npts,4) 1-based S,I,J,K; w: (npts,NPA); target: (nsteps,npts).
-        Returns (loss, dL/dF2_0 (NS,NR,NT,NE,NPA), dL/dFGEOS (nsteps,NS,NT,NE,NPA))."""
+        Returns (loss, dL/dF2_0 (NS,NR,NT,NE,NPA) in Fortran order, dL/dFGEOS
+        (nsteps,NS,NT,NE,NPA) in C order)."""
         pts = np.ascontiguousarray(pts, dtype=np.int32)
         npts = pts.shape[0]
         w = np.ascontiguousarray(w, dtype=np.float64)
@@ -548,11 +550,11 @@ class RamGpu:
             raise ValueError("bscale must have nsteps*NS entries")
         loss = C.c_double(0.0)
         gf = np.zeros(self.dims, order="F")
-        gbf = np.zeros(nsteps * self.ns * self.nt * self.ne * self.npa)
-        self._check(self.lib.ramgpu_adjoint_run(
+        gb = np.zeros((nsteps, self.ns, self.nt, self.ne, self.npa))
+        self._check(self.lib.ramgpu_adjoint_run_rows(
             self.h, nsteps, ckpt_every, None if kpa is None else _p(kpa), None if bsa is None else _p(bsa),
-            npts, pts.ctypes.data_as(_ip), _p(w), _p(target), C.byref(loss), _p(gf), _p(gbf)))
-        return loss.value, gf, _per_step(gbf, nsteps, self)
+            npts, pts.ctypes.data_as(_ip), _p(w), _p(target), C.byref(loss), _p(gf), _p(gb)))
+        return loss.value, gf, gb
 
     def set_plane_shape(self, threads=0, maxc=0):
         """Block size and row bound of the plane kernels (0, 0: the library's choice)."""
@@ -673,7 +675,8 @@ class RamBatch:
         """Misfit losses and gradients of every member (ramgpu_batch_adjoint_run).
         pts[m]: (npts_m,4) 1-based S,I,J,K; w[m]: (npts_m,NPA_m); target[m]:
         (nsteps,npts_m); kp: (nsteps, M); bscale: (nsteps, sum NS) or None.
-        Returns (loss[M], [dL/dF2_0 per member], [dL/dFGEOS (nsteps,NS,NT,NE,NPA) per member or None])."""
+        Returns (loss[M], [dL/dF2_0 per member], [dL/dFGEOS (nsteps,NS,NT,NE,NPA) per member or None],
+        each step's array in Fortran order)."""
         M = len(self.members)
         kp = np.ascontiguousarray(kp, dtype=np.float64)
         if kp.shape != (nsteps, M):
