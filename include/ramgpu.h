@@ -411,9 +411,10 @@ int ramgpu_adjoint_run_rows(ramgpu_ctx *ctx, int nsteps, int ckpt_every, const d
  * reference, which runs one problem per process: it serves ensemble
  * forecasts and ensemble data assimilation).  Members are contexts created
  * on one device, each with its own grid sizes, species, fields and F2; the
- * ensemble does not own them and must be destroyed before them.  Every kernel
- * of a step is one launch over all members, and a step is one captured HIP
- * graph, replayed per step.  A member's results are bit-identical to those
+ * ensemble does not own them and must be destroyed before them.  A kernel
+ * of a step is one launch over all members (one per shape of its members'
+ * kernels where these are large), and a step is one captured HIP graph,
+ * replayed per step.  A member's results are bit-identical to those
  * of stepping it alone with ramgpu_ram_run / ramgpu_ram_run_schedule. */
 typedef struct ramgpu_batch ramgpu_batch;
 int ramgpu_batch_create(ramgpu_batch **batch, ramgpu_ctx *const *members, int nmembers);
@@ -447,7 +448,7 @@ int ramgpu_batch_autotune(ramgpu_batch *batch, int reps, double *ms_best /* [3] 
 int ramgpu_batch_get_shapes(ramgpu_batch *batch, int *caps /* [3] */);
 int ramgpu_batch_set_shapes(ramgpu_batch *batch, const int *caps /* [3] */);
 /* Reverse mode of an ensemble: ramgpu_adjoint_run for every member at once
- * (each kernel one launch over all members), from the members' current F2,
+ * (all members in the same launches), from the members' current F2,
  * with the per-member schedule of ramgpu_batch_ram_run_schedule (kp
  * required, bscale may be NULL).  Member m has npts[m] misfit points
  * pts[m][4p..4p+3], weights w[m][p*NPA_m + L-1] and targets

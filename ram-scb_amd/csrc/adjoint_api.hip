@@ -46,9 +46,6 @@ void launch_plane_bwd_t(int seq, dim3 grid, size_t lds, hipStream_t st, const La
   }
 }
 
-// Rows per thread the step's plane adjoint is built for.
-#define ADJ_ROWS(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12)
-
 // Rows per thread of the step's plane adjoint: step_shape's rule with its own
 // threads and LDS (MI355X, us by rows: 475 planes of 35x72 4: 52, 5: 59, 6: 44,
 // 8: 54, 9: 53, 12: 51).
@@ -77,6 +74,7 @@ void launch_plane_adj(StepShape sh, dim3 grid, size_t lds, hipStream_t st, const
   case r: hipLaunchKernelGGL((k_plane_adj<r>), grid, blk, lds, st, L, x, adj); break;
     ADJ_ROWS(ROWS)
 #undef ROWS
+    default: hipLaunchKernelGGL(k_plane_adj_mixed, grid, blk, lds, st, L);  // kMixedRows
   }
 }
 
@@ -85,6 +83,7 @@ void set_plane_bwd_lds_limit(size_t limit) {
   (void)hipFuncSetAttribute((const void *)k_plane_adj<r>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)limit);
   ADJ_ROWS(ADJ_K)
 #undef ADJ_K
+  (void)hipFuncSetAttribute((const void *)k_plane_adj_mixed, hipFuncAttributeMaxDynamicSharedMemorySize, (int)limit);
   set_bwd_lds_limit_t<kPlaneThreads>(limit);
   set_bwd_lds_limit_t<kPlaneMaxThreads>(limit);
 }

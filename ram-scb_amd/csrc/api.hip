@@ -385,9 +385,6 @@ void launch_plane(int seq, PlaneShape sh, dim3 grid, size_t lds, hipStream_t st,
     launch_plane_t<16>(seq, sh.threads, grid, lds, st, L, rec);
 }
 
-// Rows per thread the fused step's plane kernel is built for.
-#define STEP_ROWS(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16)
-
 // Rows per thread of the fused step's plane kernel, a function of NE, NPA and
 // the problem's planes per CU.
 // A plane's cost is the rows that its busiest SIMD sweeps, set-up counting as
@@ -435,6 +432,9 @@ void launch_step(int seq, StepShape sh, dim3 grid, size_t lds, hipStream_t st, c
     break;
     STEP_ROWS(ROWS)
 #undef ROWS
+    default:  // kMixedRows
+      if (seq == SEQ_TAPE) hipLaunchKernelGGL(k_plane_mixed<SEQ_TAPE>, grid, blk, lds, st, L, rec);
+      else hipLaunchKernelGGL(k_plane_mixed<SEQ_STEP>, grid, blk, lds, st, L, rec);
   }
 }
 
@@ -523,6 +523,7 @@ int set_plane_lds_limit(size_t limit) {
       (const void *)k_plane_step<SEQ_STEPX, r>,
       STEP_ROWS(STEP_K)
 #undef STEP_K
+      (const void *)k_plane_mixed<SEQ_STEP>, (const void *)k_plane_mixed<SEQ_TAPE>,
       (const void *)k_p_bwd, (const void *)k_pitch_diffusion};
 #undef PLANE_K
   for (const void *f : fns) {

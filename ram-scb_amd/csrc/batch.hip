@@ -1,10 +1,11 @@
 // batch.hip -- ensembles: many independent problems stepped together.
 //
 // The members are ordinary contexts on one device, each with its own grid
-// sizes, species, fields and F2.  Every kernel of the split step is ONE
-// launch over all members: a job table lists (member, species, first block)
-// units and a per-block map sends each virtual block to its unit, so members
-// of different sizes share a grid.  The launches of one step are captured
+// sizes, species, fields and F2.  A kernel of the split step is one launch
+// over all members, or one per shape of its members' kernels where these are
+// many blocks each (mixed_launch): a job table lists (member, species, first
+// block) units and a per-block map sends each virtual block to its unit, so
+// members of different sizes share a grid.  The launches of one step are captured
 // once into a HIP graph and replayed per step; the Kp / boundary-scale
 // schedule is read on the device through a step counter, so every replay is
 // the same graph.  An autotuner picks, per kernel, how many resident blocks
@@ -18,6 +19,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <numeric>
+#include <set>
 #include <utility>
 #include <vector>
 
@@ -41,9 +43,10 @@ struct Plan {
   int *vmap = nullptr;
   int nv = 0;
   int cap = 0;  // 0: one block per virtual block; else the persistent grid size
-  // sweep and plane kinds: one launch per shape of the members' kernels,
-  // over the virtual blocks [v0, v0 + nv) of its members; a sweep's shape is
-  // its rows (0: one thread per line) and the line's cells' chunks
+  // sweep and plane kinds: the launches, each over the virtual blocks
+  // [v0, v0 + nv) of its members: one per shape of the members' kernels (a
+  // sweep's is its rows, 0 being one thread per line, and its block), or one
+  // with every member's own rows (kMixedRows) where that is faster (mixed_launch)
   struct Group {
     StepShape sh;
     size_t lds;
@@ -114,8 +117,19 @@ int blocks_of(const ramgpu_batch *b, int kind, const ramgpu_ctx *c) {
 
 bool per_member(int kind) { return kind == BK_SCHED || kind == BK_COEFIJ || kind == BK_MEM || kind == BK_COPY; }
 
+// Whether members of several kernel shapes go in one launch, each with the
+// rows it has alone, in blocks of the widest (the waves a member does not need
+// only meet its barriers).  A launch per shape leaves CUs idle and pays its
+// latency while it has few blocks; with many, the wide blocks cost more.  A
+// step of uneven ensembles on MI355X in us, per shape / mixed (in brackets the
+// planes per shape and CU): 4 members up to 14x15x19x41 143 / 86 (0.9), 8 up to
+// 24x25x29x61 326 / 238 (1.7), 4 up to 40x41x45x90 380 / 349 (4.8), 32 up to
+// 38x39x43x89 1243 / 1232 (4.4), 64 up to 30x31x35x73 1691 / 1728 (6.2), 64 up to
+// 41x42x46x90 3653 / 4062 (12.7).
+bool mixed_launch(size_t shapes, long units, int ncu) { return shapes > 1 && units <= 4L * ncu * (long)shapes; }
+
 // Job table and block map of one kernel kind, members in order; the sweep
-// and plane kinds with the members of one kernel shape together.
+// and plane kinds with the members of one launch together.
 int build_plan(ramgpu_batch *b, int kind) {
   std::vector<Job> jobs;
   std::vector<int> vmap;
@@ -136,10 +150,24 @@ int build_plan(ramgpu_batch *b, int kind) {
     *lds = h.lds;
     return StepShape{h.threads, h.rows};
   };
-  auto shape = [&](size_t mi) {
+  auto own_shape = [&](size_t mi) {
     size_t lds;
     const StepShape h = shape_of(b->m[mi], &lds);
     return std::make_pair(h.rows, h.threads);
+  };
+  std::set<std::pair<int, int>> shapes;
+  long units = 0;
+  int wide = 0;
+  for (size_t mi : order)
+    if (grouped && own_shape(mi).first != 0) {
+      shapes.insert(own_shape(mi));
+      units += (long)b->m[mi]->ns * blocks_of(b, kind, b->m[mi]);
+      wide = std::max(wide, own_shape(mi).second);
+    }
+  const bool mixed = grouped && mixed_launch(shapes.size(), units, b->ncu);
+  auto shape = [&](size_t mi) {
+    const std::pair<int, int> h = own_shape(mi);
+    return (mixed && h.first != 0) ? std::make_pair(kMixedRows, wide) : h;
   };
   if (grouped)
     std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) { return shape(x) < shape(y); });
@@ -147,10 +175,13 @@ int build_plan(ramgpu_batch *b, int kind) {
   for (size_t o = 0; o < order.size(); ++o) {
     const size_t mi = order[o];
     const ramgpu_ctx *c = b->m[mi];
+    int rows = 0;
     if (grouped) {
       size_t lds = 0;
-      const StepShape sh = shape_of(c, &lds);
-      if (o == 0 || shape(order[o - 1]) != shape(mi)) groups.push_back(Plan::Group{sh, 0, (int)vmap.size(), 0});
+      rows = shape_of(c, &lds).rows;
+      const std::pair<int, int> h = shape(mi);
+      if (o == 0 || shape(order[o - 1]) != h)
+        groups.push_back(Plan::Group{StepShape{h.second, h.first}, 0, (int)vmap.size(), 0});
       groups.back().lds = std::max(groups.back().lds, lds);
     }
     const int nsp = per_member(kind) ? 1 : c->ns;
@@ -158,7 +189,7 @@ int build_plan(ramgpu_batch *b, int kind) {
     if (nb >= (1 << kVmapShift) || jobs.size() + nsp >= (1u << (31 - kVmapShift)))
       return fail(RAMGPU_EINVAL, "ensemble too large for the launch tables");
     const int j0 = (int)jobs.size();
-    for (int s = 0; s < nsp; ++s) jobs.push_back(Job{(int)mi, s, (int)vmap.size(), nb});
+    for (int s = 0; s < nsp; ++s) jobs.push_back(Job{(int)mi, s, (int)vmap.size(), nb, rows});
     if (kind == BK_PLANE || kind == BK_PLB) {
       // the species of each run of 8 planes in turn: a plane's species land
       // on one XCD, whose L2 serves them the plane's tables (Launch::ilv)
@@ -198,7 +229,7 @@ unsigned grid_for(const ramgpu_batch *b, int kind) {
   return (unsigned)((p.cap > 0 && p.cap < p.nv) ? p.cap : p.nv);
 }
 
-// The fused plane kernel of every member: one launch per shape.
+// The fused plane kernel of every member.
 void enq_planes(ramgpu_batch *b, int kind, int seq, Launch L, int rec) {
   const Plan &p = b->plan[kind];
   const int *vmap = L.vmap;
@@ -210,8 +241,8 @@ void enq_planes(ramgpu_batch *b, int kind, int seq, Launch L, int rec) {
   }
 }
 
-// DRIFTR or DRIFTP (kind BK_P or BK_POOP) of every member: one launch per
-// shape.  L: the launch's slots.
+// DRIFTR or DRIFTP (kind BK_P or BK_POOP) of every member.  L: the launch's
+// slots.
 void enq_lines(ramgpu_batch *b, int kind, Launch L, int mode) {
   const Plan &p = b->plan[kind];
   L.jobs = p.jobs;

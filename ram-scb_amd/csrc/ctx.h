@@ -22,6 +22,7 @@ template <int FINAL> __global__ void k_r_bwd(Launch L, const double *xin, double
 __global__ void k_p_bwd(Launch L, const double *xin, double *adj);
 template <int SEQ, int BT> __global__ void k_plane_bwd(Launch L, const double *xin, double *adj);
 template <int R> __global__ void k_plane_adj(Launch L, const double *xin, double *adj);
+__global__ void k_plane_adj_mixed(Launch L);
 __global__ void k_misfit(const double *f2, int nr, int nt, int ne, int npa, int npts, const int *pts,
                          const double *w, const double *target, double *loss_out, double *lam);
 __global__ void k_misfit_ens(Launch L, int step, int adjoint);
@@ -40,6 +41,7 @@ template <int MODE, int R> __global__ void k_r_rows(Launch L);
 template <int MODE, int R> __global__ void k_p_rows(Launch L);
 template <int SEQ, int MAXC> __global__ void k_plane(Launch L, int rec);
 template <int SEQ, int R> __global__ void k_plane_step(Launch L, int rec);
+template <int SEQ> __global__ void k_plane_mixed(Launch L, int rec);
 __global__ void k_finalize(Launch L, int cflmask, int summode);
 __global__ void k_vs(double *vt, const double *lz, const double *phi, const double *kp_ptr,
                      double kp_val, int nr1, int nt, const double *bs_src, double *bs_dst, int ns);
@@ -48,6 +50,9 @@ __global__ void k_f2_in(double *dst, const double *src, int ns, int nr, int nt, 
 __global__ void k_f2_out(double *dst, const double *src, int ns, int nr, int nt, int ne, int npa);
 }  // namespace ramgpu
 
+// Rows per thread the fused step's plane kernel and its adjoint are built for.
+#define STEP_ROWS(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16)
+#define ADJ_ROWS(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12)
 
 using ramgpu::Tab;
 using ramgpu::kMaxSpecies;

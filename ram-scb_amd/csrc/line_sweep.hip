@@ -45,30 +45,34 @@ __device__ __forceinline__ void line_max(double m, double *red, int w, int lane,
   }
 }
 
-}  // namespace
+// the barriers of a unit, for the waves of a mixed launch's block that its
+// lines do not need
+__device__ __forceinline__ void line_barriers(int n) {
+  for (int x = 0; x < n; ++x) __syncthreads();
+}
 
 // MODE 0: sweep; 1: sweep and record the CFL maximum; 2: the last sweep of
 // ram_run: also the SUMRC partial sum of src/ModRamRun.f90:246-255, then
 // F2(:,:,NT)=F2(:,:,1) and the magnetopause mask (:186,197-201).  In mode 2
 // the J=NT lines are not swept: the seam overwrites them with the lines J=1,
 // whose threads store both.
-template <int MODE, int R>
-__global__ void __launch_bounds__(1024, line_simd_waves(R)) k_r_rows(Launch L) {
-  extern __shared__ double sm[];
-  for (int vb = blockIdx.x; vb < L.nv; vb += gridDim.x) {
-    const CUnit u = const_unit(L, vb);
+// MIXED: the block may have more waves than the line has chunks.
+template <int MODE, int R, bool MIXED>
+__device__ __forceinline__ void r_rows_unit(const Launch &L, const CUnit &u, double *sm) {
+  {
     CTab &t = *u.t;
     fetched(t.nr, t.nt, t.ne, t.npa, t.ns, t.rne, t.f2, t.tape, t.q1, t.p4, t.rij, t.rsi, t.betalim,
             t.fgeos, t.fnhs, t.bscale, t.conf1, t.conf2, (int)blockDim.x);
     const int s = u.s, NR = t.nr, NT = t.nt, NE = t.ne, P = NE * t.npa;
-    const int G = (P + 63) >> 6, Q = blockDim.x >> 6;
+    const int G = (P + 63) >> 6, Q = MIXED ? line_chunks(NR, R) : blockDim.x >> 6;
     const int j = u.b / G, q0 = (u.b - j * G) * 64;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const LineLds d = line_lds(sm, Q);
     if (MODE == 2 && j == NT - 1) {
       if (threadIdx.x == 0) t.partials[((size_t)kSumRadial * t.ns + s) * t.maxblk + u.b] = 0.0;
-      continue;
+      return;
     }
+    if (MIXED && w >= Q) return line_barriers(MODE == 0 ? 2 : 3);
     const int i0 = w * R;
     const bool act = q0 + lane < P;
     const int q = min(q0 + lane, P - 1);
@@ -215,24 +219,23 @@ __global__ void __launch_bounds__(1024, line_simd_waves(R)) k_r_rows(Launch L) {
 // but for the face J=NT-1 upwinded from above, whose N-1 is 1 (:250-251); the
 // flux of face NT is also face 1's (:261-262); F2(I,1) = F2(I,NT) (:272).
 // MODE 0: sweep; 1: sweep and record the CFL maximum.
-template <int MODE, int R>
-__global__ void __launch_bounds__(1024, line_simd_waves(R)) k_p_rows(Launch L) {
-  extern __shared__ double sm[];
-  for (int vb = blockIdx.x; vb < L.nv; vb += gridDim.x) {
-    const CUnit u = const_unit(L, vb);
+template <int MODE, int R, bool MIXED>
+__device__ __forceinline__ void p_rows_unit(const Launch &L, const CUnit &u, double *sm) {
+  {
     CTab &t = *u.t;
     fetched(t.nr, t.nt, t.ne, t.npa, t.ns, t.rne, t.f2, t.tape, t.pl, t.p2, t.pij, t.betalim, t.omet,
             (int)blockDim.x);
     const int s = u.s, NR = t.nr, NT = t.nt, NE = t.ne, P = NE * t.npa;
-    const int G = (P + 63) >> 6, Q = blockDim.x >> 6;
+    const int G = (P + 63) >> 6, Q = MIXED ? line_chunks(NT, R) : blockDim.x >> 6;
     const size_t so = (size_t)s * f2_species_stride(t);
     if (u.b >= (NR - 1) * G) {  // out of place: the unswept I=1 rows, a cell per thread
-      const int x = (u.b - (NR - 1) * G) * blockDim.x + threadIdx.x;
-      if (x < NT * P) as_global(launch_dst(L, t) + so)[x] = as_global(launch_src(L, t) + so)[x];
-      continue;
+      const int T = 64 * Q, x = (u.b - (NR - 1) * G) * T + threadIdx.x;
+      if ((!MIXED || (int)threadIdx.x < T) && x < NT * P) as_global(launch_dst(L, t) + so)[x] = as_global(launch_src(L, t) + so)[x];
+      return;
     }
     const int i1 = u.b / G, q0 = (u.b - i1 * G) * 64, i = i1 + 1;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (MIXED && w >= Q) return line_barriers(MODE == 0 ? 2 : 3);
     const LineLds d = line_lds(sm, Q);
     const int j0 = w * R;
     const bool act = q0 + lane < P;
@@ -335,14 +338,57 @@ __global__ void __launch_bounds__(1024, line_simd_waves(R)) k_p_rows(Launch L) {
   }
 }
 
+}  // namespace
+
+template <int MODE, int R>
+__global__ void __launch_bounds__(1024, line_simd_waves(R)) k_r_rows(Launch L) {
+  extern __shared__ double sm[];
+  for (int vb = blockIdx.x; vb < L.nv; vb += gridDim.x) r_rows_unit<MODE, R, false>(L, const_unit(L, vb), sm);
+}
+template <int MODE, int R>
+__global__ void __launch_bounds__(1024, line_simd_waves(R)) k_p_rows(Launch L) {
+  extern __shared__ double sm[];
+  for (int vb = blockIdx.x; vb < L.nv; vb += gridDim.x) p_rows_unit<MODE, R, false>(L, const_unit(L, vb), sm);
+}
+
+// Cells per thread the line kernels are built for (more of them spill).
+#define LINE_ROWS(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8)
+
+// An ensemble's members in one launch, each with the rows it has alone.
+template <int MODE>
+__global__ void __launch_bounds__(1024, line_simd_waves(8)) k_r_mixed(Launch L) {
+  extern __shared__ double sm[];
+  for (int vb = blockIdx.x; vb < L.nv; vb += gridDim.x) {
+    const CUnit u = const_unit(L, vb);
+    switch (u.rows) {
+#define ROWS(r) \
+  case r: r_rows_unit<MODE, r, true>(L, u, sm); break;
+      LINE_ROWS(ROWS)
+#undef ROWS
+    }
+    if (L.nv > (int)gridDim.x) __syncthreads();  // the next unit may lay its LDS out otherwise
+  }
+}
+template <int MODE>
+__global__ void __launch_bounds__(1024, line_simd_waves(8)) k_p_mixed(Launch L) {
+  extern __shared__ double sm[];
+  for (int vb = blockIdx.x; vb < L.nv; vb += gridDim.x) {
+    const CUnit u = const_unit(L, vb);
+    switch (u.rows) {
+#define ROWS(r) \
+  case r: p_rows_unit<MODE, r, true>(L, u, sm); break;
+      LINE_ROWS(ROWS)
+#undef ROWS
+    }
+    if (L.nv > (int)gridDim.x) __syncthreads();  // the next unit may lay its LDS out otherwise
+  }
+}
+
 }  // namespace ramgpu
 
 using namespace ramgpu;
 
 namespace ramgpu_host {
-
-// Cells per thread the line kernels are built for (more of them spill).
-#define LINE_ROWS(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8)
 
 // Cells per thread of k_r_rows or k_p_rows for lines of n cells, 0 for one
 // thread per line (k_r, k_p), of which a problem has `lines` in all.
@@ -387,6 +433,11 @@ void launch_r(int mode, LineShape sh, dim3 grid, hipStream_t st, const Launch &L
     break;
     LINE_ROWS(ROWS)
 #undef ROWS
+    case kMixedRows:
+      if (mode == 0) hipLaunchKernelGGL(k_r_mixed<0>, grid, blk, lds, st, L);
+      else if (mode == 1) hipLaunchKernelGGL(k_r_mixed<1>, grid, blk, lds, st, L);
+      else hipLaunchKernelGGL(k_r_mixed<2>, grid, blk, lds, st, L);
+      break;
     default:
       if (mode == 0) hipLaunchKernelGGL(k_r<0>, grid, blk, lds, st, L);
       else if (mode == 1) hipLaunchKernelGGL(k_r<1>, grid, blk, lds, st, L);
@@ -405,6 +456,10 @@ void launch_p(int mode, LineShape sh, dim3 grid, hipStream_t st, const Launch &L
     break;
     LINE_ROWS(ROWS)
 #undef ROWS
+    case kMixedRows:
+      if (mode == 0) hipLaunchKernelGGL(k_p_mixed<0>, grid, blk, lds, st, L);
+      else hipLaunchKernelGGL(k_p_mixed<1>, grid, blk, lds, st, L);
+      break;
     default:
       if (mode == 0) hipLaunchKernelGGL(k_p<0>, grid, blk, lds, st, L);
       else hipLaunchKernelGGL(k_p<1>, grid, blk, lds, st, L);

@@ -35,11 +35,10 @@ __device__ __forceinline__ double from_lane_above0(double v) {
 
 // x0: tape slot 0; slots 0..4 hold the inputs of the five phases and slot 7
 // the drift phases' clamp decisions (k_plane_step<SEQ_TAPE>).
-template <int R>
-__global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_adj(Launch L, const double *xin, double *adj) {
-  extern __shared__ __align__(16) double sm[];
-  for (int vb = blockIdx.x; vb < L.nv; vb += gridDim.x) {
-    const CUnit u = const_unit(L, vb);
+// MIXED: the block may have more threads than the plane needs (adj_threads).
+template <int R, bool MIXED>
+__device__ __forceinline__ void plane_adj_unit(const Launch &L, const double *xin, double *adj, const CUnit &u, double *sm) {
+  {
     CTab *const tp = u.t;
 #define t (*tp)
     fetched(t.ns, t.nr, t.nt, t.ne, t.npa, t.rnt, t.rne, t.f2, t.tape, t.lam, t.kle, t.klm, t.kll, t.lt4, t.kt, t.edot,
@@ -64,6 +63,11 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_adj(
     double *const ex = kt + (SKT_N + 2) * NE;
 
     const int W = adj_wave_cells(NE), halo = (64 - W) / 2, c_raw = wv * W + lane - halo;
+    const int T = MIXED ? (ncol + W - 1) / W * 64 : (int)blockDim.x;
+    if (MIXED && tid >= T) {  // whole waves: the unit's barriers
+      for (int x = 0; x < (halo ? 10 : 8); ++x) __syncthreads();
+      return;
+    }
     const bool own = c_raw >= 0 && c_raw < ncol && lane >= halo && lane < halo + W;
     const int c_ = min(max(c_raw, 0), ncol - 1);
     const int q_ = fast_div(c_, NE, t.rne), k_ = c_ - q_ * NE;
@@ -88,7 +92,7 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_adj(
       const gptr<const double> gk = as_global(t.kt + (size_t)s * SKT_N * NE);
       const gptr<const double> ge = as_global(t.edot + ((size_t)s * NR + i) * NE), gl = as_global(t.latl + ((size_t)s * NR + i) * NE),
                                gx = as_global(t.ex64);
-      const int T = blockDim.x, n1 = 4 * NPA, n3 = 2 * NPA, nk = SKT_N * NE;
+      const int n1 = 4 * NPA, n3 = 2 * NPA, nk = SKT_N * NE;
       d2 *const a0 = (d2 *)cf, *const a1 = (d2 *)cm, *const a3 = (d2 *)lt;
       // rows past NPA: zero terms, so that their faces carry nothing
 #pragma unroll 2
@@ -327,12 +331,37 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_adj(
       for (int n = 0; n < R; ++n)
         if (n < nr) g[(unsigned)((l0 + n) * NE + k)] = y[n];
     }
-    if (L.nv > (int)gridDim.x) __syncthreads();  // LDS is rewritten for the block's next plane
 #undef t
 #undef THREAD_CELLS
 #undef PLANE_SCALARS
   }
 }
+
+template <int R>
+__global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_adj(Launch L, const double *xin, double *adj) {
+  extern __shared__ __align__(16) double sm[];
+  for (int vb = blockIdx.x; vb < L.nv; vb += gridDim.x) {
+    plane_adj_unit<R, false>(L, xin, adj, const_unit(L, vb), sm);
+    if (L.nv > (int)gridDim.x) __syncthreads();  // LDS is rewritten for the block's next plane
+  }
+}
+
+// An ensemble's members in one launch, each with the rows it has alone.
+#if ADJ_PART == 3
+__global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_adj_mixed(Launch L) {
+  extern __shared__ __align__(16) double sm[];
+  for (int vb = blockIdx.x; vb < L.nv; vb += gridDim.x) {
+    const CUnit u = const_unit(L, vb);
+    switch (u.rows) {
+#define ROWS(r) \
+  case r: plane_adj_unit<r, true>(L, nullptr, nullptr, u, sm); break;
+      ADJ_ROWS(ROWS)
+#undef ROWS
+    }
+    if (L.nv > (int)gridDim.x) __syncthreads();
+  }
+}
+#endif
 
 // in groups (ADJ_PART of the build), each a translation unit of its own
 #define ADJ_INST(r) template __global__ void k_plane_adj<r>(Launch, const double *, double *);
@@ -342,7 +371,7 @@ ADJ_INST(ADJ_ONE)
 ADJ_INST(2) ADJ_INST(3) ADJ_INST(4) ADJ_INST(5)
 #elif ADJ_PART == 1
 ADJ_INST(6) ADJ_INST(7) ADJ_INST(8)
-#else
+#elif ADJ_PART == 2
 ADJ_INST(9) ADJ_INST(10) ADJ_INST(11) ADJ_INST(12)
 #endif
 

@@ -84,14 +84,14 @@ __device__ inline void step_line_tables(CTab &t, const StepLds &d, int i, int j,
 // positions, FLCscatter (src/ModRamRun.f90:81-172).  rec: bit 0 record the
 // CFL maxima, bit 1 COULMU's clamp (TimeRamElapsed > 0), bit 2 FLCscatter
 // acts (TimeRamElapsed >= Dt_bc).
-template <int SEQ, int R>
-__global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step(Launch L, int rec) {
+// MIXED: the block may have more threads than the plane needs (step_threads).
+template <int SEQ, int R, bool MIXED>
+__device__ __forceinline__ void plane_step_unit(const Launch &L, int rec, const CUnit &u, double *sm) {
   constexpr bool TAPE = SEQ == SEQ_TAPE, X = SEQ == SEQ_STEPX;
   constexpr bool kKeepE = R <= 4 && !X, kKeepMu = R <= (TAPE ? 8 : 9) && !X;
   constexpr int kSums = X ? kStepXSums : kStepSums;
-  extern __shared__ __align__(16) double sm[];
-  for (int vb = blockIdx.x; vb < L.nv; vb += gridDim.x) {
-    const CUnit u = const_unit(L, vb);
+  static_assert(!(MIXED && X), "the barriers of SEQ_STEPX depend on its processes");
+  {
     CTab *const tp = u.t;
 #define t (*tp)
     const int NE = t.ne, NPA = t.npa, NT = t.nt, NR = t.nr;
@@ -101,7 +101,7 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step
     if (u.b >= blocks_kl(t)) {  // out of place: copy plane (I=1, J) of the unswept row
       const size_t off = sstr + (size_t)(u.b - blocks_kl(t)) * NE * NPA;
       block_copy<8>(dst + off, src + off, NE * NPA);
-      continue;
+      return;
     }
     const int s = u.s, i = 1 + fast_div(u.b, NT, t.rnt), j = u.b - (i - 1) * NT;  // I = i+1 >= 2
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -119,6 +119,11 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step
     d.red = d.ex + 64;
     d.cmx = (unsigned long long *)(d.red + 16 * kSums);
     const bool apart = (X ? t.stepx_apart : t.step_apart) != 0;
+    const int W = t.step_cells, T = MIXED ? (ncol + W - 1) / W * 64 : (int)blockDim.x;
+    if (MIXED && tid >= T) {  // whole waves: the unit's barriers
+      for (int x = 0; x < (apart ? 6 : 8); ++x) __syncthreads();
+      return;
+    }
     d.H = apart ? (double *)(d.cmx + NE + kStepSpread * NPA) : d.F;
     if constexpr (X) {
       const int o = (int)((double *)(d.cmx + NE + kStepSpread * NPA) - sm) + (apart ? 4 * ncol : 0);
@@ -129,7 +134,7 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step
     // this thread's column; a wave's lane 0 repeats the last column of the
     // wave before (step_wave_cells), so that every energy face's upper
     // neighbour is the next lane
-    const int W = t.step_cells, c_raw = wv * W + lane - (64 - W);
+    const int c_raw = wv * W + lane - (64 - W);
     const bool own = c_raw < ncol && lane >= 64 - W;
     const int c_ = min(max(c_raw, 0), ncol - 1);
     const int q_ = fast_div(c_, NE, t.rne), k_ = c_ - q_ * NE;
@@ -155,7 +160,6 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step
       const gptr<const double> g2 = as_global((const double *)(t.kll + ij * NPA));  // HDNS, 1/FNHS
       const int n1 = 4 * NPA, n2 = NPA, n3 = 2 * NPA;
       d2 *const l0_ = (d2 *)d.cf, *const l1_ = (d2 *)d.cm, *const l3_ = (d2 *)d.lt;
-      const int T = blockDim.x;
       d2 v0 = {0, 0}, v1 = {0, 0}, v3 = {0, 0};
       double v2 = 0.0;
       if (tid < n1) {
@@ -709,13 +713,13 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step
     // and the loss chain's next barriers
     if (tid < kSums) {
       double v = 0.0;
-      for (int w = 0; w < (int)(blockDim.x >> 6); ++w) v += d.red[w * kSums + tid];
+      for (int w = 0; w < (T >> 6); ++w) v += d.red[w * kSums + tid];
       CTab &tt = *fresh_uniform(tp);
       tt.partials[((size_t)tid * tt.ns + s) * tt.maxblk + u.b] = v;
     }
     if (record) {
       unsigned long long *g = fresh_uniform(tp)->cflmax + (size_t)s * (2 + NE + NPA);
-      for (int e = tid; e < NE + NPA; e += blockDim.x) {
+      for (int e = tid; e < NE + NPA; e += T) {
         unsigned long long m;
         if (e < NE) {
           m = d.cmx[e];
@@ -729,10 +733,34 @@ __global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step
         if (m > __hip_atomic_load(&g[2 + e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(&g[2 + e], m);
       }
     }
-    if (L.nv > (int)gridDim.x) __syncthreads();  // LDS is rewritten for the block's next plane
 #undef t
 #undef THREAD_CELLS
 #undef PLANE_SCALARS
+  }
+}
+
+template <int SEQ, int R>
+__global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_step(Launch L, int rec) {
+  extern __shared__ __align__(16) double sm[];
+  for (int vb = blockIdx.x; vb < L.nv; vb += gridDim.x) {
+    plane_step_unit<SEQ, R, false>(L, rec, const_unit(L, vb), sm);
+    if (L.nv > (int)gridDim.x) __syncthreads();  // LDS is rewritten for the block's next plane
+  }
+}
+
+// An ensemble's members in one launch, each with the rows it has alone.
+template <int SEQ>
+__global__ void __launch_bounds__(kPlaneMaxThreads, kStepSimdWaves) k_plane_mixed(Launch L, int rec) {
+  extern __shared__ __align__(16) double sm[];
+  for (int vb = blockIdx.x; vb < L.nv; vb += gridDim.x) {
+    const CUnit u = const_unit(L, vb);
+    switch (u.rows) {
+#define ROWS(r) \
+  case r: plane_step_unit<SEQ, r, true>(L, rec, u, sm); break;
+      STEP_ROWS(ROWS)
+#undef ROWS
+    }
+    if (L.nv > (int)gridDim.x) __syncthreads();
   }
 }
 
@@ -752,8 +780,12 @@ STEP_INST(6) STEP_INST(7) STEP_INST(8)
 STEP_INST(9) STEP_INST(10) STEP_INST(11)
 #elif STEP_PART == 3
 STEP_INST(12) STEP_INST(13)
-#else
+#elif STEP_PART == 4
 STEP_INST(14) STEP_INST(15) STEP_INST(16)
+#elif STEP_PART == 5
+template __global__ void k_plane_mixed<SEQ_STEP>(Launch, int);
+#else
+template __global__ void k_plane_mixed<SEQ_TAPE>(Launch, int);
 #endif
 
 }  // namespace ramgpu

@@ -158,10 +158,12 @@ struct Tab {
   int mnpts;
 };
 
-// One unit of a launch: blocks [b0, b0+nb) of species s of problem tabs[tab].
+// One unit of a launch: blocks [b0, b0+nb) of species s of problem tabs[tab];
+// rows: the rows per thread of its kernel, where a launch has several.
 struct Job {
-  int tab, s, b0, nb;
+  int tab, s, b0, nb, rows;
 };
+constexpr int kMixedRows = -1;  // LineShape, StepShape: each job of the launch by its own rows
 // vmap entries: a virtual block's job and its block within the job
 constexpr int kVmapShift = 16;
 inline __host__ __device__ int vmap_entry(int job, int b) { return (job << kVmapShift) | b; }

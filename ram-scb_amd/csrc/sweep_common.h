@@ -295,16 +295,16 @@ __device__ __forceinline__ Unit unit_of(const Launch &L, int vb) {
 // The unit of virtual block vb with the descriptor in constant memory.
 struct CUnit {
   CTab *t;
-  int s, b;
+  int s, b, rows;
 };
 __device__ __forceinline__ CUnit const_unit(const Launch &L, int vb) {
   if (!L.vmap) {
     const Unit u = unit_of(L, vb);
-    return {as_const(L.tabs), u.s, u.b};
+    return {as_const(L.tabs), u.s, u.b, 0};
   }
   const int e = as_const(L.vmap)[vb];
   const cptr<Job> jb = as_const(L.jobs) + (e >> kVmapShift);
-  return {as_const(L.tabs) + jb->tab, jb->s, e & ((1 << kVmapShift) - 1)};
+  return {as_const(L.tabs) + jb->tab, jb->s, e & ((1 << kVmapShift) - 1), jb->rows};
 }
 
 // ---------------------------------------------------------------------------

@@ -21,7 +21,7 @@ LIB = PKG / "libramgpu.so"
 HIP_SOURCES = ["kernels.hip", "api.hip", "batch.hip", "adjoint.hip", "adjoint_api.hip", "moments.hip",
                "coulomb.hip", "pitch.hip", "bounce.hip", "hostio.hip", "line_sweep.hip"]
 # sources compiled once per part: (source, macro, parts)
-HIP_PARTS = [("plane_step.hip", "STEP_PART", 5), ("plane_adjoint.hip", "ADJ_PART", 3)]
+HIP_PARTS = [("plane_step.hip", "STEP_PART", 7), ("plane_adjoint.hip", "ADJ_PART", 4)]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17",
