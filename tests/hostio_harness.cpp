@@ -15,6 +15,7 @@
 
 static std::atomic<long> g_news_left{-1};  // allocations that still succeed (< 0: all)
 static std::atomic<long> g_mallocs{0}, g_frees{0};
+static std::atomic<size_t> g_malloc_bytes{0};
 
 static void *counted(size_t n) {
   if (g_news_left.load() >= 0 && g_news_left.fetch_sub(1) <= 0) {
@@ -32,8 +33,9 @@ void operator delete(void *p, size_t) noexcept { std::free(p); }
 void operator delete[](void *p, size_t) noexcept { std::free(p); }
 
 extern "C" {
-hipError_t hipMalloc(void **p, size_t) {
+hipError_t hipMalloc(void **p, size_t n) {
   ++g_mallocs;
+  g_malloc_bytes += n;
   *p = std::malloc(1);
   return hipSuccess;
 }
@@ -108,23 +110,36 @@ static int no_memory() {
 }
 
 // kept blocks: those of sizes no longer asked for make room for the latest
+// call's; of a call that holds more than is kept, as many as fit stay
 static int kept_blocks() {
   const size_t MB = size_t(1) << 20;
   void *p[8], *q;
-  for (int i = 0; i < 8; ++i) EXPECT(dev_take(0, &p[i], (900 + i) * MB));
-  for (int i = 0; i < 8; ++i) dev_give(0, p[i], (900 + i) * MB);
-  EXPECT(dev_cached(0) <= 4096 * MB);
-  long m = g_mallocs;
-  for (int i = 4; i < 8; ++i) EXPECT(dev_take(0, &p[i], (900 + i) * MB));  // the last four given
-  EXPECT(g_mallocs == m && dev_cached(0) == 0);
-  for (int i = 4; i < 8; ++i) dev_give(0, p[i], (900 + i) * MB);
+  for (int first : {0, 4})
+    for (int call = 0; call < 60; ++call) {
+      const long m = g_mallocs;
+      for (int i = first; i < first + 4; ++i) EXPECT(dev_take(0, &p[i], (900 + i) * MB));
+      EXPECT(call < 58 || (g_mallocs == m && dev_cached(0) == 0));
+      for (int i = first; i < first + 4; ++i) dev_give(0, p[i], (900 + i) * MB);
+      EXPECT(dev_cached(0) <= 4096 * MB);
+    }
+  EXPECT(dev_cached(0) == (904 + 905 + 906 + 907) * MB);
+  const size_t big[6] = {2000, 900, 700, 450, 300, 200};  // 4550: the last ones find no room
+  for (int call = 0; call < 60; ++call) {
+    const size_t b = g_malloc_bytes;
+    for (int i = 0; i < 6; ++i) EXPECT(dev_take(1, &p[i], big[i] * MB));
+    EXPECT(call < 58 || g_malloc_bytes - b <= 500 * MB);
+    for (int i = 0; i < 6; ++i) dev_give(1, p[i], big[i] * MB);
+    EXPECT(dev_take(0, &q, 100 * MB));  // a call in between
+    dev_give(0, q, 100 * MB);
+    EXPECT(dev_cached(0) + dev_cached(1) <= 4096 * MB);
+  }
   EXPECT(dev_take(0, &q, 5000 * MB));  // more than is ever kept: the others stay
+  const size_t kept = dev_cached(1);
   dev_give(0, q, 5000 * MB);
-  EXPECT(dev_cached(0) == (904 + 905 + 906 + 907) * MB);
-  EXPECT(dev_take(1, &q, 907 * MB));  // another device's block is not this one's
-  EXPECT(dev_cached(0) == (904 + 905 + 906 + 907) * MB);
-  dev_give(1, q, 907 * MB);
-  EXPECT(dev_cached(0) + dev_cached(1) <= 4096 * MB && dev_cached(1) == 907 * MB);
+  EXPECT(kept > 4000 * MB && dev_cached(1) == kept);
+  EXPECT(dev_take(0, &q, 900 * MB));  // another device's block is not this one's
+  EXPECT(dev_cached(1) == kept);
+  dev_give(0, q, 900 * MB);
   context_opened();
   context_closed();
   EXPECT(dev_cached(0) == 0 && dev_cached(1) == 0 && g_mallocs == g_frees);

@@ -1,8 +1,8 @@
 """The host side of bulk transfers and kept device blocks (csrc/hostio.hip),
 run without a device: hostio_harness.cpp stands in for the HIP calls.
 no_memory: a transfer that cannot allocate still moves the data, with no
-exception out of the C ABI.  kept_blocks: at most 4 GiB stay, the blocks given
-back last, and all go with the last context."""
+exception out of the C ABI.  kept_blocks: at most 4 GiB stay, those of the
+latest calls, and all go with the last context."""
 import shutil
 import subprocess
 from pathlib import Path
