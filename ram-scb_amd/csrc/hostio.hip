@@ -23,11 +23,12 @@ namespace {
 
 using namespace ramgpu_host;
 
-// Smaller arrays take the runtime's own copy: to the host the ring gains from
-// 10 MB on (0.75 -> 0.69 ms; 40 MB 4.0 -> 1.7, 265 MB 25.9 -> 8.7), to the
-// device, where no pages are faulted in, from 40 MB on (1.48 -> 1.35, 100 MB
-// 3.6 -> 2.6; 10 MB 0.33 -> 0.58).
-constexpr size_t kPipeMinToHost = size_t(8) << 20, kPipeMinToDevice = size_t(32) << 20;
+// Smaller arrays take the runtime's own copy.  A whole get_f2 by it and by the
+// ring: 9 MB 0.53 -> 0.48 ms into pages that are there, 0.65 -> 0.61 into fresh
+// ones, 40 MB 4.0 -> 1.7, 265 MB 25.9 -> 8.7.  A whole put_f2, where no pages
+// are faulted in: 34 MB 1.06 -> 1.09, 36 MB 1.21 -> 1.13, 40 MB 1.46 -> 1.21,
+// 100 MB 3.6 -> 2.6 (10 MB 0.33 -> 0.58).
+constexpr size_t kPipeMinToHost = size_t(8) << 20, kPipeMinToDevice = size_t(34) << 20;
 constexpr int kSlots = 8;
 constexpr size_t kSlotBytes = size_t(4) << 20; // 32 MiB of pinned memory per process
 constexpr int kMaxThreads = 6;
