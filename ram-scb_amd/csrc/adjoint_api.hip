@@ -96,21 +96,42 @@ void launch_plane_bwd(int seq, int threads, dim3 grid, size_t lds, hipStream_t s
     launch_plane_bwd_t<kPlaneMaxThreads>(seq, grid, lds, st, L, x, adj);
 }
 
+// Tiles cost a second trip through LDS and want cells enough each: a thread per
+// cell is faster for small arrays and where NS*NR*NE is short (us, cells /
+// tiles, in and out: 1x6x7x6x13, 26 KB 4.6 / 5.7, 2.6 / 4.2; 2x6x7x13x35, 0.3 MB
+// 4.7 / 6.0, 3.0 / 4.4; 4x6x12x20x31, 1.4 MB 5.1 / 5.6, 6.0 / 5.4; 3x4x25x35x45,
+// 3.8 MB 8.2 / 8.6, 12.6 / 9.8; 4x6x16x31x40, 3.8 MB 8.1 / 6.8, 12.7 / 7.0;
+// 1x7x25x35x71, 3.5 MB 7.7 / 9.8, 11.3 / 13.0; 1x4x48x64x90, 8.8 MB 13.9 / 16.8,
+// 20.3 / 22.1; 1x5x48x64x90, 11 MB 17.7 / 17.3, 24.4 / 22.7).
+static bool f2_by_tiles(bool in, size_t row_cells, size_t bytes) {
+  return row_cells >= 320 && bytes >= (in ? 3000000u : 1200000u);
+}
+
+int launch_f2(ramgpu_ctx *c, bool in, double *dst, const double *src, int ns) {
+  const size_t row_cells = (size_t)ns * c->nr * c->ne;
+  const bool tiles = f2_by_tiles(in, row_cells, row_cells * c->nt * c->npa * sizeof(double));
+#define F2(IN, TILES)                                                                                             \
+  hipLaunchKernelGGL((k_f2<IN, TILES>), dim3(TILES ? 2048 : 1024), dim3(256), 0, c->stream, dst, src, ns, c->nr, c->nt, \
+                     c->ne, c->npa)
+  if (in && tiles) F2(true, true);
+  else if (in) F2(true, false);
+  else if (tiles) F2(false, true);
+  else F2(false, false);
+#undef F2
+  return launch_check("k_f2");
+}
+
 // host Fortran-layout F2 <-> device-layout buffer (through the context's stage)
 int upload_f2(ramgpu_ctx *c, double *dst, const double *host) {
   const size_t n = (size_t)c->ns * c->nr * c->nt * c->ne * c->npa;
   const int rc = copy_to_device(c->device, c->stream, c->d_stage, host, n * sizeof(double));
   if (rc) return rc;
-  hipLaunchKernelGGL(k_f2_in, dim3(2048), dim3(256), 0, c->stream, dst, (const double *)c->d_stage, c->ns, c->nr,
-                     c->nt, c->ne, c->npa);
-  return launch_check("k_f2_in");
+  return launch_f2(c, true, dst, c->d_stage, c->ns);
 }
 
 int download_f2(ramgpu_ctx *c, double *host, const double *src) {
   const size_t n = (size_t)c->ns * c->nr * c->nt * c->ne * c->npa;
-  hipLaunchKernelGGL(k_f2_out, dim3(2048), dim3(256), 0, c->stream, c->d_stage, src, c->ns, c->nr, c->nt, c->ne,
-                     c->npa);
-  int rc = launch_check("k_f2_out");
+  const int rc = launch_f2(c, false, c->d_stage, src, c->ns);
   if (rc) return rc;
   return copy_to_host(c->device, c->stream, host, c->d_stage, n * sizeof(double));
 }

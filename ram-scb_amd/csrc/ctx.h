@@ -46,8 +46,8 @@ __global__ void k_finalize(Launch L, int cflmask, int summode);
 __global__ void k_vs(double *vt, const double *lz, const double *phi, const double *kp_ptr,
                      double kp_val, int nr1, int nt, const double *bs_src, double *bs_dst, int ns);
 __global__ void k_copy(double2 *dst, const double2 *src, size_t n2);
-__global__ void k_f2_in(double *dst, const double *src, int ns, int nr, int nt, int ne, int npa);
-__global__ void k_f2_out(double *dst, const double *src, int ns, int nr, int nt, int ne, int npa);
+template <bool IN, bool TILES>
+__global__ void k_f2(double *dst, const double *src, int ns, int nr, int nt, int ne, int npa);
 }  // namespace ramgpu
 
 // Rows per thread the fused step's plane kernel and its adjoint are built for.
@@ -228,6 +228,8 @@ void dev_give(int device, void *p, size_t bytes);
 size_t dev_cached(int device);
 void context_opened();
 void context_closed();
+// F2 of ns species from Fortran's order to the device's (in) or back
+int launch_f2(ramgpu_ctx *c, bool in, double *dst, const double *src, int ns);
 // host Fortran-layout F2 <-> device-layout buffer, through the context's stage
 int upload_f2(ramgpu_ctx *c, double *dst, const double *host);
 int download_f2(ramgpu_ctx *c, double *host, const double *src);

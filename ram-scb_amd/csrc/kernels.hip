@@ -1691,7 +1691,7 @@ __global__ void k_copy(double2 *__restrict__ dst, const double2 *__restrict__ sr
 // cells a thread in flight.  In / out, a thread per cell -> tiles:
 // 4x20x25x35x72 (40 MB) 98 / 65 -> 25 / 22 us (3.2 and 3.7 TB/s moved),
 // 4x40x49x35x72 (158 MB) 385 / 525 -> 70 / 81 us, 1x20x25x35x72 21 / 22 ->
-// 14 / 13 us; at 0.3 MB the second trip through LDS costs 2 us.
+// 14 / 13 us.  Which arrays take it: f2_by_tiles.
 template <bool IN>
 __device__ __forceinline__ void f2_tiles(double *dst, const double *src, int ns, int nr, int nt, int ne, int npa) {
   constexpr int TR = 128, TK = 64, T = 2048, U = T / 256;  // blocks of 256 threads
@@ -1741,12 +1741,34 @@ __device__ __forceinline__ void f2_tiles(double *dst, const double *src, int ns,
     __syncthreads();  // the tile is read
   }
 }
-__global__ void __launch_bounds__(256) k_f2_in(double *dst, const double *src, int ns, int nr, int nt, int ne, int npa) {
-  f2_tiles<true>(dst, src, ns, nr, nt, ne, npa);
+// The same by a thread per cell, contiguous in the device's order (fewer than
+// 2^31 cells: f2_by_tiles).
+template <bool IN>
+__device__ __forceinline__ void f2_cells(double *dst, const double *src, int ns, int nr, int nt, int ne, int npa) {
+  const unsigned n = (unsigned)ns * nr * nt * ne * npa;
+  for (unsigned x = blockIdx.x * blockDim.x + threadIdx.x; x < n; x += gridDim.x * blockDim.x) {
+    unsigned r = x;  // device index: k fastest, then l, j, i, s
+    const unsigned k = r % ne;
+    r /= ne;
+    const unsigned l = r % npa;
+    r /= npa;
+    const unsigned j = r % nt;
+    r /= nt;
+    const unsigned i = r % nr, s = r / nr;
+    const size_t h = s + (size_t)ns * (i + (size_t)nr * (j + (size_t)nt * (k + (size_t)ne * l)));
+    if (IN) dst[x] = src[h];
+    else dst[h] = src[x];
+  }
 }
-__global__ void __launch_bounds__(256) k_f2_out(double *dst, const double *src, int ns, int nr, int nt, int ne, int npa) {
-  f2_tiles<false>(dst, src, ns, nr, nt, ne, npa);
+template <bool IN, bool TILES>
+__global__ void __launch_bounds__(256) k_f2(double *dst, const double *src, int ns, int nr, int nt, int ne, int npa) {
+  if constexpr (TILES) f2_tiles<IN>(dst, src, ns, nr, nt, ne, npa);
+  else f2_cells<IN>(dst, src, ns, nr, nt, ne, npa);
 }
+template __global__ void k_f2<true, true>(double *, const double *, int, int, int, int, int);
+template __global__ void k_f2<true, false>(double *, const double *, int, int, int, int, int);
+template __global__ void k_f2<false, true>(double *, const double *, int, int, int, int, int);
+template __global__ void k_f2<false, false>(double *, const double *, int, int, int, int, int);
 
 // explicit instantiations used by the host code
 template __global__ void k_r<0>(Launch);

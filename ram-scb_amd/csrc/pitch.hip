@@ -31,9 +31,7 @@ int upload_coef(ramgpu_ctx *c, double **slot, const double *d1, const double *d2
   if (d2)
     for (size_t e = 0; e < n; ++e) sum[e] = d1[e] + d2[e];  // ATAW+ATAC, src/ModRamWPI.f90:675
   HIP_TRY(hipMemcpyAsync(c->d_stage, sum.data(), n * sizeof(double), hipMemcpyHostToDevice, c->stream));
-  hipLaunchKernelGGL(k_f2_in, dim3(2048), dim3(256), 0, c->stream, *slot, c->d_stage, 1,
-                     c->nr, c->nt, c->ne, c->npa);
-  int rc = launch_check("k_f2_in");
+  const int rc = launch_f2(c, true, *slot, c->d_stage, 1);
   if (rc) return rc;
   HIP_TRY(hipStreamSynchronize(c->stream));  // the host sum goes out of scope
   return RAMGPU_OK;
