@@ -99,17 +99,20 @@ void launch_plane_bwd(int seq, int threads, dim3 grid, size_t lds, hipStream_t s
 // Tiles cost a second trip through LDS and want cells enough each: a thread per
 // cell is faster for small arrays and where NS*NR*NE is short (us, cells /
 // tiles, in and out: 1x6x7x6x13, 26 KB 4.6 / 5.7, 2.6 / 4.2; 2x6x7x13x35, 0.3 MB
-// 4.7 / 6.0, 3.0 / 4.4; 4x6x12x20x31, 1.4 MB 5.1 / 5.6, 6.0 / 5.4; 3x4x25x35x45,
-// 3.8 MB 8.2 / 8.6, 12.6 / 9.8; 4x6x16x31x40, 3.8 MB 8.1 / 6.8, 12.7 / 7.0;
+// 4.7 / 6.0, 3.0 / 4.4; 4x6x12x20x31, 1.4 MB 5.1 / 5.6, 6.0 / 5.4; 1x14x17x33x65,
+// 4.1 MB 7.8 / 8.8, 11.4 / 10.4; 4x6x12x31x64, 4.6 MB 9.9 / 7.8, 14.7 / 7.3;
 // 1x7x25x35x71, 3.5 MB 7.7 / 9.8, 11.3 / 13.0; 1x4x48x64x90, 8.8 MB 13.9 / 16.8,
-// 20.3 / 22.1; 1x5x48x64x90, 11 MB 17.7 / 17.3, 24.4 / 22.7).
-static bool f2_by_tiles(bool in, size_t row_cells, size_t bytes) {
-  return row_cells >= 320 && bytes >= (in ? 3000000u : 1200000u);
+// 20.3 / 22.1; 1x5x48x64x90, 11 MB 17.7 / 17.3, 24.4 / 22.7).  In planes of a
+// multiple of 2048 cells, eight blocks, each XCD keeps to its own pitch angles
+// and so to its own lines of the Fortran array: 1x16x20x32x64, 5.2 MB 6.9 / 8.4,
+// 6.4 / 8.8 (32x63 10.2 / 8.5, 12.9 / 8.8); 4x10x20x32x64, 13 MB 12.0 / 11.0.
+static bool f2_by_tiles(bool in, size_t row_cells, int plane, size_t bytes) {
+  return row_cells >= 320 && bytes >= (plane % 2048 == 0 ? 13000000u : in ? 4400000u : 1200000u);
 }
 
 int launch_f2(ramgpu_ctx *c, bool in, double *dst, const double *src, int ns) {
   const size_t row_cells = (size_t)ns * c->nr * c->ne;
-  const bool tiles = f2_by_tiles(in, row_cells, row_cells * c->nt * c->npa * sizeof(double));
+  const bool tiles = f2_by_tiles(in, row_cells, c->ne * c->npa, row_cells * c->nt * c->npa * sizeof(double));
 #define F2(IN, TILES)                                                                                             \
   hipLaunchKernelGGL((k_f2<IN, TILES>), dim3(TILES ? 2048 : 1024), dim3(256), 0, c->stream, dst, src, ns, c->nr, c->nt, \
                      c->ne, c->npa)
