@@ -598,11 +598,10 @@ __device__ void plane_mu_bwd(const Tab &t, const PlaneCtx &c, const PlaneLds &d,
   }
 }
 
-// Loss operators: F2 *= factor on their cell ranges, so the adjoint is
-// multiplied by the same factors.  which: 0 CHAREXCHANGE, 1 ATMOL, 2 the
-// chain CEX, ATMOL, ATMOL, CEX of ram_run.
-template <int BT>
-__device__ void plane_loss_bwd(const Tab &t, const PlaneCtx &c, const PlaneLds &d, double *Y, int which) {
+// CHAREXCHANGE or ATMOL: F2 *= factor on its cell range, so the adjoint is
+// multiplied by the same factor.
+template <int BT, bool ATMOL>
+__device__ void plane_loss_bwd(const PlaneCtx &c, const PlaneLds &d, double *Y) {
   const int NE = c.NE;
   const bool cex = c.cex != 0;
   const int upa = c.upa;
@@ -610,25 +609,9 @@ __device__ void plane_loss_bwd(const Tab &t, const PlaneCtx &c, const PlaneLds &
   for (int n = 0; n < 8; ++n)
     if (n < c.nmine) {
       CELL_KL_T(n, BT);
-      const bool cx = cex && k >= 1 && l >= 1 && which != 1;
-      const bool atm = k >= 1 && l + 1 >= upa && which != 0;
-      double y = Y[cc];
-      const double cxf = cx ? cex_factor(d, NE, k, l, d.pc[PC_DTS]) : 1.0;
-      const double af = atm ? atm_factor(d, NE, k, l) : 1.0;
-      // WAVELO's factor (1 for K=1 and species without it), on L>=2
-      const double wf = (l >= 1) ? d.kt[KT_WAVE * NE + k] : 1.0;
-      if (which == 2) {  // the chain WAVELO, CEX, ATMOL, ATMOL, CEX, WAVELO, reversed
-        y = y * wf;
-        if (cx) y = y * cxf;
-        if (atm) y = y * af;
-        if (atm) y = y * af;
-        if (cx) y = y * cxf;
-        y = y * wf;
-      } else {
-        if (cx) y = y * cxf;
-        if (atm) y = y * af;
-      }
-      d.H[cc] = y;
+      const double y = Y[cc];
+      if (ATMOL) d.H[cc] = (k >= 1 && l + 1 >= upa) ? y * atm_factor(d, NE, k, l) : y;
+      else d.H[cc] = (cex && k >= 1 && l >= 1) ? y * cex_factor(d, NE, k, l, d.pc[PC_DTS]) : y;
     }
   __syncthreads();
 }
@@ -641,7 +624,7 @@ __global__ void __launch_bounds__(BT, 4) k_plane_bwd(Launch L, const double *xin
   for (int vb = blockIdx.x; vb < L.nv; vb += gridDim.x) {
     const Unit u = unit_of(L, vb);
     const Tab &t = *u.t;
-    constexpr bool need_loss = SEQ == SEQ_CEX || SEQ == SEQ_ATM || SEQ == SEQ_LOSS;
+    constexpr bool need_loss = SEQ == SEQ_CEX || SEQ == SEQ_ATM;
     const size_t po = (size_t)u.s * f2_species_stride(t);
     const double *x0 = xin ? xin : launch_src(L, t);
     PlaneCtx c;
@@ -654,9 +637,7 @@ __global__ void __launch_bounds__(BT, 4) k_plane_bwd(Launch L, const double *xin
     __syncthreads();
     if constexpr (SEQ == SEQ_E) plane_e_bwd<BT>(t, c, d, Y);
     else if constexpr (SEQ == SEQ_MU) plane_mu_bwd<BT>(t, c, d, Y);
-    else if constexpr (SEQ == SEQ_CEX) plane_loss_bwd<BT>(t, c, d, Y, 0);
-    else if constexpr (SEQ == SEQ_ATM) plane_loss_bwd<BT>(t, c, d, Y, 1);
-    else if constexpr (SEQ == SEQ_LOSS) plane_loss_bwd<BT>(t, c, d, Y, 2);
+    else plane_loss_bwd<BT, SEQ == SEQ_ATM>(c, d, Y);
     block_copy<4>(ga, d.H, c.P);
     __syncthreads();
   }
@@ -773,7 +754,5 @@ template __global__ void k_plane_bwd<SEQ_CEX, 512>(Launch, const double *, doubl
 template __global__ void k_plane_bwd<SEQ_CEX, 1024>(Launch, const double *, double *);
 template __global__ void k_plane_bwd<SEQ_ATM, 512>(Launch, const double *, double *);
 template __global__ void k_plane_bwd<SEQ_ATM, 1024>(Launch, const double *, double *);
-template __global__ void k_plane_bwd<SEQ_LOSS, 512>(Launch, const double *, double *);
-template __global__ void k_plane_bwd<SEQ_LOSS, 1024>(Launch, const double *, double *);
 
 }  // namespace ramgpu

@@ -23,8 +23,7 @@ namespace ramgpu_host {
 template <int BT>
 void set_bwd_lds_limit_t(size_t limit) {
   const void *fns[] = {(const void *)k_plane_bwd<SEQ_E, BT>,   (const void *)k_plane_bwd<SEQ_MU, BT>,
-                       (const void *)k_plane_bwd<SEQ_CEX, BT>, (const void *)k_plane_bwd<SEQ_ATM, BT>,
-                       (const void *)k_plane_bwd<SEQ_LOSS, BT>};
+                       (const void *)k_plane_bwd<SEQ_CEX, BT>, (const void *)k_plane_bwd<SEQ_ATM, BT>};
   for (const void *f : fns) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)limit);
 }
 
@@ -34,16 +33,17 @@ void set_bwd_lds_limit_t(size_t limit) {
 int plane_bwd_threads(int ne, int npa) { return (ne * npa <= 8 * kPlaneThreads) ? kPlaneThreads : kPlaneMaxThreads; }
 
 template <int BT>
-void launch_plane_bwd_t(int seq, dim3 grid, size_t lds, hipStream_t st, const Launch &L, const double *x,
-                        double *adj) {
+int launch_plane_bwd_t(int seq, dim3 grid, size_t lds, hipStream_t st, const Launch &L, const double *x,
+                       double *adj) {
   const dim3 blk(BT);
   switch (seq) {
     case SEQ_E: hipLaunchKernelGGL((k_plane_bwd<SEQ_E, BT>), grid, blk, lds, st, L, x, adj); break;
     case SEQ_MU: hipLaunchKernelGGL((k_plane_bwd<SEQ_MU, BT>), grid, blk, lds, st, L, x, adj); break;
     case SEQ_CEX: hipLaunchKernelGGL((k_plane_bwd<SEQ_CEX, BT>), grid, blk, lds, st, L, x, adj); break;
     case SEQ_ATM: hipLaunchKernelGGL((k_plane_bwd<SEQ_ATM, BT>), grid, blk, lds, st, L, x, adj); break;
-    default: hipLaunchKernelGGL((k_plane_bwd<SEQ_LOSS, BT>), grid, blk, lds, st, L, x, adj); break;
+    default: return fail(RAMGPU_EINVAL, "no plane adjoint for sequence %d", seq);
   }
+  return RAMGPU_OK;
 }
 
 // Rows per thread of the step's plane adjoint: step_shape's rule with its own
@@ -88,12 +88,10 @@ void set_plane_bwd_lds_limit(size_t limit) {
   set_bwd_lds_limit_t<kPlaneMaxThreads>(limit);
 }
 
-void launch_plane_bwd(int seq, int threads, dim3 grid, size_t lds, hipStream_t st, const Launch &L, const double *x,
-                      double *adj) {
-  if (threads <= kPlaneThreads)
-    launch_plane_bwd_t<kPlaneThreads>(seq, grid, lds, st, L, x, adj);
-  else
-    launch_plane_bwd_t<kPlaneMaxThreads>(seq, grid, lds, st, L, x, adj);
+int launch_plane_bwd(int seq, int threads, dim3 grid, size_t lds, hipStream_t st, const Launch &L, const double *x,
+                     double *adj) {
+  return threads <= kPlaneThreads ? launch_plane_bwd_t<kPlaneThreads>(seq, grid, lds, st, L, x, adj)
+                                  : launch_plane_bwd_t<kPlaneMaxThreads>(seq, grid, lds, st, L, x, adj);
 }
 
 // Tiles cost a second trip through LDS and want cells enough each: a thread per
@@ -255,13 +253,14 @@ int bwd_plane(ramgpu_ctx *c, int seq, const double *x, double *adj, int s0, int 
   }
   const Launch L = launch_of(c, s0, nsp, blocks_kl(c->t));
   const size_t lds = bwd_lds(c);
+  int rc = RAMGPU_OK;
   tbeg(c, RAMGPU_KERNEL_PLANE_BWD);
   if (seq == SEQ_STEP)
     launch_plane_adj(c->adj, dim3(L.nv), adj_lds_bytes(c->ne, c->npa, c->adj.rows), c->stream, L, x, adj);
   else
-    launch_plane_bwd(seq, plane_bwd_threads(c->ne, c->npa), dim3(L.nv), lds, c->stream, L, x, adj);
+    rc = launch_plane_bwd(seq, plane_bwd_threads(c->ne, c->npa), dim3(L.nv), lds, c->stream, L, x, adj);
   tend(c);
-  return launch_check("k_plane_bwd");
+  return rc ? rc : launch_check("k_plane_bwd");
 }
 
 // One ram_run step (all species) from tape slot T_R1 (the step's input,

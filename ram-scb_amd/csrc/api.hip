@@ -364,7 +364,7 @@ PlaneShape plane_shape_for(int ne, int npa, int T) {
 }
 
 template <int MAXC>
-void launch_plane_t(int seq, int threads, dim3 grid, size_t lds, hipStream_t st, const Launch &L, int rec) {
+int launch_plane_t(int seq, int threads, dim3 grid, size_t lds, hipStream_t st, const Launch &L, int rec) {
   const dim3 blk(threads);
   switch (seq) {
     case SEQ_E: hipLaunchKernelGGL((k_plane<SEQ_E, MAXC>), grid, blk, lds, st, L, rec); break;
@@ -374,15 +374,15 @@ void launch_plane_t(int seq, int threads, dim3 grid, size_t lds, hipStream_t st,
     case SEQ_SUM: hipLaunchKernelGGL((k_plane<SEQ_SUM, MAXC>), grid, blk, lds, st, L, rec); break;
     case SEQ_WAVE: hipLaunchKernelGGL((k_plane<SEQ_WAVE, MAXC>), grid, blk, lds, st, L, rec); break;
     case SEQ_COULEN: hipLaunchKernelGGL((k_plane<SEQ_COULEN, MAXC>), grid, blk, lds, st, L, rec); break;
-    default: hipLaunchKernelGGL((k_plane<SEQ_COULMU, MAXC>), grid, blk, lds, st, L, rec); break;
+    case SEQ_COULMU: hipLaunchKernelGGL((k_plane<SEQ_COULMU, MAXC>), grid, blk, lds, st, L, rec); break;
+    default: return fail(RAMGPU_EINVAL, "no plane kernel for sequence %d", seq);
   }
+  return RAMGPU_OK;
 }
 
-void launch_plane(int seq, PlaneShape sh, dim3 grid, size_t lds, hipStream_t st, const Launch &L, int rec) {
-  if (sh.maxc <= 8)
-    launch_plane_t<8>(seq, sh.threads, grid, lds, st, L, rec);
-  else
-    launch_plane_t<16>(seq, sh.threads, grid, lds, st, L, rec);
+int launch_plane(int seq, PlaneShape sh, dim3 grid, size_t lds, hipStream_t st, const Launch &L, int rec) {
+  return sh.maxc <= 8 ? launch_plane_t<8>(seq, sh.threads, grid, lds, st, L, rec)
+                      : launch_plane_t<16>(seq, sh.threads, grid, lds, st, L, rec);
 }
 
 // Rows per thread of the fused step's plane kernel, a function of NE, NPA and
@@ -447,15 +447,16 @@ int run_plane(ramgpu_ctx *c, int seq, int rec, int s0, int nsp, const double *sr
   L.ilv = 1;  // a plane's species on one XCD
   const size_t lds = seq_coul(seq) ? plane_coul_lds_bytes(c->ne, c->npa, c->plane.threads)
                                     : plane_fwd_lds_bytes(c->ne, c->npa, c->plane.threads);
+  int rc = RAMGPU_OK;
   tbeg(c, RAMGPU_KERNEL_PLANE);
   if (seq == SEQ_STEPX)
     launch_step(seq, c->stepx, dim3(L.nv), step_lds_bytes(c->ne, c->npa, c->stepx.rows, true), c->stream, L, rec);
   else if (seq == SEQ_STEP || seq == SEQ_TAPE)
     launch_step(seq, c->step, dim3(L.nv), step_lds_bytes(c->ne, c->npa, c->step.rows), c->stream, L, rec);
   else
-    launch_plane(seq, c->plane, dim3(L.nv), lds, c->stream, L, rec);
+    rc = launch_plane(seq, c->plane, dim3(L.nv), lds, c->stream, L, rec);
   tend(c);
-  return launch_check("k_plane");
+  return rc ? rc : launch_check("k_plane");
 }
 
 int run_finalize(ramgpu_ctx *c, int cflmask, int summode, int s0, int nsp) {

@@ -705,13 +705,7 @@ int ramgpu_batch_adjoint_run(ramgpu_batch *b, int nsteps, int ckpt_every, const 
     }
   }
   const int nseg = (nsteps + ckpt_every - 1) / ckpt_every, seglen = std::min(ckpt_every, nsteps);
-  // plane adjoint LDS
-  size_t bwd_lds = 0, lds_limit = b->m[0]->lds_limit;
-  for (ramgpu_ctx *c : b->m) {
-    bwd_lds = std::max(bwd_lds, plane_bwd_lds_bytes(c->ne, c->npa));
-  }
-  if (bwd_lds > lds_limit) return fail(RAMGPU_EINVAL, "plane adjoint does not fit the device LDS");
-  set_plane_bwd_lds_limit(lds_limit);
+  set_plane_bwd_lds_limit(b->m[0]->lds_limit);
   // memory plan
   size_t nall = 0, ngall = 0;
   for (ramgpu_ctx *c : b->m) {

@@ -188,7 +188,7 @@ void launch_p(int mode, LineShape sh, dim3 grid, hipStream_t st, const ramgpu::L
 // launch k_plane_step<seq, rows>
 void launch_step(int seq, StepShape sh, dim3 grid, size_t lds, hipStream_t st, const ramgpu::Launch &L, int rec);
 // launch k_plane<seq, maxc>
-void launch_plane(int seq, PlaneShape sh, dim3 grid, size_t lds, hipStream_t st, const ramgpu::Launch &L, int rec);
+int launch_plane(int seq, PlaneShape sh, dim3 grid, size_t lds, hipStream_t st, const ramgpu::Launch &L, int rec);
 // tape slots: the inputs of the operators of one ram_run step, in order
 // (T_E1..T_E2 consecutive: the plane kernels address them from T_E1)
 // T_CLAMP: the plane phases' clamp decisions, one byte plane per drift
@@ -200,8 +200,8 @@ StepShape adj_shape(int ne, int npa, long planes, int ncu, size_t lds_cu);
 void launch_plane_adj(StepShape sh, dim3 grid, size_t lds, hipStream_t st, const ramgpu::Launch &L, const double *x,
                       double *adj);
 void set_plane_bwd_lds_limit(size_t limit);
-void launch_plane_bwd(int seq, int threads, dim3 grid, size_t lds, hipStream_t st, const ramgpu::Launch &L,
-                      const double *x, double *adj);
+int launch_plane_bwd(int seq, int threads, dim3 grid, size_t lds, hipStream_t st, const ramgpu::Launch &L,
+                     const double *x, double *adj);
 // Coulomb collisions: the COULPARA tables (formed when stale), and whether
 // the plane kernels' LDS with them fits blocks of `threads`
 int coul_tables(ramgpu_ctx *c);

@@ -2,10 +2,12 @@
 //
 // F2 is kept on the device per species in a [I][J][L][K] layout (K fastest):
 // the (K,L) plane of one (I,J) cell is one contiguous run of NE*NPA doubles.
-// The radial and local-time sweeps run one thread per line with consecutive
-// lanes on consecutive (L,K) positions, so every load and store of a wave is
-// one contiguous run; the energy and pitch-angle sweeps (plus the pointwise
-// loss operators between them) stage whole (K,L) planes in LDS.
+// The radial and local-time sweeps run one thread per line, or per piece of a
+// line where the lines are few, with consecutive lanes on consecutive (L,K)
+// positions, so every load and store of a wave is one contiguous run; the
+// energy and pitch-angle sweeps take a whole (K,L) plane per block, in the
+// fused step with its rows in registers (and the loss operators between them),
+// as single operators in LDS.
 //
 // Coefficient tables hold the reference's intermediate quantities (its
 // GPA, GPR1.., DRD1.., CMUDOT.. terms) computed in the reference's expression

@@ -538,7 +538,6 @@ enum PlaneSeq : int {
   SEQ_ATM = 3,   // ATMOL
   SEQ_SUM = 4,   // SUMRC partial sum, slot 0
   SEQ_STEP = 5,  // the middle of ram_run: DRIFTE, DRIFTMU, loss chain, DRIFTMU, DRIFTE (k_plane_step)
-  SEQ_LOSS = 6,  // the loss chain alone (plane adjoints)
   SEQ_TAPE = 7,  // SEQ_STEP out of place, also writing the input of each later phase to a tape (k_plane_step)
   SEQ_WAVE = 8,  // WAVELO
   SEQ_COULEN = 9,   // COULEN
@@ -585,15 +584,11 @@ __device__ __forceinline__ PlaneLds plane_lds(double *sm, int ne, int npa) {
 }
 
 struct PlaneCtx {
-  int s, i, j, NE, NPA, NT, P, nmine, nmax;  // nmax: the most cells any thread of the block owns
+  int s, i, j, NE, NPA, NT, P, nmine;  // nmine: the cells this thread owns
   int cex, upa;  // the species' charge-exchange kind, UPA(I)
   size_t ij;
   double rlz, rrlz, qs, beta;
   float rne;
-  // row-wise ownership of the forward plane kernels: this thread owns K = ke
-  // of rows L = le0, le0+lestep, .. with lestep = blockDim/NE
-  int ke, le0, lestep;
-  bool eact;
 };
 
 // (K,L) of the n-th cell owned by this thread of a BT-thread block (plane adjoints): cell threadIdx.x + n*BT
@@ -794,11 +789,6 @@ __device__ inline void plane_setup(const Tab &t, const Unit &u, double *sm, cons
   c.beta = t.betalim;
   c.rne = t.rne;
   c.nmine = (c.P - tid + T - 1) / T;  // cells tid, tid+blockDim, .. < P
-  c.nmax = (c.P + T - 1) / T;
-  c.lestep = T / NE;
-  c.le0 = fast_div(tid, NE, c.rne);
-  c.ke = tid - c.le0 * NE;
-  c.eact = tid < c.lestep * NE;
   d = plane_lds(sm, NE, NPA);
   const int P = c.P;
   const double *gF = src + (size_t)c.s * f2_species_stride(t) + c.ij * P;
