@@ -702,8 +702,8 @@ __global__ void k_misfit_ens(Launch L, int step, int adjoint) {
 // n arrays (NS,NT,NE,NPA) from Fortran's order to C's: of one array the
 // columns (S,J,K), contiguous in src for each L, become rows of NPA, placed by
 // S, J, K.  Bound by memory; 64x32 tiles through LDS, so that both sides move
-// whole runs (30 of 1x25x35x72, 15 MB, in two launches: 24 us, where NumPy took
-// 8 ms on the host).
+// whole runs (30 of 1x25x35x72, 15 MB: 13 us, where NumPy took 8 ms on the
+// host).
 __global__ void __launch_bounds__(256) k_fgeos_rows(double *__restrict__ dst, const double *__restrict__ src, int n, int ns,
                                                     int nt, int ne, int npa) {
   constexpr int TC = 64, TL = 32;

@@ -387,17 +387,16 @@ int ramgpu_ram_run_bwd(ramgpu_ctx *c, double *adj, double *fgeos_adj) {
 
 namespace {
 
-// the nsteps adjoints of FGEOS at bbar to the host, each array in C's order:
-// NR of them at a time through the context's stage (NR of FGEOS's size)
-int download_fgeos_rows(ramgpu_ctx *c, double *host, const double *bbar, int nsteps) {
+// the nsteps adjoints of FGEOS at bbar to the host, each array in C's order,
+// through stage, which holds `room` of them
+int download_fgeos_rows(ramgpu_ctx *c, double *host, const double *bbar, int nsteps, double *stage, size_t room) {
   const size_t ng = nfg(c);
-  for (int n0 = 0; n0 < nsteps; n0 += c->nr) {
-    const int m = std::min(c->nr, nsteps - n0);
-    hipLaunchKernelGGL(k_fgeos_rows, dim3(2048), dim3(256), 0, c->stream, c->d_stage, bbar + (size_t)n0 * ng, m, c->ns,
-                       c->nt, c->ne, c->npa);
+  for (size_t n0 = 0; n0 < (size_t)nsteps; n0 += room) {
+    const size_t m = std::min(room, nsteps - n0);
+    hipLaunchKernelGGL(k_fgeos_rows, dim3(2048), dim3(256), 0, c->stream, stage, bbar + n0 * ng, (int)m, c->ns, c->nt, c->ne,
+                       c->npa);
     int rc = launch_check("k_fgeos_rows");
-    if (rc || (rc = copy_to_host(c->device, c->stream, host + (size_t)n0 * ng, c->d_stage, (size_t)m * ng * sizeof(double))))
-      return rc;
+    if (rc || (rc = copy_to_host(c->device, c->stream, host + n0 * ng, stage, m * ng * sizeof(double)))) return rc;
   }
   return RAMGPU_OK;
 }
@@ -566,7 +565,8 @@ int adjoint_run(ramgpu_ctx *c, int nsteps, int ckpt_every, const double *kp, con
   }
   if (grad_f2 && (rc = download_f2(c, grad_f2, lam))) return rc;
   if (grad_fgeos) {
-    if (rows) return download_fgeos_rows(c, grad_fgeos, bbar, nsteps);
+    // the tape is free by now and holds seglen * T_N * NR of them
+    if (rows) return download_fgeos_rows(c, grad_fgeos, bbar, nsteps, tape, tape_n / ng);
     if ((rc = copy_to_host(c->device, c->stream, grad_fgeos, bbar, (size_t)nsteps * ng * sizeof(double)))) return rc;
   }
   return RAMGPU_OK;

@@ -2,8 +2,8 @@
 (nsteps,NS,NT,NE,NPA) array from RamGpu, Fortran-ordered steps from RamBatch,
 both with the values of the C ABI's Fortran-ordered ones (to 1e-12: two runs
 add the stale ghosts' terms atomically, in any order); at the edges of the
-reordering tiles (64 columns S,J,K by 32 L) and with more steps than go
-through the stage at a time (NR)."""
+reordering tiles (64 columns S,J,K by 32 L) and with more steps than the tape
+holds at a time (10 NR a step of a segment)."""
 import ctypes as C
 
 import numpy as np
@@ -19,8 +19,9 @@ pytestmark = [pytest.mark.gpu,
 
 TOL = 1e-12
 
-# species, (NR, NT, NE, NPA), steps: less than a tile, whole tiles, one more in each direction
-CASES = [(1, (5, 4, 4, 5), 3), (1, (4, 8, 8, 32), 9), (2, (4, 5, 13, 33), 4), (3, (5, 7, 9, 64), 11), (2, (6, 8, 20, 13), 2)]
+# species, (NR, NT, NE, NPA), steps: less than a tile, whole tiles, one more in each direction; more than 80 steps of NR = 4
+CASES = [(1, (5, 4, 4, 5), 3), (1, (4, 8, 8, 32), 9), (2, (4, 5, 13, 33), 4), (3, (5, 7, 9, 64), 11), (2, (6, 8, 20, 13), 2),
+         (1, (4, 4, 5, 6), 83)]
 
 
 @pytest.mark.parametrize("ns,grid,nsteps", CASES, ids=lambda v: "x".join(map(str, v)) if type(v) is tuple else str(v))
