@@ -2,7 +2,7 @@
 """Benchmark of the FP64 RAM split step on one MI355X.
 
 Headline workload (the batched ensemble): 512 members in one launch per
-kernel, 256 of 4 species on 20x25x35x72 and 256 of 4 species on
+kernel (the plane kernel: one per grid), 256 of 4 species on 20x25x35x72 and 256 of 4 species on
 40x48x48x90 (e-, H+, He+, O+ at 1:0.7:0.05:0.25; the electrons take the
 reference's default WAVELO lifetimes), per-member Kp ~ U(1,7) and boundary
 flux scale ~ LogNormal(0,0.5), dt = 5 s split steps under a captured HIP
@@ -43,7 +43,7 @@ More objects in the same line:
     checkpoints every 10 steps, against the 60-step forward alone;
   "batched_adjoint": the same misfit gradient for an ensemble of 4-species
     40x96x64x90 members (Kp ~ U(1,8) per member), 120 steps with checkpoints
-    every 20, in one launch per kernel, against the ensemble's forward;
+    every 20, all members in the same launches, against the ensemble's forward;
   "moments": ANISCH of every species (and with FLUX) on the resident F2;
   "computehI": the SCB->RAM bounce integrals from 101-sample field lines
     (dipole lines with 3% noise in B, smoothing on) on the 20x25x35x72 and

@@ -397,10 +397,12 @@ int launch_plane(int seq, PlaneShape sh, dim3 grid, size_t lds, hipStream_t st, 
 //   48x90 (40x48): 6: 612, 9: 453, 10: 553, 16: 734
 //   64x90 (20x48): 8: 385, 10: 456, 12: 308, 16: 411
 // One species of 20x25x35x72 has under two planes per CU: 6 rows 37, 12 rows 42.
-// x: SEQ_STEPX, whose line solves and tables take more LDS; the same rule is
-// right for it (plane launch with Coulomb collisions in us, by rows; 35x72, 4
-// species: 6: 252, 8: 269, 11: 213, 12: 230, 15: 288; 48x90, 2 species of
-// 20x24: 6: 231, 8: 257, 9: 163, 10: 177).
+// x: SEQ_STEPX, whose line solves and tables take more LDS.  It keeps no Courant
+// numbers, and from 7 rows on spills (120 bytes a lane at 9, 204 at 11), so the
+// terms have other reasons there, but the rule finds its best rows too (plane
+// launch with Coulomb collisions in us, by rows; 35x72, 4 species: 6: 252, 8: 269,
+// 11: 213, 12: 230, 15: 288; 48x90, 2 species of 20x24: 6: 231, 8: 257, 9: 163,
+// 10: 177).
 // The last chunk needs two rows: R with NPA mod R = 1 is left out.
 StepShape step_shape(int ne, int npa, long planes, int ncu, size_t lds_cu, bool x) {
   StepShape best{0, 0};

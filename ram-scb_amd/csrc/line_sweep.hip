@@ -351,7 +351,9 @@ __global__ void __launch_bounds__(1024, line_simd_waves(R)) k_p_rows(Launch L) {
   for (int vb = blockIdx.x; vb < L.nv; vb += gridDim.x) p_rows_unit<MODE, R, false>(L, const_unit(L, vb), sm);
 }
 
-// Cells per thread the line kernels are built for (more of them spill).
+// Cells per thread the line kernels are built for: more of them spill.  Of these
+// k_r_rows and k_p_rows at 2 cells and k_p_rows at 6 spill up to 7 registers
+// (8 to 28 bytes a lane), being held to the waves of line_simd_waves.
 #define LINE_ROWS(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8)
 
 // An ensemble's members in one launch, each with the rows it has alone.

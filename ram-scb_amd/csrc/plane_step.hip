@@ -20,7 +20,7 @@
 // out, and with whole chunks per thread six barriers a plane are left of
 // eighteen.  The rest is a block's start (one memory round trip, all tables
 // in flight with the plane) and its last wave.  Plane launch of 4 species,
-// before and after, by events: 35x72 (20x25 grid) 148 -> 94 us, 48x90 (40x48)
+// before and after, by events: 35x72 (20x25 grid) 148 -> 96 us, 48x90 (40x48)
 // 747 -> 453, 64x90 (20x48) 448 -> 308.
 #include <hip/hip_runtime.h>
 
